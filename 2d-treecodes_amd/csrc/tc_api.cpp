@@ -896,7 +896,7 @@ size_t tc_srv_context_bytes(tc_context *c)
 {
     size_t b = tc_tree_bytes(c->tree) + c->io.cap + c->cnt.cap;
     for (const TcScratch *w : {&c->ws, &c->tws})
-        for (const DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->scan_tmp, &w->istart, &w->ilevel, &w->info,
+        for (const DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->istart, &w->ilevel, &w->info,
                                 &w->tkeys, &w->tperm, &w->tsorted, &w->bbox_part, &w->ints, &w->packed, &w->work,
                                 &w->flist})
             b += d->cap;
@@ -912,7 +912,7 @@ void tc_srv_context_trim(tc_context *c)
     c->tree_kind = TC_KIND_NONE;
     c->io.release();
     for (TcScratch *w : {&c->ws, &c->tws})
-        for (DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->scan_tmp, &w->istart, &w->ilevel, &w->info,
+        for (DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->istart, &w->ilevel, &w->info,
                           &w->tkeys, &w->tperm, &w->tsorted, &w->bbox_part, &w->ints, &w->packed, &w->work,
                           &w->flist})
             d->release();

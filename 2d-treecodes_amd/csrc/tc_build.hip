@@ -20,10 +20,7 @@ constexpr int RS_ITEMS = 20;   // keys per thread per tile
 constexpr int RS_TILE = RS_NT * RS_ITEMS;
 constexpr int RS_BINS = 256;   // 8-bit digits: passes at bits 0, 8, 16, 24 (30-bit keys)
 constexpr int KH_GRID = 1024;  // most workgroups of the key kernel (each adds its digit totals once)
-constexpr int SCAN_NT = 1024;
-constexpr int SCAN_ITEMS = 8;
-constexpr int SCAN_CHUNK = SCAN_NT * SCAN_ITEMS;
-constexpr int TB_CHUNK = 1024;  // positions per wave in the internal-cell census
+constexpr int SCAN_NT = 1024;  // threads of the census workgroup
 
 __constant__ double c_binom[64 * 64];  // C(n, k) rounded to double, n, k < 64
 
@@ -63,69 +60,6 @@ TC_DEV uint32_t block_scan_excl(uint32_t v, uint32_t *s_w, uint32_t *total)
         *total = s_w[NW];
     __syncthreads();
     return res;
-}
-
-// Single-block exclusive scan of n items with a running carry.
-__global__ __launch_bounds__(SCAN_NT) void k_scan_single(const uint32_t *in, uint32_t *out, int n, uint32_t *total)
-{
-    __shared__ uint32_t s_w[SCAN_NT / 64 + 1];
-    uint32_t carry = 0;
-    for (int base = 0; base < n; base += SCAN_CHUNK) {
-        uint32_t v[SCAN_ITEMS];
-        uint32_t sum = 0;
-        const int i0 = base + threadIdx.x * SCAN_ITEMS;
-#pragma unroll
-        for (int j = 0; j < SCAN_ITEMS; ++j) {
-            v[j] = (i0 + j < n) ? in[i0 + j] : 0u;
-            sum += v[j];
-        }
-        uint32_t tot;
-        uint32_t pre = block_scan_excl<SCAN_NT>(sum, s_w, &tot) + carry;
-#pragma unroll
-        for (int j = 0; j < SCAN_ITEMS; ++j) {
-            if (i0 + j < n)
-                out[i0 + j] = pre;
-            pre += v[j];
-        }
-        carry += tot;
-    }
-    if (threadIdx.x == 0 && total)
-        *total = carry;
-}
-
-__global__ __launch_bounds__(SCAN_NT) void k_scan_partial(const uint32_t *in, int n, uint32_t *part)
-{
-    __shared__ uint32_t s_w[SCAN_NT / 64 + 1];
-    const int i0 = blockIdx.x * SCAN_CHUNK + threadIdx.x * SCAN_ITEMS;
-    uint32_t sum = 0;
-#pragma unroll
-    for (int j = 0; j < SCAN_ITEMS; ++j)
-        sum += (i0 + j < n) ? in[i0 + j] : 0u;
-    uint32_t tot;
-    block_scan_excl<SCAN_NT>(sum, s_w, &tot);
-    if (threadIdx.x == 0)
-        part[blockIdx.x] = tot;
-}
-
-__global__ __launch_bounds__(SCAN_NT) void k_scan_final(const uint32_t *in, uint32_t *out, int n,
-                                                         const uint32_t *part)
-{
-    __shared__ uint32_t s_w[SCAN_NT / 64 + 1];
-    const int i0 = blockIdx.x * SCAN_CHUNK + threadIdx.x * SCAN_ITEMS;
-    uint32_t v[SCAN_ITEMS];
-    uint32_t sum = 0;
-#pragma unroll
-    for (int j = 0; j < SCAN_ITEMS; ++j) {
-        v[j] = (i0 + j < n) ? in[i0 + j] : 0u;
-        sum += v[j];
-    }
-    uint32_t pre = block_scan_excl<SCAN_NT>(sum, s_w, nullptr) + part[blockIdx.x];
-#pragma unroll
-    for (int j = 0; j < SCAN_ITEMS; ++j) {
-        if (i0 + j < n)
-            out[i0 + j] = pre;
-        pre += v[j];
-    }
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint32_t v, size_t n)
@@ -718,43 +652,68 @@ __global__ __launch_bounds__(256) void k_gather_src(const double4 *packed, const
 // sorted position i is internal iff key[i-1] leaves the cell and key[i+cap]
 // stays in it, so every internal cell is found from three key reads, and its
 // breadth-first rank is a scan over (level, position).
-TC_DEV void cell_range(const uint32_t *keys, int n, int cap, int i, int &lo, int &hi)
+// A wave covers 64 IT consecutive positions, item j of lane l being position
+// base + 64 j + l; all the keys it needs are requested before the first is
+// used (one memory round trip per wave instead of IT).  Few items per wave where
+// the positions are few (more waves, shorter chains), many where they fill the
+// GPU anyway and the census table (TC_LMAX counts per workgroup) should stay
+// short.  Count and emission at 65,536 positions, key by key with IT = 16: 11 +
+// 16 us, with IT = 4: 5 + 6 us; at 2^24 positions 49 + 73 us, with IT = 16: 30 + 60 us.
+constexpr int TB_IT_SMALL = 4, TB_IT = 16, TB_SMALL_N = 1 << 20;
+
+// Internal levels [lo, hi] of the cells starting at this lane's positions
+// (none where hi < lo).
+template <int IT> TC_DEV void cell_ranges(const uint32_t *keys, int n, int cap, int base, int (&lo)[IT], int (&hi)[IT])
 {
-    lo = 1;
-    hi = 0;
-    if (i >= n)
-        return;
-    const uint32_t k = keys[i];
-    lo = (i == 0) ? 0 : tc_common_level(keys[i - 1], k) + 1;
-    hi = (i + cap < n) ? min(TC_LMAX - 1, tc_common_level(k, keys[i + cap])) : -1;
+    uint32_t k[IT], kp[IT], kc[IT];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const int i = base + 64 * j + tc_lane();
+        k[j] = i < n ? keys[i] : 0u;
+        kp[j] = i < n && i > 0 ? keys[i - 1] : 0u;
+        kc[j] = i + cap < n ? keys[i + cap] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const int i = base + 64 * j + tc_lane();
+        lo[j] = i >= n ? 1 : (i == 0 ? 0 : tc_common_level(kp[j], k[j]) + 1);
+        hi[j] = i >= n ? 0 : (i + cap < n ? min(TC_LMAX - 1, tc_common_level(k[j], kc[j])) : -1);
+    }
 }
 
-__global__ __launch_bounds__(256) void k_int_count(const uint32_t *keys, int n, int cap, uint32_t *cnt_tab,
-                                                    int nblk)
+// The workgroup's internal cells per level: into s_cnt[wave][level].
+template <int IT> TC_DEV void cell_counts(const int (&lo)[IT], const int (&hi)[IT], uint32_t (*s_cnt)[TC_LMAX])
 {
-    __shared__ uint32_t s_cnt[4][TC_LMAX];
-    const int lane = tc_lane(), wid = threadIdx.x >> 6;
-    const int base = (blockIdx.x * 4 + wid) * TB_CHUNK;
     uint32_t c[TC_LMAX];
 #pragma unroll
     for (int L = 0; L < TC_LMAX; ++L)
         c[L] = 0;
-    for (int j = 0; j < TB_CHUNK / 64; ++j) {
-        int lo, hi;
-        cell_range(keys, n, cap, base + j * 64 + lane, lo, hi);
-        if (!tc_ballot(hi >= lo))
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        if (!tc_ballot(hi[j] >= lo[j]))
             continue;
 #pragma unroll
         for (int L = 0; L < TC_LMAX; ++L)
-            c[L] += __popcll(tc_ballot(L >= lo && L <= hi));
+            c[L] += __popcll(tc_ballot(L >= lo[j] && L <= hi[j]));
     }
-    if (lane == 0)
+    if (tc_lane() == 0)
 #pragma unroll
         for (int L = 0; L < TC_LMAX; ++L)
-            s_cnt[wid][L] = c[L];
+            s_cnt[threadIdx.x >> 6][L] = c[L];
     __syncthreads();
+}
+
+template <int IT>
+__global__ __launch_bounds__(256) void k_int_count(const uint32_t *keys, int n, int cap, uint32_t *cnt_tab,
+                                                    int stride)
+{
+    __shared__ uint32_t s_cnt[4][TC_LMAX];
+    const int base = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 64 * IT;
+    int lo[IT], hi[IT];
+    cell_ranges<IT>(keys, n, cap, base, lo, hi);
+    cell_counts<IT>(lo, hi, s_cnt);
     if (threadIdx.x < TC_LMAX)
-        cnt_tab[threadIdx.x * nblk + blockIdx.x] =
+        cnt_tab[(size_t)threadIdx.x * stride + blockIdx.x] =
             s_cnt[0][threadIdx.x] + s_cnt[1][threadIdx.x] + s_cnt[2][threadIdx.x] + s_cnt[3][threadIdx.x];
 }
 
@@ -763,106 +722,113 @@ __global__ __launch_bounds__(256) void k_int_count(const uint32_t *keys, int n, 
 constexpr int INFO_BOX = 20;
 constexpr size_t INFO_BYTES = sizeof(int) * INFO_BOX + sizeof(double) * 4;
 
-// The census scan in one workgroup (k_scan_single over the level-major
-// counts, TC_LMAX rows of nblk) with k_level_starts' record: the thread that
-// writes the first prefix of a level also writes that level's start.
-__global__ __launch_bounds__(SCAN_NT) void k_census_single(const uint32_t *in, uint32_t *out, int nblk,
-                                                            uint32_t *total, const uint32_t *bad, const double *box,
-                                                            int *info)
+// The census in one workgroup: cnt holds TC_LMAX rows (levels) of nblk counts,
+// `stride` (a multiple of 4) apart; wave L sums, then scans row L, 1,024 counts
+// a step, so the rows run side by side, each step is one round of wide loads
+// and no count needs its level by division.  Writes every block's first rank
+// per level (level-major breadth-first order) to offs and the census record.
+// 4,096 blocks (2^24 positions): 11 us; the scan over all rows as one array
+// took 25 us in four launches.
+__global__ __launch_bounds__(SCAN_NT) void k_census(const uint32_t *cnt, uint32_t *offs, int nblk, int stride,
+                                                     const uint32_t *bad, const double *box, int *info)
 {
-    __shared__ uint32_t s_w[SCAN_NT / 64 + 1];
-    const int n = TC_LMAX * nblk;
-    uint32_t carry = 0;
-    for (int base = 0; base < n; base += SCAN_CHUNK) {
-        uint32_t v[SCAN_ITEMS];
-        uint32_t sum = 0;
-        const int i0 = base + threadIdx.x * SCAN_ITEMS;
+    static_assert(TC_LMAX < SCAN_NT / 64, "one wave per level");
+    __shared__ uint32_t s_tot[SCAN_NT / 64];
+    const int lane = tc_lane(), L = threadIdx.x >> 6;
+    // 16 counts of this lane from step b0: positions b0 + 256 j + 4 lane .. + 3
+    auto load = [&](int b0, uint4 (&v)[4]) {
 #pragma unroll
-        for (int j = 0; j < SCAN_ITEMS; ++j) {
-            v[j] = (i0 + j < n) ? in[i0 + j] : 0u;
-            sum += v[j];
+        for (int j = 0; j < 4; ++j) {
+            const int b = b0 + 256 * j + 4 * lane;
+            v[j] = b < nblk ? *reinterpret_cast<const uint4 *>(cnt + (size_t)L * stride + b) : make_uint4(0, 0, 0, 0);
+            v[j].y = b + 1 < nblk ? v[j].y : 0u;  // a row's last words may be padding
+            v[j].z = b + 2 < nblk ? v[j].z : 0u;
+            v[j].w = b + 3 < nblk ? v[j].w : 0u;
         }
-        uint32_t tot;
-        uint32_t pre = block_scan_excl<SCAN_NT>(sum, s_w, &tot) + carry;
+    };
+    uint32_t tot = 0;
+    if (L < TC_LMAX)
+        for (int b0 = 0; b0 < nblk; b0 += 1024) {
+            uint4 v[4];
+            load(b0, v);
 #pragma unroll
-        for (int j = 0; j < SCAN_ITEMS; ++j) {
-            const int i = i0 + j;
-            if (i < n) {
-                out[i] = pre;
-                if (i % nblk == 0)
-                    info[i / nblk] = (int)pre;
-            }
-            pre += v[j];
+            for (int j = 0; j < 4; ++j)
+                tot += (v[j].x + v[j].y) + (v[j].z + v[j].w);
         }
-        carry += tot;
-    }
-    if (threadIdx.x == 0) {
-        *total = carry;
-        info[TC_LMAX] = (int)carry;
-        info[TC_LMAX + 1] = (int)*bad;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+        tot += __shfl_xor(tot, off, 64);
+    if (lane == 0)
+        s_tot[L] = tot;
+    __syncthreads();
+    uint32_t start = 0;
+    for (int q = 0; q < L; ++q)
+        start += s_tot[q];
+    if (lane == 0) {
+        if (L <= TC_LMAX)
+            info[L] = (int)start;  // row TC_LMAX: the total
+        if (L == 0)
+            info[TC_LMAX + 1] = (int)*bad;
     }
     if (threadIdx.x >= 32 && threadIdx.x < 36)
         reinterpret_cast<double *>(info + INFO_BOX)[threadIdx.x - 32] = box[threadIdx.x - 32];
+    if (L >= TC_LMAX)
+        return;
+    for (int b0 = 0; b0 < nblk; b0 += 1024) {
+        uint4 v[4];
+        load(b0, v);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t sum = (v[j].x + v[j].y) + (v[j].z + v[j].w);
+            uint32_t x = sum;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t y = __shfl_up(x, off, 64);
+                if (lane >= off)
+                    x += y;
+            }
+            const int b = b0 + 256 * j + 4 * lane;
+            uint4 o;
+            o.x = start + x - sum;
+            o.y = o.x + v[j].x;
+            o.z = o.y + v[j].y;
+            o.w = o.z + v[j].z;
+            if (b < nblk)  // within the padded row
+                *reinterpret_cast<uint4 *>(offs + (size_t)L * stride + b) = o;
+            start += (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+        }
+    }
 }
 
-__global__ void k_level_starts(const uint32_t *offs, int nblk, const uint32_t *total, const uint32_t *bad,
-                               const double *box, int *info)
-{
-    const int L = threadIdx.x;
-    if (L < TC_LMAX)
-        info[L] = (int)offs[L * nblk];
-    if (L == TC_LMAX)
-        info[TC_LMAX] = (int)*total;
-    if (L == TC_LMAX + 1)
-        info[TC_LMAX + 1] = (int)*bad;
-    if (L >= 32 && L < 36)
-        reinterpret_cast<double *>(info + INFO_BOX)[L - 32] = box[L - 32];
-}
-
+template <int IT>
 __global__ __launch_bounds__(256) void k_int_emit(const uint32_t *keys, int n, int cap, const uint32_t *offs,
-                                                   int nblk, int *istart, int *ilevel)
+                                                   int stride, int *istart, int *ilevel)
 {
     __shared__ uint32_t s_cnt[4][TC_LMAX];
-    const int lane = tc_lane(), wid = threadIdx.x >> 6;
-    const int base = (blockIdx.x * 4 + wid) * TB_CHUNK;
+    const int wid = threadIdx.x >> 6;
+    const int base = (blockIdx.x * 4 + wid) * 64 * IT;
     uint32_t c[TC_LMAX];
 #pragma unroll
     for (int L = 0; L < TC_LMAX; ++L)
-        c[L] = 0;
-    for (int j = 0; j < TB_CHUNK / 64; ++j) {
-        int lo, hi;
-        cell_range(keys, n, cap, base + j * 64 + lane, lo, hi);
-        if (!tc_ballot(hi >= lo))
-            continue;
+        c[L] = offs[(size_t)L * stride + blockIdx.x];
+    int lo[IT], hi[IT];
+    cell_ranges<IT>(keys, n, cap, base, lo, hi);
+    cell_counts<IT>(lo, hi, s_cnt);
 #pragma unroll
-        for (int L = 0; L < TC_LMAX; ++L)
-            c[L] += __popcll(tc_ballot(L >= lo && L <= hi));
-    }
-    if (lane == 0)
-#pragma unroll
-        for (int L = 0; L < TC_LMAX; ++L)
-            s_cnt[wid][L] = c[L];
-    __syncthreads();
-#pragma unroll
-    for (int L = 0; L < TC_LMAX; ++L) {
-        uint32_t o = offs[L * nblk + blockIdx.x];
+    for (int L = 0; L < TC_LMAX; ++L)
         for (int w = 0; w < wid; ++w)
-            o += s_cnt[w][L];
-        c[L] = o;
-    }
-    for (int j = 0; j < TB_CHUNK / 64; ++j) {
-        const int i = base + j * 64 + lane;
-        int lo, hi;
-        cell_range(keys, n, cap, i, lo, hi);
-        if (!tc_ballot(hi >= lo))
+            c[L] += s_cnt[w][L];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        if (!tc_ballot(hi[j] >= lo[j]))
             continue;
 #pragma unroll
         for (int L = 0; L < TC_LMAX; ++L) {
-            const bool f = L >= lo && L <= hi;
+            const bool f = L >= lo[j] && L <= hi[j];
             const unsigned long long b = tc_ballot(f);
             if (f) {
                 const uint32_t r = c[L] + __popcll(b & tc_lanemask_lt());
-                istart[r] = i;
+                istart[r] = base + 64 * j + tc_lane();
                 ilevel[r] = L;
             }
             c[L] += __popcll(b);
@@ -870,96 +836,105 @@ __global__ __launch_bounds__(256) void k_int_emit(const uint32_t *keys, int n, i
     }
 }
 
-// Clears every node's child field (leaves keep 0; k_int_nodes then sets the
-// internal ones) and writes the root's range, level and cell.
-__global__ __launch_bounds__(256) void k_topo_init(uint32_t *child, int nn, int n, int2 *se, int *level,
-                                                   int2 *cell)
+constexpr int NODES_WAVE_T = 16384;
+
+// The root of a tree without internal nodes (one leaf).
+__global__ void k_topo_leaf(uint32_t *child, int n, int2 *se, int *level, int2 *cell)
 {
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < nn; i += gridDim.x * 256)
-        child[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        se[0] = make_int2(0, n);
-        level[0] = 0;
-        cell[0] = make_int2(0, 0);
-    }
+    child[0] = 0u;
+    se[0] = make_int2(0, n);
+    level[0] = 0;
+    cell[0] = make_int2(0, 0);
 }
 
-__global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *keys, int n, int cap, const int *istart,
-                                                    const int *ilevel, const int *info, int T, int *selfid,
+// First position in [lo, hi) where pred is false (pred holds on a prefix of
+// the range), searched by a group of G lanes that hold the same range: G evenly
+// spread probes a round, one memory access each.
+template <int G> TC_DEV int group_count(bool ok)
+{
+    return __popcll((tc_ballot(ok) >> (tc_lane() & ~(G - 1))) & (G == 64 ? ~0ull : (1ull << G) - 1ull));
+}
+template <int G, class Pred> TC_DEV int group_partition(int lo, int hi, Pred &&pred)
+{
+    while (hi > lo) {
+        const int step = (hi - lo + G - 1) / G;
+        const int p = lo + (tc_lane() & (G - 1)) * step;
+        const int c = group_count<G>(p < hi && pred(p));
+        if (c == 0)
+            return lo;
+        const int last = lo + (c - 1) * step;  // the last probe where it held
+        hi = min(hi, last + step);
+        lo = last + 1;
+    }
+    return lo;
+}
+
+// One internal node (breadth-first rank r) per group of G lanes: its id from
+// its parent's rank, the end of its cell, the ranges of its four children.  A
+// search by one thread is a chain of some 70 dependent loads (22 us at 2^16, 56
+// us at 2^24 sources whatever the leaf size).  By a wave (G = 64) it is about
+// 8 rounds, the shortest chain, taken while the nodes are too few to fill the
+// GPU; beyond NODES_WAVE_T nodes, 16 lanes a node keep four times as many searches in
+// flight.  2^16 sources: 22 -> 7 us, 2^20: 31 -> 13 us (G = 64), 2^23: 38 -> 33 us
+// (G = 16).  Every node writes its children's records; a child that
+// is internal writes its own child field (its rank is its own), so only leaves'
+// are cleared here.
+template <int G>
+__global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ keys, int n, int cap,
+                                                    const int *__restrict__ istart, const int *__restrict__ ilevel,
+                                                    const int *__restrict__ info, int T, int *__restrict__ selfid,
                                                     uint32_t *child, int2 *se, int *level, int2 *cell)
 {
-    const int r = blockIdx.x * 256 + threadIdx.x;
+    const int r = blockIdx.x * (256 / G) + threadIdx.x / G, lane = threadIdx.x % G;
     if (r >= T)
         return;
     const int L = ilevel[r], i = istart[r];
     const uint32_t key = keys[i];
     const int sh = 2 * (TC_LMAX - L);
-    const uint32_t prefix = sh >= 32 ? 0u : (key >> sh);
-    int self = 0;
+    const uint32_t prefix = key >> sh;  // sh <= 30
+    int self = 0, e = n;
     if (L > 0) {
-        int lo = info[L - 1], hi = info[L];
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (istart[mid] <= i)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        self = 1 + 4 * (lo - 1) + (int)(prefix & 3u);
+        // the parent: the last internal cell of level L - 1 starting at or before i
+        const int l0 = info[L - 1];
+        const int pr = group_partition<G>(l0, info[L], [&](int p) { return istart[p] <= i; }) - 1;
+        self = 1 + 4 * pr + (int)(prefix & 3u);
+        // the cell's end: bracketed by doubling steps, one lane each
+        const int b0 = i + cap + 1;  // the cell holds more than cap sources
+        constexpr int NP = G < 30 ? G : 30;
+        const int o = lane < NP ? (1 << lane) - 1 : INT_MAX;
+        const bool in = o < n - b0 && (keys[b0 + o] >> sh) == prefix;
+        const int c = group_count<G>(in);  // probes 0 .. c-1 lie inside
+        const int lo = c ? b0 + (1 << (c - 1)) : b0;
+        const int hi = c < NP ? (int)min((long long)n, (long long)b0 + (1ll << c) - 1) : n;
+        e = group_partition<G>(lo, hi, [&](int p) { return (keys[p] >> sh) == prefix; });
     }
-    selfid[r] = self;
-    child[self] = (uint32_t)(1 + 4 * r);
-
-    // end of the cell: first position whose level-L prefix differs
-    int e;
-    if (L == 0) {
-        e = n;
-    } else {
-        int lo = i + cap + 1, hi = n, step = 1;
-        while (true) {
-            const int probe = lo + step - 1;
-            if (probe >= n) {
-                hi = n;
-                break;
-            }
-            if ((keys[probe] >> sh) != prefix) {
-                hi = probe;
-                break;
-            }
-            lo = probe + 1;
-            step <<= 1;
+    if (lane == 0) {
+        selfid[r] = self;
+        child[self] = (uint32_t)(1 + 4 * r);
+        if (L == 0) {
+            se[0] = make_int2(0, n);
+            level[0] = 0;
+            cell[0] = make_int2(0, 0);
         }
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if ((keys[mid] >> sh) == prefix)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        e = lo;
     }
     const int csh = sh - 2;
     int b[5];
     b[0] = i;
     b[4] = e;
+#pragma unroll
     for (int c = 1; c < 4; ++c) {
         const uint32_t target = ((prefix << 2) | (uint32_t)c) << csh;
-        int lo = b[c - 1], hi = e;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (keys[mid] < target)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        b[c] = lo;
+        b[c] = group_partition<G>(b[c - 1], e, [&](int p) { return keys[p] < target; });
     }
-    const int cx = (int)tc_compact15(prefix), cy = (int)tc_compact15(prefix >> 1);
-    for (int c = 0; c < 4; ++c) {
-        const int k = 1 + 4 * r + c;
-        se[k] = make_int2(b[c], b[c + 1]);
+    if (lane < 4) {
+        const int cs = lane == 0 ? b[0] : (lane == 1 ? b[1] : (lane == 2 ? b[2] : b[3]));
+        const int ce = lane == 0 ? b[1] : (lane == 1 ? b[2] : (lane == 2 ? b[3] : b[4]));
+        const int k = 1 + 4 * r + lane;
+        se[k] = make_int2(cs, ce);
         level[k] = L + 1;
-        cell[k] = make_int2(2 * cx + (c & 1), 2 * cy + (c >> 1));
+        cell[k] = make_int2(2 * (int)tc_compact15(prefix) + (lane & 1), 2 * (int)tc_compact15(prefix >> 1) + (lane >> 1));
+        if (ce - cs <= cap || L + 1 == TC_LMAX)
+            child[k] = 0u;
     }
 }
 
@@ -1372,24 +1347,6 @@ void tc_fill_u32(uint32_t *p, uint32_t v, size_t n, hipStream_t st)
     TC_HIP(hipGetLastError());
 }
 
-void tc_scan_exclusive_u32(const uint32_t *in, uint32_t *out, int n, uint32_t *total_d, TcScratch &ws,
-                           hipStream_t st)
-{
-    if (n <= 4 * SCAN_CHUNK) {
-        k_scan_single<<<1, SCAN_NT, 0, st>>>(in, out, n, total_d);
-        TC_HIP(hipGetLastError());
-        return;
-    }
-    const int nb = tiles_of(n, SCAN_CHUNK);
-    ws.scan_tmp.reserve(sizeof(uint32_t) * (size_t)(2 * nb + 4));
-    uint32_t *part = ws.scan_tmp.as<uint32_t>();
-    uint32_t *partx = part + nb;
-    k_scan_partial<<<nb, SCAN_NT, 0, st>>>(in, n, part);
-    k_scan_single<<<1, SCAN_NT, 0, st>>>(part, partx, nb, total_d);
-    k_scan_final<<<nb, SCAN_NT, 0, st>>>(in, out, n, partx);
-    TC_HIP(hipGetLastError());
-}
-
 void tc_upload_binomials(hipStream_t st)
 {
     std::vector<double> tab(64 * 64, 0.0);
@@ -1576,20 +1533,19 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     tc_sort_points(x, y, v, n, box, keys, perm, t.src.as<double4>(), ws, st, false, ev);
 
     // census of internal cells
-    const int nblk = tiles_of(n, 4 * TB_CHUNK);
-    ws.part.reserve(sizeof(uint32_t) * ((size_t)2 * TC_LMAX * nblk + 8));
+    const bool few = n <= TB_SMALL_N;
+    const int nblk = tiles_of(n, 256 * (few ? TB_IT_SMALL : TB_IT));
+    const int stride = (nblk + 3) & ~3;
+    ws.part.reserve(sizeof(uint32_t) * (size_t)2 * TC_LMAX * stride);
     uint32_t *cnt = ws.part.as<uint32_t>();
-    uint32_t *offs = cnt + (size_t)TC_LMAX * nblk;
-    uint32_t *total = offs + (size_t)TC_LMAX * nblk;
+    uint32_t *offs = cnt + (size_t)TC_LMAX * stride;
     ws.info.reserve(sizeof(int) * 32);
     int *info = ws.info.as<int>();
-    k_int_count<<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, nblk);
-    if (TC_LMAX * nblk <= 4 * SCAN_CHUNK) {
-        k_census_single<<<1, SCAN_NT, 0, st>>>(cnt, offs, nblk, total, tc_bbox_bad_flag(ws, n), box, info);
-    } else {
-        tc_scan_exclusive_u32(cnt, offs, TC_LMAX * nblk, total, ws, st);
-        k_level_starts<<<1, 64, 0, st>>>(offs, nblk, total, tc_bbox_bad_flag(ws, n), box, info);
-    }
+    if (few)
+        k_int_count<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, stride);
+    else
+        k_int_count<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, stride);
+    k_census<<<1, SCAN_NT, 0, st>>>(cnt, offs, nblk, stride, tc_bbox_bad_flag(ws, n), box, info);
     TC_HIP(hipGetLastError());
     static_assert(INFO_BYTES <= sizeof(int) * 32 && INFO_BYTES <= TcScratch::PINNED_BYTES, "census record size");
     char *hp = static_cast<char *>(ws.host_pinned());
@@ -1628,11 +1584,18 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     int *lev = reinterpret_cast<int *>(se + nn);
     int2 *cell = reinterpret_cast<int2 *>(lev + ((nn + 1) & ~1));
 
-    k_topo_init<<<std::min(tiles_of(nn, 256), 4096), 256, 0, st>>>(child, nn, n, se, lev, cell);
     if (T > 0) {
-        k_int_emit<<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, nblk, ws.istart.as<int>(), ws.ilevel.as<int>());
-        k_int_nodes<<<tiles_of(T, 256), 256, 0, st>>>(keys, n, leafcap, ws.istart.as<int>(), ws.ilevel.as<int>(),
-                                                      info, T, t.selfid.as<int>(), child, se, lev, cell);
+        if (few)
+            k_int_emit<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, ws.istart.as<int>(),
+                                                           ws.ilevel.as<int>());
+        else
+            k_int_emit<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, ws.istart.as<int>(),
+                                                     ws.ilevel.as<int>());
+        const auto nodes_kernel = T <= NODES_WAVE_T ? k_int_nodes<64> : k_int_nodes<16>;
+        nodes_kernel<<<T <= NODES_WAVE_T ? tiles_of(T, 4) : tiles_of(T, 16), 256, 0, st>>>(keys, n, leafcap, ws.istart.as<int>(), ws.ilevel.as<int>(), info,
+                                                    T, t.selfid.as<int>(), child, se, lev, cell);
+    } else {
+        k_topo_leaf<<<1, 1, 0, st>>>(child, n, se, lev, cell);
     }
     TC_HIP(hipGetLastError());
     if (ev)

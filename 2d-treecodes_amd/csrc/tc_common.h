@@ -301,7 +301,7 @@ struct TcTree {
 
 // Scratch reused across calls of one context.
 struct TcScratch {
-    DevBuf k2, v2, hist, part, scan_tmp, istart, ilevel, info, tkeys, tperm, tsorted, bbox_part, ints, packed, work,
+    DevBuf k2, v2, hist, part, istart, ilevel, info, tkeys, tperm, tsorted, bbox_part, ints, packed, work,
         flist;
     // pinned host memory for the per-solve readbacks (tree census, flags): a
     // copy into pageable memory costs a staged transfer of its own
@@ -315,7 +315,7 @@ struct TcScratch {
     }
     void release()
     {
-        for (DevBuf *b : {&k2, &v2, &hist, &part, &scan_tmp, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
+        for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
                           &bbox_part, &ints, &packed, &work, &flist})
             b->release();
         if (pinned)
@@ -326,7 +326,7 @@ struct TcScratch {
     // exist (host_pinned() at set-up), so no call made with this scratch allocates.
     void bind(TcArena *a)
     {
-        for (DevBuf *b : {&k2, &v2, &hist, &part, &scan_tmp, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
+        for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
                           &bbox_part, &ints, &packed, &work, &flist})
             b->bind(a);
     }
@@ -454,7 +454,5 @@ void tc_copy16(const void *src, void *dst, size_t bytes, hipStream_t st);
 void tc_direct_sums(const double *xs, const double *ys, const double *vs, int n, const double *xt,
                     const double *yt, const int *idx, int nidx, int force, double *out0, double *out1,
                     hipStream_t st);
-void tc_scan_exclusive_u32(const uint32_t *in, uint32_t *out, int n, uint32_t *total_d, TcScratch &ws,
-                           hipStream_t st);
 void tc_fill_u32(uint32_t *p, uint32_t v, size_t n, hipStream_t st);
 void tc_upload_binomials(hipStream_t st);

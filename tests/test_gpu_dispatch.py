@@ -1,0 +1,19 @@
+"""Both sides of the size rules that choose between kernel variants, against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import compare_tree, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+# census items per wave (2^20 sources), lanes per node of the topology search (16,384 internal
+# nodes), blocks of 1,024 and 4,096 positions, one-source leaves down to level 15, a lone leaf
+@pytest.mark.parametrize("n,leaf", [(1, 1), (2, 1), (64, 1), (1023, 1), (1025, 3), (4097, 1), (20000, 1),
+                                    (1 << 20, 32), ((1 << 20) + 1, 512), ((1 << 20) + 4095, 24)])
+def test_topology_variants(pkg, oracle, wl, n, leaf):
+    xs, ys, vs, *_ = wl.mixed_plummer_potential(n, seed=n % 97)
+    ctx = pkg.Context(pot_order=6, pot_leaf=leaf)
+    ctx.potential(0.5, xs, ys, vs, xs[:1], ys[:1])
+    compare_tree(ctx.tree(), oracle.Tree(xs, ys, vs, leaf, 6))
+    ctx.close()
