@@ -878,12 +878,13 @@ template <int G, class Pred> TC_DEV int group_partition(int lo, int hi, Pred &&p
 // flight.  2^16 sources: 22 -> 7 us, 2^20: 31 -> 13 us (G = 64), 2^23: 38 -> 33 us
 // (G = 16).  Every node writes its children's records; a child that
 // is internal writes its own child field (its rank is its own), so only leaves'
-// are cleared here.
+// are cleared here.  Leaves the parent's rank in ilevel and the count of
+// internal children in pend for the upward pass.
 template <int G>
 __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ keys, int n, int cap,
-                                                    const int *__restrict__ istart, const int *__restrict__ ilevel,
+                                                    const int *__restrict__ istart, int *ilevel,
                                                     const int *__restrict__ info, int T, int *__restrict__ selfid,
-                                                    uint32_t *child, int2 *se, int *level, int2 *cell)
+                                                    uint32_t *pend, uint32_t *child, int2 *se, int *level, int2 *cell)
 {
     const int r = blockIdx.x * (256 / G) + threadIdx.x / G, lane = threadIdx.x % G;
     if (r >= T)
@@ -892,12 +893,12 @@ __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ 
     const uint32_t key = keys[i];
     const int sh = 2 * (TC_LMAX - L);
     const uint32_t prefix = key >> sh;  // sh <= 30
-    int self = 0, e = n;
+    int self = 0, up = 0, e = n;
     if (L > 0) {
         // the parent: the last internal cell of level L - 1 starting at or before i
         const int l0 = info[L - 1];
-        const int pr = group_partition<G>(l0, info[L], [&](int p) { return istart[p] <= i; }) - 1;
-        self = 1 + 4 * pr + (int)(prefix & 3u);
+        up = group_partition<G>(l0, info[L], [&](int p) { return istart[p] <= i; }) - 1;
+        self = 1 + 4 * up + (int)(prefix & 3u);
         // the cell's end: bracketed by doubling steps, one lane each
         const int b0 = i + cap + 1;  // the cell holds more than cap sources
         constexpr int NP = G < 30 ? G : 30;
@@ -910,6 +911,7 @@ __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ 
     }
     if (lane == 0) {
         selfid[r] = self;
+        ilevel[r] = up;  // read by this wave alone, above
         child[self] = (uint32_t)(1 + 4 * r);
         if (L == 0) {
             se[0] = make_int2(0, n);
@@ -926,6 +928,7 @@ __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ 
         const uint32_t target = ((prefix << 2) | (uint32_t)c) << csh;
         b[c] = group_partition<G>(b[c - 1], e, [&](int p) { return keys[p] < target; });
     }
+    bool inner = false;
     if (lane < 4) {
         const int cs = lane == 0 ? b[0] : (lane == 1 ? b[1] : (lane == 2 ? b[2] : b[3]));
         const int ce = lane == 0 ? b[1] : (lane == 1 ? b[2] : (lane == 2 ? b[3] : b[4]));
@@ -933,9 +936,13 @@ __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ 
         se[k] = make_int2(cs, ce);
         level[k] = L + 1;
         cell[k] = make_int2(2 * (int)tc_compact15(prefix) + (lane & 1), 2 * (int)tc_compact15(prefix >> 1) + (lane >> 1));
-        if (ce - cs <= cap || L + 1 == TC_LMAX)
+        inner = ce - cs > cap && L + 1 < TC_LMAX;
+        if (!inner)
             child[k] = 0u;
     }
+    const uint32_t ni = (uint32_t)group_count<G>(inner);
+    if (lane == 0)
+        pend[r] = ni << 8 | ni;
 }
 
 // Reduce-scatter form of the pairwise lane tree: at offsets 32, 16, ..., 1 a
@@ -1092,206 +1099,290 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
 // Parent update of upward.cpp:95-218 and upward_e2e (upward-kernels.m4:95-149)
 // for internal node `rank`, by one wavefront.  The children's translations run
 // in parallel: lane group g (E2E_G lanes: 16 for p <= 16, else 32) takes child
-// g of a round, one lane of it forms the powers z0^-j by the reference's
-// recurrence, lane l the coefficient l+1.  Each child's contribution lands in
-// LDS and lanes add them in order c = 0..3, so every coefficient is formed by
-// the same operations as a child-by-child loop.
+// g of a round, lane l of it the coefficient l + 1.  Every lane runs the
+// reference's recurrence for the powers z0^-j itself and keeps the one it
+// needs (two dependent operations a step, no LDS round trip), and the binomials
+// come from a table in LDS: read from memory inside the sum they were most of
+// the kernel's time (one cache round trip per term).  Each child's contribution lands
+// in LDS and lanes add them in order c = 0..3, so every coefficient is formed
+// by the same operations as a child-by-child loop.
 template <int P> constexpr int E2E_G = P <= 16 ? 16 : 32;
 
-template <int P> struct E2eLds {
-    double rinv[64 / E2E_G<P>][P + 1], iinv[64 / E2E_G<P>][P + 1];
-    double rc[64 / E2E_G<P>][P + 1], ic[64 / E2E_G<P>][P + 1];
-    double cre[4][P], cim[4][P];
-};
+// C(l, k) at [k * P + l], k <= l < P: lane l reads consecutive words
+template <int P> TC_DEV void e2e_binom(double *s_binom)
+{
+    for (int i = threadIdx.x; i < P * P; i += blockDim.x)
+        s_binom[i] = c_binom[(i % P) * 64 + i / P];
+}
 
-template <int P>
-TC_DEV void e2e_node(int rank, const int *selfid, const int2 *se, const int *level, const int2 *cell,
-                     const double *box, TcNode *nodes, double4 *nodew, double *exps, E2eLds<P> &L)
+// Node data passed between waves of one launch: agent-scope accesses go past
+// the XCDs' own L2s, which are not coherent with each other.
+template <bool AGENT> TC_DEV unsigned long long node_load_u64(const void *p)
+{
+    const unsigned long long *q = static_cast<const unsigned long long *>(p);
+    return AGENT ? __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *q;
+}
+template <bool AGENT> TC_DEV double node_load(const double *p)
+{
+    return __longlong_as_double((long long)node_load_u64<AGENT>(p));
+}
+template <bool AGENT> TC_DEV void node_store(double *p, double v)
+{
+    if (AGENT)
+        __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), (unsigned long long)__double_as_longlong(v),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        *p = v;
+}
+
+// CHAIN: a child was written by this launch; else all by earlier ones (plain,
+// cached loads).  SHARED: another wave of this launch may read the node.
+template <int P, bool CHAIN, bool SHARED>
+TC_DEV void e2e_node(int rank, const int *selfid, const double *box, TcNode *nodes, double4 *nodew, double *exps,
+                     double2 (*s_a)[P], double *s_rec, const double *s_binom,
+                     double ninv)
 {
     constexpr int G = E2E_G<P>, NCH = 64 / G;
     const int lane = tc_lane();
     const int grp = lane / G, gl = lane % G;
-    const int id = selfid[rank];
     const int cb = 1 + 4 * rank;
-    const int l = level[id];
-    const int2 cc = cell[id];
+    const int id = selfid[rank];
+
+    // the children's records (256 contiguous bytes) and weights (128), a word
+    // per lane, and this lane's coefficients: one round of loads.  Level, cell
+    // and source range follow from the children's.
+    unsigned long long rec = 0;
+    if (lane < 48)
+        rec = node_load_u64<CHAIN>(lane < 32 ? reinterpret_cast<const double *>(nodes + cb) + lane
+                                             : reinterpret_cast<const double *>(nodew + cb) + (lane - 32));
+    double2 co[4 / NCH];
+#pragma unroll
+    for (int q = 0; q < 4 / NCH; ++q) {
+        const double *ca = exps + (size_t)2 * P * (cb + q * NCH + grp);
+        co[q] = gl < P ? make_double2(node_load<CHAIN>(ca + gl), node_load<CHAIN>(ca + P + gl)) : make_double2(0.0, 0.0);
+    }
+    if (lane < 48)
+        s_rec[lane] = __longlong_as_double((long long)rec);
+    tc_wave_sync();
+    auto word = [&](int k) { return (unsigned long long)__double_as_longlong(s_rec[k]); };
+    const unsigned long long se0 = word(4), se3 = word(8 * 3 + 4), cl0 = word(5), cc0 = word(6);
+    const int2 range = make_int2((int)(unsigned)se0, (int)(se3 >> 32));
+    const int l = (int)(cl0 >> 32) - 1;
+    const int2 cc = make_int2((int)(unsigned)cc0 >> 1, (int)(cc0 >> 32) >> 1);
     const double xmin = box[0], ymin = box[1], ext = box[2];
 
-    TcNode ch[4];
-    double4 cw[4];
     double msum = 0, wsum = 0, wxsum = 0, wysum = 0;
-    for (int c = 0; c < 4; ++c) {
-        ch[c] = nodes[cb + c];
-        cw[c] = nodew[cb + c];
-        msum += ch[c].mass;
-        wsum += cw[c].x;
-        wxsum += cw[c].y;
-        wysum += cw[c].z;
-    }
-    const double h = ext / (double)(1 << l);
-    const double xcp = wsum != 0 ? wxsum / wsum : (xmin + h * (double)cc.x) + 0.5 * h;
-    const double ycp = wsum != 0 ? wysum / wsum : (ymin + h * (double)cc.y) + 0.5 * h;
-    double rr = 0;
-    for (int c = 0; c < 4; ++c) {
-        if (cw[c].x != 0) {
-            const double rx = xcp - ch[c].xcom, ry = ycp - ch[c].ycom;
-            const double v = ch[c].r + sqrt(rx * rx + ry * ry);
-            rr = rr < v ? v : rr;
-        }
-    }
-    const double rcap = (double)1.4143f * ext / (double)(1 << l);
-    const double rad = rcap < rr ? rcap : rr;
-
     int zcount = 0, nz = 0;
+#pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const bool neg = fabs(cw[c].x) < 1.1e-16;
+        const double w = s_rec[32 + 4 * c];
+        msum += s_rec[8 * c + 3];
+        wsum += w;
+        wxsum += s_rec[32 + 4 * c + 1];
+        wysum += s_rec[32 + 4 * c + 2];
+        const bool neg = fabs(w) < 1.1e-16;
         zcount += neg;
         if (!neg)
             nz = c;
     }
+    // (scaling by 2^-l rounds as dividing by 2^l does)
+    const double h = ldexp(ext, -l);
+    const double xcp = wsum != 0 ? wxsum / wsum : (xmin + h * (double)cc.x) + 0.5 * h;
+    const double ycp = wsum != 0 ? wysum / wsum : (ymin + h * (double)cc.y) + 0.5 * h;
+    // radius: lanes c, c + 4, ... take child c; the maximum over the four
+    double rr = 0;
+    {
+        const int c = lane & 3;
+        const double rx = xcp - s_rec[8 * c], ry = ycp - s_rec[8 * c + 1];
+        const double v = s_rec[8 * c + 2] + sqrt(rx * rx + ry * ry);
+        rr = s_rec[32 + 4 * c] != 0 && rr < v ? v : rr;
+#pragma unroll
+        for (int off = 1; off < 4; off <<= 1) {
+            const double o = __shfl_xor(rr, off, 64);
+            rr = rr < o ? o : rr;
+        }
+    }
+    const double rcap = ldexp((double)1.4143f * ext, -l);
+    const double rad = rcap < rr ? rcap : rr;
+
     double dre = 0, dim = 0;
     if (zcount == 3) {
         if (lane < P) {
-            dre = exps[(size_t)2 * P * (cb + nz) + lane];
-            dim = exps[(size_t)2 * P * (cb + nz) + P + lane];
+            dre = node_load<CHAIN>(exps + (size_t)2 * P * (cb + nz) + lane);
+            dim = node_load<CHAIN>(exps + (size_t)2 * P * (cb + nz) + P + lane);
         }
     } else if (zcount < 3) {
-        for (int c0 = 0; c0 < 4; c0 += NCH) {
-            // this lane's child (the index differs between lane groups, so it
-            // is loaded rather than picked out of ch[], which would go to scratch)
-            const int c = c0 + grp;
-            const TcNode chc = nodes[cb + c];
-            const bool act = nodew[cb + c].x != 0;
-            const double x0 = chc.xcom - xcp, y0 = chc.ycom - ycp;
-            const bool ident = x0 == 0 && y0 == 0;
-            const double *ca = exps + (size_t)2 * P * (cb + c);
-            // the child's coefficients, requested now so that the load overlaps
-            // the powers of 1/z0 below
-            double car = 0, cai = 0;
-            if (act && gl < P) {
-                car = ca[gl];
-                cai = ca[P + gl];
-            }
-            if (act && !ident && gl == 0) {
-                const double r2z0 = x0 * x0 + y0 * y0;
-                const double ri1 = x0 / r2z0, ii1 = -y0 / r2z0;
-                double ri = ri1, ii = ii1;
-                L.rinv[grp][1] = ri;
-                L.iinv[grp][1] = ii;
-                for (int j = 2; j <= P; ++j) {
-                    const double rn = ri * ri1 - ii * ii1;
-                    const double in = ri * ii1 + ii * ri1;
-                    ri = rn;
-                    ii = in;
-                    L.rinv[grp][j] = ri;
-                    L.iinv[grp][j] = ii;
-                }
-            }
-            tc_wave_sync();
-            if (act && !ident && gl < P) {
-                const int jj = gl + 1;
-                L.rc[grp][jj] = car * L.rinv[grp][jj] - cai * L.iinv[grp][jj];
-                L.ic[grp][jj] = car * L.iinv[grp][jj] + cai * L.rinv[grp][jj];
-            }
-            tc_wave_sync();
-            if (gl < P) {
-                double cre = 0, cim = 0;
-                if (act && ident) {
-                    cre = car;
-                    cim = cai;
-                } else if (act) {
-                    const int ll = gl + 1;
-                    const double mass = chc.mass;
-                    double rt = (ll == 1) ? -mass : mass * (-(1.0 / (double)ll));
-                    double it = L.ic[grp][1];
-                    rt = rt + L.rc[grp][1];
-                    for (int k = 2; k <= ll; ++k) {
-                        const double bk = c_binom[(ll - 1) * 64 + (k - 1)];
-                        rt = rt + L.rc[grp][k] * bk;
-                        it = it + L.ic[grp][k] * bk;
-                    }
-                    const double ri = L.rinv[grp][ll], ii = L.iinv[grp][ll];
-                    const double invz2 = ri * ri + ii * ii;
-                    const double invinv = invz2 != 0 ? 1 / invz2 : 0;
-                    const double rz = ri * invinv;
-                    const double iz = -ii * invinv;
-                    cre = rt * rz - it * iz;
-                    cim = rt * iz + it * rz;
-                }
-                L.cre[c][gl] = cre;
-                L.cim[c][gl] = cim;
-            }
-            tc_wave_sync();
+        double zr[4 / NCH], zi[4 / NCH], mq[4 / NCH];  // z0^-(gl + 1); the child's mass
+        double r1[4 / NCH], i1[4 / NCH], rj[4 / NCH], ij[4 / NCH];
+        bool act[4 / NCH], ident[4 / NCH];
+#pragma unroll
+        for (int q = 0; q < 4 / NCH; ++q) {
+            const int c = q * NCH + grp;  // this lane's child
+            const double x0 = s_rec[8 * c] - xcp, y0 = s_rec[8 * c + 1] - ycp;
+            mq[q] = s_rec[8 * c + 3];
+            act[q] = s_rec[32 + 4 * c] != 0;
+            ident[q] = x0 == 0 && y0 == 0;
+            const double r2z0 = x0 * x0 + y0 * y0;
+            zr[q] = rj[q] = r1[q] = x0 / r2z0;
+            zi[q] = ij[q] = i1[q] = -y0 / r2z0;
         }
-        if (lane < P) {
-            for (int c = 0; c < 4; ++c) {
-                if (cw[c].x == 0)
-                    continue;
-                dre += L.cre[c][lane];
-                dim += L.cim[c][lane];
+#pragma unroll 4
+        for (int j = 1; j < P; ++j) {
+#pragma unroll
+            for (int q = 0; q < 4 / NCH; ++q) {
+                const double rn = rj[q] * r1[q] - ij[q] * i1[q];
+                const double in = rj[q] * i1[q] + ij[q] * r1[q];
+                rj[q] = rn;
+                ij[q] = in;
+                zr[q] = j == gl ? rn : zr[q];
+                zi[q] = j == gl ? in : zi[q];
             }
+        }
+#pragma unroll
+        for (int q = 0; q < 4 / NCH; ++q)
+            if (gl < P)
+                s_a[q * NCH + grp][gl] = make_double2(co[q].x * zr[q] - co[q].y * zi[q],
+                                                      co[q].x * zi[q] + co[q].y * zr[q]);
+        tc_wave_sync();
+        double2 res[4 / NCH];
+#pragma unroll
+        for (int q = 0; q < 4 / NCH; ++q) {
+            const double2 *a = s_a[q * NCH + grp];
+            double rt = mq[q] * ninv;
+            double it = a[0].y;
+            rt = rt + a[0].x;
+#pragma unroll 4
+            for (int k = 1; k < P; ++k) {
+                if (k <= gl && gl < P) {
+                    const double bk = s_binom[k * P + gl];
+                    rt = rt + a[k].x * bk;
+                    it = it + a[k].y * bk;
+                }
+            }
+            const double invz2 = zr[q] * zr[q] + zi[q] * zi[q];
+            const double invinv = invz2 != 0 ? 1 / invz2 : 0;
+            const double rz = zr[q] * invinv;
+            const double iz = -zi[q] * invinv;
+            res[q] = make_double2(rt * rz - it * iz, rt * iz + it * rz);
+            // z0 = 0 translates by the identity; w = 0 children add nothing
+            if (!act[q])
+                res[q] = make_double2(0.0, 0.0);
+            else if (ident[q])
+                res[q] = co[q];
         }
         tc_wave_sync();
+#pragma unroll
+        for (int q = 0; q < 4 / NCH; ++q)
+            if (gl < P)
+                s_a[q * NCH + grp][gl] = res[q];
+        tc_wave_sync();
+        if (lane < P) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const double2 v = s_a[c][lane];
+                dre = s_rec[32 + 4 * c] != 0 ? dre + v.x : dre;
+                dim = s_rec[32 + 4 * c] != 0 ? dim + v.y : dim;
+            }
+        }
     }
     if (lane < P) {
-        exps[(size_t)2 * P * id + lane] = dre;
-        exps[(size_t)2 * P * id + P + lane] = dim;
+        node_store<SHARED>(exps + (size_t)2 * P * id + lane, dre);
+        node_store<SHARED>(exps + (size_t)2 * P * id + P + lane, dim);
     }
+    // the record and weights, a word per lane again
+    tc_wave_sync();
     if (lane == 0) {
-        const int2 r = se[id];
-        TcNode nd;
-        nd.xcom = xcp;
-        nd.ycom = ycp;
-        nd.r = rad;
-        nd.mass = msum;
-        nd.s = r.x;
-        nd.e = r.y;
-        nd.child = cb;
-        nd.level = l;
-        nd.cx = cc.x;
-        nd.cy = cc.y;
-        nd.rr = rad * rad;
-        nodes[id] = nd;
-        nodew[id] = make_double4(wsum, wxsum, wysum, 0.0);
+        auto pair = [](int lo, int hi) {
+            return __longlong_as_double((long long)((unsigned)lo | ((unsigned long long)(unsigned)hi << 32)));
+        };
+        s_rec[0] = xcp;
+        s_rec[1] = ycp;
+        s_rec[2] = rad;
+        s_rec[3] = msum;
+        s_rec[4] = pair(range.x, range.y);
+        s_rec[5] = pair(cb, l);
+        s_rec[6] = pair(cc.x, cc.y);
+        s_rec[7] = rad * rad;
+        s_rec[8] = wsum;
+        s_rec[9] = wxsum;
+        s_rec[10] = wysum;
+        s_rec[11] = 0.0;
     }
+    tc_wave_sync();
+    if (lane < 12)
+        node_store<SHARED>(lane < 8 ? reinterpret_cast<double *>(nodes + id) + lane
+                                    : reinterpret_cast<double *>(nodew + id) + (lane - 8),
+                           s_rec[lane]);
+    tc_wave_sync();  // s_a and s_rec are rewritten for the wave's next node
+}
+static_assert(offsetof(TcNode, mass) == 24 && offsetof(TcNode, s) == 32 && offsetof(TcNode, child) == 40 &&
+                  offsetof(TcNode, cx) == 48 && offsetof(TcNode, rr) == 56,
+              "e2e_node moves records as 8-byte words");
+
+// One wavefront per internal node of one level (ranks r0 .. r1 - 1).
+template <int P>
+__global__ __launch_bounds__(256) void k_e2e_level(const int *__restrict__ selfid, int r0, int r1,
+                                                   const double *__restrict__ box, TcNode *nodes, double4 *nodew,
+                                                   double *exps)
+{
+    __shared__ double s_binom[P * P];
+    __shared__ double2 s_a[4][4][P];
+    __shared__ double s_rec[4][48];
+    e2e_binom<P>(s_binom);
+    __syncthreads();
+    const int wid = threadIdx.x >> 6, rank = tc_uniform(r0 + (int)blockIdx.x * 4 + wid);
+    if (rank < r1)
+        e2e_node<P, false, false>(rank, selfid, box, nodes, nodew, exps, s_a[wid], s_rec[wid], s_binom,
+                                  -(1.0 / (double)(tc_lane() % E2E_G<P> + 1)));
 }
 
-// One wavefront per internal node of one level (ranks r0..r1-1).
+// The top T internal nodes in one launch, children before parents; those from
+// rank tlast on (their level's children come from k_e2e_level) and those whose
+// children are all leaves are the starting points, one wave each.  pend[r] =
+// (internal children of rank r) << 8 | (of these, not finished yet), parent[r]
+// its parent's rank (k_int_nodes).  After a node its wave takes one off the
+// parent's count; the wave that takes the last goes on with the parent, the
+// others leave, so no wave ever waits for another.  A node's stores have
+// completed (vmcnt 0) before its parent's count is taken off.  A level costs
+// about 4 us of latency here, but agent-scope traffic makes a node dearer
+// (3 ns against 1.5 at 2^24 sources), so levels that fill the GPU go level by
+// level and E2E_CHAIN_T nodes or fewer this way.  Upward pass above the leaves,
+// with one launch per level above 64 nodes and one workgroup for the levels
+// below it (bound by one CU's FP64 rate): 235 -> 146 us at 2^24 sources (order 9),
+// 142 -> 90 at 2^23 (order 8), 45 -> 17 at 2^16 (order 12), 71 -> 37 at 10,000
+// (order 24).
+constexpr int E2E_CHAIN_T = 4096;
 template <int P>
-__global__ __launch_bounds__(64) void k_e2e_level(const int *selfid, int r0, int r1, const int2 *se,
-                                                   const int *level, const int2 *cell, const double *box,
-                                                   TcNode *nodes, double4 *nodew, double *exps)
+__global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, const int *__restrict__ parent,
+                                             uint32_t *pend, int T, int tlast, const double *__restrict__ box,
+                                             TcNode *nodes, double4 *nodew, double *exps)
 {
-    __shared__ E2eLds<P> L;
-    const int rank = r0 + blockIdx.x;
-    if (rank >= r1)
-        return;
-    e2e_node<P>(rank, selfid, se, level, cell, box, nodes, nodew, exps, L);
-}
-
-// The small top levels in one launch: levels lt-1 .. 0 (ranks starts[L] ..
-// starts[L+1]-1, at most 4 nodes per wave each), E2E_TOP_WAVES waves striding
-// over a level's nodes, a workgroup barrier between levels (children before
-// parents).
-constexpr int E2E_TOP_WAVES = 16;
-template <int P>
-__global__ __launch_bounds__(64 * E2E_TOP_WAVES) void k_e2e_top(const int *selfid, const int *starts, int lt,
-                                                                 const int2 *se, const int *level,
-                                                                 const int2 *cell, const double *box,
-                                                                 TcNode *nodes, double4 *nodew, double *exps)
-{
-    __shared__ E2eLds<P> L[E2E_TOP_WAVES];
+    __shared__ double s_binom[P * P];
+    __shared__ double2 s_a[4][4][P];
+    __shared__ double s_rec[4][48];
     const int wid = threadIdx.x >> 6;
-    for (int lv = lt - 1; lv >= 0; --lv) {
-        const int r0 = starts[lv], r1 = starts[lv + 1];
-        for (int rank = r0 + wid; rank < r1; rank += E2E_TOP_WAVES)
-            e2e_node<P>(rank, selfid, se, level, cell, box, nodes, nodew, exps, L[wid]);
-        // the next level reads what this one wrote; the readers are waves of
-        // this workgroup, which share one CU and its vector L1, so the
-        // barrier's workgroup-scope release / acquire orders the global
-        // writes (device-scope fences would write back and invalidate caches
-        // at every level)
-        __syncthreads();
+    int rank = tc_uniform((int)(blockIdx.x * 4 + wid));
+    const bool start = rank < T && (rank >= tlast || (pend[rank] >> 8) == 0);
+    if (!__syncthreads_or(start))
+        return;
+    e2e_binom<P>(s_binom);
+    __syncthreads();
+    if (!start)
+        return;
+    const double ninv = -(1.0 / (double)(tc_lane() % E2E_G<P> + 1));  // -1 / (this lane's coefficient index)
+    e2e_node<P, false, true>(rank, selfid, box, nodes, nodew, exps, s_a[wid], s_rec[wid], s_binom, ninv);
+    while (rank != 0) {
+        const int up = tc_uniform(parent[rank]);
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // and no store moves below (a compiler fence here)
+        uint32_t left = 0;
+        if (tc_lane() == 0)
+            left = __hip_atomic_fetch_sub(&pend[up], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffu;
+        if (tc_uniform((int)left) != 1)
+            break;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        rank = up;
+        e2e_node<P, true, true>(rank, selfid, box, nodes, nodew, exps, s_a[wid], s_rec[wid], s_binom, ninv);
     }
 }
 
@@ -1470,7 +1561,7 @@ void tc_morton_sort(const double *x, const double *y, const double *v, int n, co
 
 template <int P>
 static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, const int *lev, const int2 *cell,
-                          const int *selfid, const int *starts_d, bool fp32, bool deriv, hipStream_t st)
+                          const int *parent, uint32_t *pend, bool fp32, bool deriv, hipStream_t st)
 {
     const double *box = t.box_d.as<double>();
     k_leaf_upward<P><<<tiles_of(t.nnodes, 4), 256, 0, st>>>(child, se, lev, cell, t.src.as<double4>(), box,
@@ -1478,22 +1569,23 @@ static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, cons
                                                              t.nodew.as<double4>(),
                                                              fp32 ? t.src32.as<float4>() : nullptr);
     TC_HIP(hipGetLastError());
-    // levels whose node count is small run together in one launch
-    int lt = 0;
-    while (lt < TC_LMAX && t.level_start[lt + 1] - t.level_start[lt] <= 4 * E2E_TOP_WAVES)
-        ++lt;
+    // levels lt and below one launch each, the levels above in one
+    int lt = TC_LMAX;
+    while (t.level_start[lt] > E2E_CHAIN_T)
+        --lt;
     for (int L = TC_LMAX - 1; L >= lt; --L) {
         const int r0 = t.level_start[L], r1 = t.level_start[L + 1];
         if (r1 > r0) {
-            k_e2e_level<P><<<r1 - r0, 64, 0, st>>>(selfid, r0, r1, se, lev, cell, box, t.nodes.as<TcNode>(),
-                                                    t.nodew.as<double4>(), t.exps.as<double>());
+            k_e2e_level<P><<<tiles_of(r1 - r0, 4), 256, 0, st>>>(t.selfid.as<int>(), r0, r1, box, t.nodes.as<TcNode>(),
+                                                                  t.nodew.as<double4>(), t.exps.as<double>());
             TC_HIP(hipGetLastError());
         }
     }
-    if (lt > 0 && t.level_start[lt] > 0) {
-        k_e2e_top<P><<<1, 64 * E2E_TOP_WAVES, 0, st>>>(selfid, starts_d, lt, se, lev, cell, box,
-                                                       t.nodes.as<TcNode>(), t.nodew.as<double4>(),
-                                                       t.exps.as<double>());
+    if (t.ninternal > 0) {
+        const int T = t.level_start[lt];
+        k_e2e<P><<<tiles_of(T, 4), 256, 0, st>>>(t.selfid.as<int>(), parent, pend, T,
+                                                 lt < TC_LMAX ? t.level_start[lt - 1] : T, box, t.nodes.as<TcNode>(),
+                                                 t.nodew.as<double4>(), t.exps.as<double>());
         TC_HIP(hipGetLastError());
     }
     if (fp32) {
@@ -1575,7 +1667,8 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     t.selfid.reserve(sizeof(int) * (size_t)(T + 1));
     if (fp32)
         t.exps32.reserve(sizeof(float2) * (size_t)(order + 1) * nn);
-    ws.istart.reserve(sizeof(int) * (size_t)(T + 1));
+    ws.istart.reserve(sizeof(int) * 2 * (size_t)(T + 1));
+    uint32_t *pend = ws.istart.as<uint32_t>() + T + 1;
     ws.ilevel.reserve(sizeof(int) * (size_t)(T + 1));
     // per-node topology scratch: child | se | level | cell
     ws.ints.reserve(sizeof(int) * (size_t)nn * 6 + 64);
@@ -1593,7 +1686,7 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
                                                      ws.ilevel.as<int>());
         const auto nodes_kernel = T <= NODES_WAVE_T ? k_int_nodes<64> : k_int_nodes<16>;
         nodes_kernel<<<T <= NODES_WAVE_T ? tiles_of(T, 4) : tiles_of(T, 16), 256, 0, st>>>(keys, n, leafcap, ws.istart.as<int>(), ws.ilevel.as<int>(), info,
-                                                    T, t.selfid.as<int>(), child, se, lev, cell);
+                                                    T, t.selfid.as<int>(), pend, child, se, lev, cell);
     } else {
         k_topo_leaf<<<1, 1, 0, st>>>(child, n, se, lev, cell);
     }
@@ -1601,10 +1694,9 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     if (ev)
         TC_HIP(hipEventRecord(ev[2], st));
 
-    const int *sid = t.selfid.as<int>();
     switch (order) {
 #define TC_CASE(P) \
-    case P: upward_launch<P>(t, child, se, lev, cell, sid, info, fp32, deriv32, st); break;
+    case P: upward_launch<P>(t, child, se, lev, cell, ws.ilevel.as<int>(), pend, fp32, deriv32, st); break;
         TC_ORDERS(TC_CASE)
 #undef TC_CASE
     }

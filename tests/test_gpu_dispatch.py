@@ -17,3 +17,15 @@ def test_topology_variants(pkg, oracle, wl, n, leaf):
     ctx.potential(0.5, xs, ys, vs, xs[:1], ys[:1])
     compare_tree(ctx.tree(), oracle.Tree(xs, ys, vs, leaf, 6))
     ctx.close()
+
+
+# the upward pass above the leaves: every level in the chained launch (at most 4,096 internal
+# nodes), the lower ones level by level beyond; one order per lane-group width
+@pytest.mark.parametrize("n,leaf,order", [(3, 1, 6), (5000, 1, 16), (60000, 16, 20), (200000, 12, 16),
+                                          (300000, 8, 32), (100000, 1, 9)])
+def test_upward_variants(pkg, oracle, wl, n, leaf, order):
+    xs, ys, vs, *_ = wl.mixed_plummer_potential(n, seed=order)
+    ctx = pkg.Context(force_order=order, force_leaf=leaf)
+    ctx.force(0.5, xs, ys, vs, np.array([0.4]), np.array([0.4]), np.array([1.0 / 512]))
+    compare_tree(ctx.tree(), oracle.Tree(xs, ys, vs, leaf, order))
+    ctx.close()
