@@ -1115,16 +1115,17 @@ TC_API int tc_potential_batch_resident(tc_context *const *ctxs, int k, const dou
             TC_HIP(hipHostMalloc(&c0->sdesc_host, sizeof(TcSortDesc) * TcBatchWs::MAXREQ, hipHostMallocDefault));
         c0->sdesc.reserve(sizeof(TcSortDesc) * TcBatchWs::MAXREQ);
         TcSortDesc *sd = static_cast<TcSortDesc *>(c0->sdesc_host);
-        int nsmall = 0;
+        int nsmall = 0, mmax = 0;
         for (int i = 0; i < k; ++i) {
-            if (m[i] > 0 && m[i] <= TC_SORT_SMALL_MAX)
+            if (m[i] > 0 && m[i] <= TC_SORT_SMALL_MAX) {
                 sd[nsmall++] = tc_sort_targets_desc(xt[i], yt[i], m[i], ctxs[i]->tws);
-            else if (m[i] > 0)
+                mmax = std::max(mmax, m[i]);
+            } else if (m[i] > 0)
                 tc_sort_targets(xt[i], yt[i], m[i], ctxs[i]->tws, st);
         }
         if (nsmall) {
             TC_HIP(hipMemcpyAsync(c0->sdesc.ptr, sd, sizeof(TcSortDesc) * nsmall, hipMemcpyHostToDevice, st));
-            tc_sort_targets_batch(c0->sdesc.as<TcSortDesc>(), nsmall, st);
+            tc_sort_targets_batch(c0->sdesc.as<TcSortDesc>(), nsmall, mmax, st);
         }
         std::vector<TcPotBatchItem> items;
         for (int i = 0; i < k; ++i) {

@@ -11,15 +11,22 @@
 #include <cfloat>
 #include <climits>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace {
 
-constexpr int RS_NT = 256;     // radix sort block size (4 waves)
-constexpr int RS_ITEMS = 20;   // keys per thread per tile
-constexpr int RS_TILE = RS_NT * RS_ITEMS;
+constexpr int RS_TILE = 5120;  // radix sort: keys per tile
+// Threads per tile.  Many tiles: 256 threads of 20 keys (three tiles per CU).  Few
+// tiles (RS_WIDE_TILES or fewer, one or two per CU): 1,024 threads of 5, so that a
+// tile's ranking, a chain of LDS round trips per key slot, is a quarter as
+// long: 12.8 -> 10.4 us a pass at 2^16 keys, 20.5 -> 17.9 at 2^20.
+constexpr int RS_NT = 256, RS_NT_WIDE = 1024, RS_WIDE_TILES = 256;
 constexpr int RS_BINS = 256;   // 8-bit digits: passes at bits 0, 8, 16, 24 (30-bit keys)
-constexpr int KH_GRID = 1024;  // most workgroups of the key kernel (each adds its digit totals once)
+// Key kernel: most workgroups (each adds its digit totals once), and points per
+// workgroup and step.  Few points are spread thinner, since a workgroup's
+// steps are a chain of memory round trips: 16.9 -> 8 us at 2^16 points, which were 13 steps of 5,120 before.
+constexpr int KH_GRID = 1024, KH_TILE_MIN = 1024;
 constexpr int SCAN_NT = 1024;  // threads of the census workgroup
 
 __constant__ double c_binom[64 * 64];  // C(n, k) rounded to double, n, k < 64
@@ -224,13 +231,15 @@ TC_DEV unsigned long long wave_digit_peers(uint32_t d, bool ok)
 // One tile of a radix pass: the tile's keys are ranked stably in LDS and
 // written out as contiguous digit runs.  start(tot, s_w) is called by every
 // thread of the block after the ranking (it may use the block scratch s_w for
-// collective scans); for digit threadIdx.x, of which the tile holds tot keys,
-// it returns the global position of the tile's first key of that digit.
-template <class Start>
+// collective scans); for digit threadIdx.x (below RS_BINS), of which the tile
+// holds tot keys, it returns the global position of the tile's first key of that
+// digit.
+template <int NT, class Start>
 TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, uint32_t *vout, int n, int shift,
                     int tile, Start &&start)
 {
-    constexpr int NW = RS_NT / 64, WITEMS = 64 * RS_ITEMS;  // waves per tile, keys per wave
+    constexpr int IT = RS_TILE / NT, NW = NT / 64, WITEMS = 64 * IT;  // keys per thread, waves per tile, keys per wave
+    static_assert(NT * IT == RS_TILE && NT >= RS_BINS, "whole tiles, a thread per digit");
     __shared__ uint32_t s_k[RS_TILE];
     __shared__ uint32_t s_v[RS_TILE];
     __shared__ uint32_t s_tileoff[RS_BINS];
@@ -252,9 +261,9 @@ TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, ui
     // lives in s_wrun[wid] (all lanes read it before the leader updates it).
     // Bounds are tested on the offset within the tile, so base + offset is
     // only formed below n (no int overflow for n near INT_MAX).
-    uint32_t k[RS_ITEMS], v[RS_ITEMS], dr[RS_ITEMS];
+    uint32_t k[IT], v[IT], dr[IT];
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; ++j) {
+    for (int j = 0; j < IT; ++j) {
         const int o = wid * WITEMS + j * 64 + lane;
         const bool ok = o < cnt;
         const int i = base + (ok ? o : 0);
@@ -262,7 +271,7 @@ TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, ui
         v[j] = ok ? (vin ? vin[i] : (uint32_t)i) : 0u;
     }
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; ++j) {
+    for (int j = 0; j < IT; ++j) {
         const bool ok = wid * WITEMS + j * 64 + lane < cnt;
         const uint32_t d = (k[j] >> shift) & (RS_BINS - 1);
         const unsigned long long peers = wave_digit_peers(d, ok);
@@ -282,22 +291,24 @@ TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, ui
         uint32_t c[NW], tot = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            c[w] = s_wrun[w][tid];
+            c[w] = tid < RS_BINS ? s_wrun[w][tid] : 0u;
             tot += c[w];
         }
         const uint32_t g = start(tot, s_w);
-        uint32_t off = block_scan_excl<RS_NT>(tot, s_w, nullptr);
-        s_gbase[tid] = g;
-        s_tileoff[tid] = off;
+        uint32_t off = block_scan_excl<NT>(tot, s_w, nullptr);
+        if (tid < RS_BINS) {
+            s_gbase[tid] = g;
+            s_tileoff[tid] = off;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            s_wrun[w][tid] = off;
-            off += c[w];
+            for (int w = 0; w < NW; ++w) {
+                s_wrun[w][tid] = off;
+                off += c[w];
+            }
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; ++j) {
+    for (int j = 0; j < IT; ++j) {
         if (wid * WITEMS + j * 64 + lane < cnt) {
             const uint32_t pos = s_wrun[wid][dr[j] & 255u] + (dr[j] >> 8);
             s_k[pos] = k[j];
@@ -306,7 +317,7 @@ TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, ui
     }
     __syncthreads();
 
-    for (int p = tid; p < cnt; p += RS_NT) {
+    for (int p = tid; p < cnt; p += NT) {
         const uint32_t kk = s_k[p];
         const uint32_t d = (kk >> shift) & (RS_BINS - 1);
         const uint32_t dst = s_gbase[d] + (uint32_t)p - s_tileoff[d];
@@ -340,7 +351,8 @@ static size_t lb_words(int ntiles) { return (size_t)LB_HIST + LB_TICKETS + (size
 // 0..t-1), exactly as with a scan of the tile histograms.  A count that stays
 // unpublished for RS_SPIN_MAX polls sets bit 1 of *err (reported by the host
 // as a failed sort) and ends the walk.
-__global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(const uint32_t *kin, const uint32_t *vin, uint32_t *kout,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_rs_pass_lb(const uint32_t *kin, const uint32_t *vin, uint32_t *kout,
                                                        uint32_t *vout, int n, int shift, const uint32_t *hist,
                                                        unsigned long long *flags, uint32_t *ticket, uint32_t *err)
 {
@@ -349,13 +361,15 @@ __global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(const uint32_t *kin, const
         s_tile = (int)atomicAdd(ticket, 1u);
     __syncthreads();
     const int tile = s_tile;
-    rs_tile(kin, vin, kout, vout, n, shift, tile, [&](uint32_t tot, uint32_t *s_w) {
+    rs_tile<NT>(kin, vin, kout, vout, n, shift, tile, [&](uint32_t tot, uint32_t *s_w) {
         const int d = threadIdx.x;
-        unsigned long long *fd = flags + d;  // fd[t * RS_BINS]: digit d of tile t
-        __hip_atomic_store(&fd[(size_t)tile * RS_BINS], (tile ? LB_AGG : LB_INC) | tot, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        const bool digit = NT == RS_BINS || d < RS_BINS;
+        unsigned long long *fd = flags + (digit ? d : 0);  // fd[t * RS_BINS]: digit d of tile t
+        if (digit)
+            __hip_atomic_store(&fd[(size_t)tile * RS_BINS], (tile ? LB_AGG : LB_INC) | tot, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
         uint32_t pre = 0;
-        bool done = tile == 0;
+        bool done = tile == 0 || !digit;
         int t = tile;  // tiles t .. tile-1 are summed
         while (!done) {
             // the counts of tiles t-1, t-2, ..., RS_LB_BATCH loads in flight at once
@@ -384,10 +398,10 @@ __global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(const uint32_t *kin, const
             }
             t -= nt;
         }
-        if (tile)
+        if (tile && digit)
             __hip_atomic_store(&fd[(size_t)tile * RS_BINS], LB_INC | (pre + tot), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-        return block_scan_excl<RS_NT>(hist[d], s_w, nullptr) + pre;
+        return block_scan_excl<NT>(digit ? hist[d] : 0u, s_w, nullptr) + pre;
     });
 }
 
@@ -396,7 +410,8 @@ __global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(const uint32_t *kin, const
 // {x, y, v, 0} in input order, so the gather after the sort reads one 32-byte
 // record per source; targets (HILBERT) by hilbert15.  Tiles of RS_TILE points
 // are taken in turn by at most KH_GRID workgroups, and each workgroup adds the
-// digit totals of all four passes into hist4 (zeroed before) once.  Each
+// digit totals of all four passes into hist4 (zeroed before) once.  step points (a
+// multiple of 256) per workgroup and turn.  Each
 // workgroup finishes the bounding box from k_bbox_partial's np partials and
 // per-workgroup flags itself (workgroup 0 writes it and the non-finite flag to
 // box_out and bad_out).
@@ -404,7 +419,7 @@ template <bool HILBERT>
 __global__ __launch_bounds__(256) void k_keys_hist(const double *x, const double *y, const double *v, int n,
                                                     const double4 *part, const uint32_t *pbad, int np,
                                                     double *box_out, uint32_t *bad_out, uint32_t *keys,
-                                                    double4 *packed, uint32_t *hist4)
+                                                    double4 *packed, uint32_t *hist4, int step)
 {
     __shared__ uint32_t h[4 * RS_BINS];
     __shared__ double s_box[4];
@@ -425,10 +440,10 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double *x, const double
         }
     }
     const double xmin = s_box[0], ymin = s_box[1], scale = s_box[3];
-    for (long long base = (long long)blockIdx.x * RS_TILE; base < n; base += (long long)gridDim.x * RS_TILE) {
+    for (long long base = (long long)blockIdx.x * step; base < n; base += (long long)gridDim.x * step) {
 #pragma unroll 4
-        for (int j = 0; j < RS_ITEMS; ++j) {
-            const long long i = base + j * 256 + threadIdx.x;
+        for (int j = 0; j < step; j += 256) {
+            const long long i = base + j + threadIdx.x;
             if (i < n) {
                 const double xi = x[i], yi = y[i];
                 const uint32_t qx = quantise(xi, xmin, scale), qy = quantise(yi, ymin, scale);
@@ -454,21 +469,26 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double *x, const double
 // bbox_finish semantics), keys (Morton or Hilbert as k_keys_hist), the same
 // stable 4-pass LSD radix sort as above with the keys in registers and each
 // pass's scatter in LDS, and for sources the gather of the sorted records.
-// One launch instead of seven, which is what a small solve is made of.
-constexpr int SS_NT = 1024, SS_ITEMS = 16, SS_N = SS_NT * SS_ITEMS;
+// One launch instead of seven, which is what a small solve is made of.  IT keys
+// per thread, the least power of two that holds the points: the ranking (8
+// ballots per key slot and pass) is what the kernel spends its time on, and
+// with 16 slots for every n it took 48 us at 1,000 points and 79 us at 10,000,
+// with the points on one wave instead of 16; 15 us now at 1,000 points, and back
+// to back on warm caches 43 -> 13.5 us at 1,000, 44 -> 22 at 4,000, 47 -> 33 at 8,000.
+constexpr int SS_NT = 1024, SS_MAX_IT = 16, SS_N = SS_NT * SS_MAX_IT;
 static_assert(SS_N == TC_SORT_SMALL_MAX, "one-workgroup sort size");
 
 // The one-workgroup sort of one point set (the body of k_sort_small and of
 // k_sort_small_batch's workgroups).
-template <bool HILBERT>
+template <bool HILBERT, int IT>
 TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ v,
                        int n, double *__restrict__ box_out, uint32_t *__restrict__ bad_out,
                        uint32_t *__restrict__ keys_out, uint32_t *__restrict__ perm_out,
                        double4 *__restrict__ src_out)
 {
-    constexpr int NW = SS_NT / 64, WITEMS = 64 * SS_ITEMS;
-    __shared__ uint32_t s_k[SS_N];
-    __shared__ uint32_t s_v[SS_N];
+    constexpr int NW = SS_NT / 64, WITEMS = 64 * IT;
+    __shared__ uint32_t s_k[SS_NT * IT];
+    __shared__ uint32_t s_v[SS_NT * IT];
     __shared__ uint32_t s_wrun[NW][RS_BINS];
     __shared__ uint32_t s_w[NW + 1];
     __shared__ double4 s_red[NW];
@@ -478,9 +498,9 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
 
     // this thread's points, item j of lane l of wave w being position
     // w * WITEMS + 64 j + l (all loads in flight at once)
-    double xr[SS_ITEMS], yr[SS_ITEMS];
+    double xr[IT], yr[IT];
 #pragma unroll
-    for (int j = 0; j < SS_ITEMS; ++j) {
+    for (int j = 0; j < IT; ++j) {
         const int i = wid * WITEMS + j * 64 + lane;
         xr[j] = i < n ? x[i] : 0.0;
         yr[j] = i < n ? y[i] : 0.0;
@@ -489,7 +509,7 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
     double xmi = 1e13, ymi = 1e13, xma = 0, yma = 0;
     bool nonfinite = false;
 #pragma unroll
-    for (int j = 0; j < SS_ITEMS; ++j) {
+    for (int j = 0; j < IT; ++j) {
         const int i = wid * WITEMS + j * 64 + lane;
         if (i < n) {
             const double a = xr[j], b = yr[j];
@@ -540,9 +560,9 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
     __syncthreads();
 
     const double xmin = s_box[0], ymin = s_box[1], scale = s_box[3];
-    uint32_t k[SS_ITEMS], vi[SS_ITEMS], dr[SS_ITEMS];
+    uint32_t k[IT], vi[IT], dr[IT];
 #pragma unroll
-    for (int j = 0; j < SS_ITEMS; ++j) {
+    for (int j = 0; j < IT; ++j) {
         const int i = wid * WITEMS + j * 64 + lane;
         const uint32_t qx = quantise(xr[j], xmin, scale), qy = quantise(yr[j], ymin, scale);
         k[j] = i < n ? (HILBERT ? hilbert15(qx, qy) : (tc_spread15(qx) | (tc_spread15(qy) << 1))) : 0u;
@@ -556,7 +576,7 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
         tc_wave_sync();
         // wave-local stable ranks, as in rs_tile
 #pragma unroll
-        for (int j = 0; j < SS_ITEMS; ++j) {
+        for (int j = 0; j < IT; ++j) {
             const bool ok = wid * WITEMS + j * 64 + lane < n;
             const uint32_t d = (k[j] >> shift) & (RS_BINS - 1);
             const unsigned long long peers = wave_digit_peers(d, ok);
@@ -589,7 +609,7 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < SS_ITEMS; ++j) {
+        for (int j = 0; j < IT; ++j) {
             if (wid * WITEMS + j * 64 + lane < n) {
                 const uint32_t pos = s_wrun[wid][dr[j] & 255u] + (dr[j] >> 8);
                 s_k[pos] = k[j];
@@ -600,7 +620,7 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
         if (shift == 24)
             break;
 #pragma unroll
-        for (int j = 0; j < SS_ITEMS; ++j) {
+        for (int j = 0; j < IT; ++j) {
             const int p = wid * WITEMS + j * 64 + lane;
             if (p < n) {
                 k[j] = s_k[p];
@@ -619,21 +639,36 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
     }
 }
 
-template <bool HILBERT>
+template <bool HILBERT, int IT>
 __global__ __launch_bounds__(SS_NT) void k_sort_small(const double *__restrict__ x, const double *__restrict__ y,
                                                       const double *__restrict__ v, int n, double *__restrict__ box_out,
                                                       uint32_t *__restrict__ bad_out, uint32_t *__restrict__ keys_out,
                                                       uint32_t *__restrict__ perm_out, double4 *__restrict__ src_out)
 {
-    sort_small<HILBERT>(x, y, v, n, box_out, bad_out, keys_out, perm_out, src_out);
+    sort_small<HILBERT, IT>(x, y, v, n, box_out, bad_out, keys_out, perm_out, src_out);
 }
 
 // Target orders of several requests at once: workgroup b sorts desc[b]'s
-// targets exactly as k_sort_small<true> does alone.
-__global__ __launch_bounds__(SS_NT) void k_sort_small_batch(const TcSortDesc *__restrict__ desc)
+// targets as k_sort_small<true> does alone (the order does not depend on IT).
+template <int IT> __global__ __launch_bounds__(SS_NT) void k_sort_small_batch(const TcSortDesc *__restrict__ desc)
 {
     const TcSortDesc &d = desc[blockIdx.x];
-    sort_small<true>(d.x, d.y, nullptr, d.n, d.box, d.bad, d.keys, d.perm, nullptr);
+    sort_small<true, IT>(d.x, d.y, nullptr, d.n, d.box, d.bad, d.keys, d.perm, nullptr);
+}
+
+// f(std::integral_constant<int, IT>) with the least IT whose SS_NT IT slots hold n points.
+template <class F> void small_items(int n, F &&f)
+{
+    if (n <= SS_NT)
+        f(std::integral_constant<int, 1>());
+    else if (n <= 2 * SS_NT)
+        f(std::integral_constant<int, 2>());
+    else if (n <= 4 * SS_NT)
+        f(std::integral_constant<int, 4>());
+    else if (n <= 8 * SS_NT)
+        f(std::integral_constant<int, 8>());
+    else
+        f(std::integral_constant<int, SS_MAX_IT>());
 }
 
 __global__ __launch_bounds__(256) void k_gather_src(const double4 *packed, const uint32_t *perm, int n,
@@ -1486,10 +1521,13 @@ void tc_sort_points(const double *x, const double *y, const double *v, int n, do
     if (n <= SS_N) {
         ws.bbox_part.reserve(sizeof(double4) + 256);
         uint32_t *bad = const_cast<uint32_t *>(tc_bbox_bad_flag(ws, n));
-        if (hilbert)
-            k_sort_small<true><<<1, SS_NT, 0, st>>>(x, y, v, n, box_d, bad, keys_out, perm_out, src_out);
-        else
-            k_sort_small<false><<<1, SS_NT, 0, st>>>(x, y, v, n, box_d, bad, keys_out, perm_out, src_out);
+        small_items(n, [&](auto it) {
+            constexpr int IT = decltype(it)::value;
+            if (hilbert)
+                k_sort_small<true, IT><<<1, SS_NT, 0, st>>>(x, y, v, n, box_d, bad, keys_out, perm_out, src_out);
+            else
+                k_sort_small<false, IT><<<1, SS_NT, 0, st>>>(x, y, v, n, box_d, bad, keys_out, perm_out, src_out);
+        });
         TC_HIP(hipGetLastError());
         if (ev) {
             // one kernel does keys and sort: both boundaries fall after it
@@ -1541,20 +1579,25 @@ void tc_morton_sort(const double *x, const double *y, const double *v, int n, co
     unsigned long long *flags = reinterpret_cast<unsigned long long *>(tickets + LB_TICKETS);
     const LbBox b = lb_box(ws, n);
     uint32_t *err = b.bad;
-    const int grid = std::min(ntiles, KH_GRID);
+    // at most RS_TILE points a step, at least KH_TILE_MIN, about one step per CU
+    const int step = std::min(RS_TILE, std::max(KH_TILE_MIN, tiles_of(tiles_of(n, 256), 256) * 256));
+    const int grid = std::min(tiles_of(n, step), KH_GRID);
     if (hilbert)
         k_keys_hist<true><<<grid, 256, 0, st>>>(x, y, nullptr, n, b.part, b.pbad, b.np, const_cast<double *>(box_d),
-                                                b.bad, keys_out, nullptr, hist4);
+                                                b.bad, keys_out, nullptr, hist4, step);
     else
         k_keys_hist<false><<<grid, 256, 0, st>>>(x, y, v, n, b.part, b.pbad, b.np, const_cast<double *>(box_d),
-                                                 b.bad, keys_out, packed, hist4);
+                                                 b.bad, keys_out, packed, hist4, step);
     TC_HIP(hipGetLastError());
     if (ev)
         TC_HIP(hipEventRecord(ev[0], st));
     for (int pass = 0; pass < 4; ++pass) {
-        k_rs_pass_lb<<<ntiles, RS_NT, 0, st>>>(kin[pass], vin[pass], kout[pass], vout[pass], n, 8 * pass,
-                                                hist4 + RS_BINS * pass, flags + (size_t)RS_BINS * ntiles * pass,
-                                                tickets + pass, err);
+        const bool wide = ntiles <= RS_WIDE_TILES;
+        const auto pass_kernel = wide ? k_rs_pass_lb<RS_NT_WIDE> : k_rs_pass_lb<RS_NT>;
+        pass_kernel<<<ntiles, wide ? RS_NT_WIDE : RS_NT, 0, st>>>(kin[pass], vin[pass], kout[pass], vout[pass], n,
+                                                                  8 * pass, hist4 + RS_BINS * pass,
+                                                                  flags + (size_t)RS_BINS * ntiles * pass,
+                                                                  tickets + pass, err);
         TC_HIP(hipGetLastError());
     }
 }
@@ -1728,11 +1771,11 @@ TcSortDesc tc_sort_targets_desc(const double *xt, const double *yt, int m, TcScr
     return d;
 }
 
-void tc_sort_targets_batch(const TcSortDesc *desc_dev, int k, hipStream_t st)
+void tc_sort_targets_batch(const TcSortDesc *desc_dev, int k, int mmax, hipStream_t st)
 {
     if (k <= 0)
         return;
-    k_sort_small_batch<<<k, SS_NT, 0, st>>>(desc_dev);
+    small_items(mmax, [&](auto it) { k_sort_small_batch<decltype(it)::value><<<k, SS_NT, 0, st>>>(desc_dev); });
     TC_HIP(hipGetLastError());
 }
 

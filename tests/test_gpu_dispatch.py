@@ -29,3 +29,21 @@ def test_upward_variants(pkg, oracle, wl, n, leaf, order):
     ctx.force(0.5, xs, ys, vs, np.array([0.4]), np.array([0.4]), np.array([1.0 / 512]))
     compare_tree(ctx.tree(), oracle.Tree(xs, ys, vs, leaf, order))
     ctx.close()
+
+
+# one-workgroup sorts with 1, 2, 4, 8, 16 keys per thread, one-launch passes with 1,024 threads a
+# tile (up to 256 tiles of 5,120 keys) and 256 beyond; many equal keys, so stability shows
+@pytest.mark.parametrize("n", [1, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 16384, 16385, 40961,
+                               256 * 5120, 256 * 5120 + 1])
+def test_sort_variants(pkg, oracle, wl, n):
+    st = wl.Stream(n)
+    x, y = np.floor(st.uniform(n) * 50) / 50, np.floor(st.uniform(n) * 40) / 40
+    ctx = pkg.Context()
+    box, keys, perm = ctx.empty(4), ctx.empty(n, np.uint32), ctx.empty(n, np.uint32)
+    ctx.morton_sort_device(ctx.to_device(x), ctx.to_device(y), box, keys, perm)
+    ctx.synchronize()
+    obox = oracle.bbox(x, y)
+    operm, oks = oracle.sort(oracle.keys(x, y, obox))
+    assert np.array_equal(box.numpy()[:3], obox)
+    assert np.array_equal(keys.numpy(), oks) and np.array_equal(perm.numpy(), operm)
+    ctx.close()
