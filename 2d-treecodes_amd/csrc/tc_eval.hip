@@ -1,7 +1,7 @@
 // tc_eval.hip -- theta-criterion traversals on gfx950.
 //
-// Potential (drivers/treecode-potential.cpp:25-86): one wavefront per 64
-// Hilbert-sorted targets.  The wave walks the tree once with a stack of
+// Potential (drivers/treecode-potential.cpp:25-86): one wavefront per 64 (FP64: 8
+// to 64) Hilbert-sorted targets.  The wave walks the tree once with a stack of
 // (node, lane mask) entries; every lane takes exactly the accept/open
 // decisions of its own per-target DFS, so each target sees the reference's
 // interaction list.  Node data and expansion coefficients are wave-uniform
@@ -23,6 +23,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cfloat>
+#include <cmath>
+#include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -47,45 +50,48 @@ TC_DEV double rcp64(double d)
     return fma(r, e, r);
 }
 
-// Natural log of a positive normal double to about 2 ulp (the P2P argument is
-// r^2 + 10 eps >= 2.2e-15).  x = 2^k m with m in [sqrt(1/2), sqrt(2)),
-// log m = 2 atanh(s), s = (m - 1)/(m + 1), |s| <= 0.1716, and
-// 2 atanh(s) = 2s (1 + z/3 + z^2/5 + ... + z^10/21) with z = s^2 <= 0.0295,
-// the Taylor series truncated where the next term is below 2^-57 relative.
-// k ln 2 uses ln 2 split into a 32-bit head (k * head exact) and a tail.
-TC_DEV double log64(double x)
+// The same by one third-order step, r (1 + e + e^2): three FMAs on an
+// estimate good to 2^-22 or better.
+TC_DEV double rcp64_3(double d)
+{
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+
+// Natural log of a positive normal double to 1.7 ulp, by table (Tang's method):
+// x = 2^k z with z in [0.6875, 1.375), c the table's value near 1/z (256
+// intervals of z; exactly 1 for the two next to z = 1, so that small logs keep
+// their relative accuracy), r = z c - 1, |r| <= 2^-8, and log x = k ln 2 - log c +
+// log(1 + r) with the series to r^7 (the next term is below 2^-59 of r).
+// tab[i] = (c, -log c) in LDS; 13 FP64 operations, 6 integer ones and one LDS
+// read.  A series in (z - 1)/(z + 1) takes 30 FP64 operations (a reciprocal and
+// 10 terms); rms error over 8e6 arguments 0.31 ulp against 0.36.  Not for
+// infinities and NaNs (the callers' targets are checked once, at the end).
+constexpr int LOG_TAB = 256;
+constexpr uint32_t LOG_OFF = 0x3FE60000u;  // high word of 0.6875
+__constant__ double2 c_logtab[LOG_TAB];
+TC_DEV double log64(double x, const double2 *tab)
 {
 #pragma clang fp contract(fast)
-    double m = __builtin_amdgcn_frexp_mant(x);  // [0.5, 1)
-    int k = __builtin_amdgcn_frexp_exp(x);
-    if (m < 0.70710678118654757) {
-        m = m + m;
-        k -= 1;
-    }
-    const double f = m - 1.0;  // exact (Sterbenz)
-    const double d = m + 1.0;
-    double r = __builtin_amdgcn_rcp(d);
-    double e = fma(-d, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-d, r, 1.0);
-    r = fma(r, e, r);
-    double q = f * r;
-    q = fma(r, fma(-q, d, f), q);  // s = f / d to ~0.5 ulp
-    const double z = q * q;
-    double P = 1.0 / 21.0;
-    P = fma(P, z, 1.0 / 19.0);
-    P = fma(P, z, 1.0 / 17.0);
-    P = fma(P, z, 1.0 / 15.0);
-    P = fma(P, z, 1.0 / 13.0);
-    P = fma(P, z, 1.0 / 11.0);
-    P = fma(P, z, 1.0 / 9.0);
-    P = fma(P, z, 1.0 / 7.0);
-    P = fma(P, z, 1.0 / 5.0);
-    P = fma(P, z, 1.0 / 3.0);
-    const double q2 = q + q;
-    const double logm = fma(q2 * z, P, q2);
-    const double kd = (double)k;
-    return fma(kd, 0.6931471803691238, fma(kd, 1.9082149292705877e-10, logm));
+    const uint32_t hi = (uint32_t)__double2hiint(x), t = hi - LOG_OFF;
+    const double kd = (double)((int32_t)t >> 20);
+    const double2 c = tab[(t >> 12) & (LOG_TAB - 1)];
+    const double z = __hiloint2double((int)(hi - (t & 0xFFF00000u)), __double2loint(x));
+    const double r = fma(z, c.x, -1.0);
+    double q = fma(r, 1.0 / 7.0, -1.0 / 6.0);
+    q = fma(q, r, 1.0 / 5.0);
+    q = fma(q, r, -1.0 / 4.0);
+    q = fma(q, r, 1.0 / 3.0);
+    q = fma(q, r, -0.5);
+    // k ln 2 with ln 2 split into a 32-bit head and a tail
+    const double lo = fma(kd, 1.9082149292705877e-10, fma(r * r, q, r));
+    return fma(kd, 0.6931471803691238, c.y) + lo;
+}
+TC_DEV void log64_table(double2 *tab)
+{
+    for (int i = threadIdx.x; i < LOG_TAB; i += blockDim.x)
+        tab[i] = c_logtab[i];
 }
 
 // ------------------------------------------------------------------ potential kernels
@@ -93,10 +99,10 @@ TC_DEV double log64(double x)
 // Q log|z| + Re sum_{j=1..p} a_j u^j with u = 1/z, evaluated by Horner's rule
 // (4 FMAs per coefficient).
 template <int P>
-TC_DEV double e2p_pot64(double rz, double iz, double mass, const double *__restrict__ ex)
+TC_DEV double e2p_pot64(double rz, double iz, double mass, const double *__restrict__ ex, const double2 *logtab)
 {
     const double r2 = fma(rz, rz, iz * iz);
-    const double inv = 1.0 / r2;
+    const double inv = rcp64_3(r2);
     const double ur = rz * inv, ui = -iz * inv;
     double ar = ex[P - 1], ai = ex[2 * P - 1];
 #pragma unroll
@@ -106,7 +112,7 @@ TC_DEV double e2p_pot64(double rz, double iz, double mass, const double *__restr
         ar = tr;
         ai = ti;
     }
-    return fma(mass * 0.5, log64(r2), fma(ur, ar, -ui * ai));
+    return fma(mass * 0.5, log64(r2, logtab), fma(ur, ar, -ui * ai));
 }
 
 // FP32 E2P on scaled coefficients b_j = a_j / s^j: Re sum b_j w^j, w = s/z
@@ -285,48 +291,44 @@ struct alignas(16) TcStackEntry {
     int node, pad;
 };
 
-// LDS of one workgroup (four waves) of the potential traversal.
-template <int P, bool F32> struct TcPotShared {
+// LDS of one workgroup (four waves) of the FP32 potential traversal.
+template <int P> struct TcPotShared32 {
     TcStackEntry stk[4][TC_STACK];
     double4 src[4][64];
-    // FP32 wave-level local expansions: beta[l P + k - 1] = (-1)^k C(l + k - 1, l),
+    // wave-level local expansions: beta[l P + k - 1] = (-1)^k C(l + k - 1, l),
     // queued node ids, their z0 = com - centre, and each wave's {centre, radius, 1 / theta'}
-    float beta[F32 ? M2L_G * P : 1];
-    int q[4][F32 ? M2L_Q : 1];
+    float beta[M2L_G * P];
+    int q[4][M2L_Q];
     double4 wc[4];
-    float2 qz[4][F32 ? M2L_Q : 1];
-};
-
-template <int P, bool F32> TC_DEV void potential_shared_init(TcPotShared<P, F32> &sh)
-{
-    if constexpr (F32) {
+    float2 qz[4][M2L_Q];
+    TC_DEV void init()
+    {
         for (int i = threadIdx.x; i < M2L_G * P; i += 256) {
             const int l = i / P, kk = i - l * P + 1;
             const double c = c_binomT[l * 64 + l + kk - 1];
-            sh.beta[i] = (float)((kk & 1) ? -c : c);
+            beta[i] = (float)((kk & 1) ? -c : c);
         }
         __syncthreads();
     }
-}
+};
 
 // One wave's traversal: targets tperm[k0 .. k0 + 63] of request rq, k0 = 64 x
 // (the wave's index within the request); shared by the one-request kernel
 // and the batched one, so a request's results do not depend on which runs it.
-template <int P, bool F32, bool CNT>
-TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ nodes,
-                           const double *__restrict__ exps, const float2 *__restrict__ exps32,
-                           const double4 *__restrict__ src, const float4 *__restrict__ src32,
-                           const double *__restrict__ xt, const double *__restrict__ yt,
-                           const uint32_t *__restrict__ tperm, double *__restrict__ out, const double th2,
-                           const int m, int k0, unsigned long long *counters)
+template <int P, bool CNT>
+TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ nodes,
+                             const float2 *__restrict__ exps32, const float4 *__restrict__ src32,
+                             const double *__restrict__ xt, const double *__restrict__ yt,
+                             const uint32_t *__restrict__ tperm, double *__restrict__ out, const double th2,
+                             const int m, int k0, unsigned long long *counters)
 {
     TcStackEntry(&s_stk)[4][TC_STACK] = sh.stk;
     double4(&s_src)[4][64] = sh.src;
     const float *s_beta = sh.beta;
-    int(&s_q)[4][F32 ? M2L_Q : 1] = sh.q;
+    int(&s_q)[4][M2L_Q] = sh.q;
     double4 *s_wc = sh.wc;
-    float2(&s_qz)[4][F32 ? M2L_Q : 1] = sh.qz;
-    static_assert(!F32 || 4 * (P + 1) * sizeof(float2) <= sizeof(s_src[0]), "staged coefficients fit a source tile");
+    float2(&s_qz)[4][M2L_Q] = sh.qz;
+    static_assert(4 * (P + 1) * sizeof(float2) <= sizeof(s_src[0]), "staged coefficients fit a source tile");
     const int wid = threadIdx.x >> 6, lane = tc_lane();
     const int k = k0 + lane;
     const bool valid = k < m;
@@ -335,10 +337,10 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
     const unsigned long long live = tc_ballot(valid);
     if (!live)
         return;
-    // FP32: centre (bounding-box middle) and radius of the wave's targets
+    // centre (bounding-box middle) and radius of the wave's targets
     int nq = 0;
     unsigned long long nm2l = 0, ne2pw = 0;
-    if constexpr (F32) {
+    {
         const int first = __builtin_ctzll(live);
         const double fx = __shfl(x, first, 64), fy = __shfl(y, first, 64);
         const double lx = valid ? x : fx, ly = valid ? y : fy;
@@ -396,13 +398,9 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
         const bool acc_ok = __builtin_amdgcn_inverse_ballot_w64(amask);
         if constexpr (CNT)
             tc0 = tc_clock();
-        if (acc_ok) {
-            if (F32)
-                acc_e2p += e2p_pot32<P>((float)dx, (float)dy, exps32 + (size_t)(P + 1) * id);
-            else
-                acc += e2p_pot64<P>(dx, dy, nd.mass, exps + (size_t)2 * P * id);
-        }
-        if (F32 && amask && ++n_e2p == 8) {
+        if (acc_ok)
+            acc_e2p += e2p_pot32<P>((float)dx, (float)dy, exps32 + (size_t)(P + 1) * id);
+        if (amask && ++n_e2p == 8) {
             acc += (double)acc_e2p;
             acc_e2p = 0.f;
             n_e2p = 0;
@@ -428,7 +426,7 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
             // target.  Chosen when k (C 9.5 + 16.5) < n 9.8, the measured
             // nanoseconds per SIMD of the two forms (FP32 op 1.18 ns, log 3.6 ns;
             // C chunks of 64 of the n sources, k active lanes).
-            if (F32 && (long long)nact * (nchunk * 19 + 33) < (long long)nsrc * 20) {
+            if ((long long)nact * (nchunk * 19 + 33) < (long long)nsrc * 20) {
                 if constexpr (CNT)
                     nslots += 64ull * (unsigned long long)nchunk * (unsigned long long)nact;
                 const float txl = (float)(x - nd.xcom), tyl = (float)(y - nd.ycom);
@@ -473,7 +471,7 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
                     }
                 }
                 acc += part * (double)LN2_HALF;
-            } else if (F32) {
+            } else {
                 // Dense: sources staged 64 at a time in LDS.  Lanes l and l^32
                 // split each tile (even / odd sources) and each computes both
                 // targets, its own and its partner's: one broadcast LDS read
@@ -528,39 +526,11 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
                 const double leafsum = own + __shfl_xor(other, 32, 64);
                 if (act)
                     acc += leafsum * (double)LN2_HALF;
-            } else {
-                if constexpr (CNT)
-                    nslots += 64ull * (unsigned long long)nsrc;
-                double leafsum = 0, leafsum2 = 0;
-                for (int b0 = nd.s; b0 < nd.e; b0 += 64) {
-                    const int cnt = min(64, nd.e - b0);
-                    if (lane < cnt)
-                        s_src[wid][lane] = src[b0 + lane];
-                    tc_wave_sync();
-                    if (act) {
-#pragma clang fp contract(fast)
-                        int j = 0;
-                        for (; j + 2 <= cnt; j += 2) {
-                            const double4 q0 = s_src[wid][j], q1 = s_src[wid][j + 1];
-                            const double ax = x - q0.x, ay = y - q0.y;
-                            const double bx = x - q1.x, by = y - q1.y;
-                            leafsum += log64(ax * ax + ay * ay + EPS_REG) * q0.z;
-                            leafsum2 += log64(bx * bx + by * by + EPS_REG) * q1.z;
-                        }
-                        if (j < cnt) {
-                            const double4 q = s_src[wid][j];
-                            const double ax = x - q.x, ay = y - q.y;
-                            leafsum += log64(ax * ax + ay * ay + EPS_REG) * q.z;
-                        }
-                    }
-                    tc_wave_sync();
-                }
-                acc += (leafsum + leafsum2) * 0.5;
             }
             if constexpr (CNT)
                 cp2p += tc_clock() - tc0;
         } else {
-            if constexpr (F32) {
+            {
                 if (omask == live) {
                     // the whole wave opens this node: children that qualify for the
                     // wave's local expansion are queued, the others pushed (order
@@ -616,7 +586,7 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
             sp += 4;
         }
     }
-    if constexpr (F32) {
+    {
         if (nq > 0) {
             // the queued translations, four nodes per pass (the source tile's
             // LDS stages their coefficients)
@@ -685,10 +655,8 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
         atomicAdd(&counters[TC_CNT_E2P], ne2p);
         atomicAdd(&counters[TC_CNT_P2P_SLOTS], nslots);
         atomicAdd(&counters[TC_CNT_E2P_SLOTS], neslots);
-        if (F32) {
-            atomicAdd(&counters[TC_CNT_M2L_WAVE], nm2l);
-            atomicAdd(&counters[TC_CNT_E2P_WAVE], ne2pw);
-        }
+        atomicAdd(&counters[TC_CNT_M2L_WAVE], nm2l);
+        atomicAdd(&counters[TC_CNT_E2P_WAVE], ne2pw);
         atomicAdd(&counters[TC_CNT_CYC_P2P], cp2p);
         atomicAdd(&counters[TC_CNT_CYC_E2P], ce2p);
         atomicAdd(&counters[TC_CNT_CYC_LOCAL], cloc);
@@ -697,8 +665,204 @@ TC_DEV void potential_wave(TcPotShared<P, F32> &sh, const TcNode *__restrict__ n
     }
 }
 
+// ------------------------------------------------------------------ FP64 potential traversal
+// A target's result must not depend on which other targets its wave holds
+// (resident solves of a few of a solve's targets repeat its bits): every lane
+// adds its own terms in the order of its own DFS, and a leaf's direct sum is
+// formed in one fixed way, as 8 partial sums over the sources j = 0..7 (mod 8)
+// of the leaf added pairwise.
+//
+// Direct sums: the k lanes that need the leaf are taken 16 at a time, and the wave
+// forms an 8 x 8 arrangement: lane (row, q) holds the partial sum q of target
+// `row` and of target `row + 8` of the batch, so a leaf costs ceil(k / 16) n / 4
+// pair evaluations a lane for n sources: what few lanes need costs little,
+// where a loop of every lane over all sources costs n whatever k.  Sources pass
+// through LDS 64 at a time (the next 64 in registers meanwhile); one read of a
+// source serves two pairs.  What bounds it: a pair is 18 FP64 operations, 7
+// 32-bit ones and one 16-byte LDS read at a data-dependent address (log64).
+// One lane per target over all sources, with a 30-operation log: 12.7 -> 8.6 ms
+// at 2^22 (order 9 / leaf 64, theta 0.3; build 0.7 ms of it), 1.11 -> 0.60 ms at
+// 2^18 (12 / 512), 0.53 -> 0.28 ms at 2^16 with 32 targets a wave.
+struct TcPotShared64 {
+    TcStackEntry stk[4][TC_STACK];
+    double2 tgt[4][64];    // the wave's targets
+    double2 xy[4][64];     // source tile
+    double v[4][64];
+    double res[4][64];     // leaf sums of the active targets
+    int act[4][64];        // the active lanes
+    double2 logtab[LOG_TAB];
+    TC_DEV void init()
+    {
+        log64_table(logtab);
+        __syncthreads();
+    }
+};
+
+// Sum over the leaf's sources [s, e) at the targets of the lanes in omask
+// (valid in those lanes; log of the squared distance, so twice the potential).
+TC_DEV double p2p_leaf64(TcPotShared64 &sh, const double4 *__restrict__ src, int s, int e, unsigned long long omask)
+{
+    const int wid = threadIdx.x >> 6, lane = tc_lane();
+    double2 *const s_xy = sh.xy[wid], *const s_t = sh.tgt[wid];
+    double *const s_v = sh.v[wid], *const s_res = sh.res[wid];
+    int *const s_act = sh.act[wid];
+    const int k = __popcll(omask), rank = __popcll(omask & tc_lanemask_lt());
+    const bool act = __builtin_amdgcn_inverse_ballot_w64(omask);
+    const int row = lane >> 3, q = lane & 7;
+    if (act)
+        s_act[rank] = lane;
+    for (int b = 0; b < k; b += 16) {
+        double a0 = 0, a1 = 0;
+        const int left = k - b;
+        // lanes past the end repeat the last source with weight zero; a leaf of one
+        // tile is staged once
+        const bool stage = b == 0 || e - s > 64;
+        double4 nx;
+        if (stage)
+            nx = src[min(s + lane, e - 1)];
+        tc_wave_sync();
+        const double2 t0 = s_t[s_act[b + min(row, left - 1)]], t1 = s_t[s_act[b + min(row + 8, left - 1)]];
+        for (int b0 = s; b0 < e; b0 += 64) {
+            const int cnt = min(64, e - b0), n8 = (cnt + 7) >> 3;
+            if (stage) {
+                tc_wave_sync();
+                s_xy[lane] = make_double2(nx.x, nx.y);
+                s_v[lane] = lane < cnt ? nx.z : 0.0;
+                if (b0 + 64 < e)
+                    nx = src[min(b0 + 64 + lane, e - 1)];
+                tc_wave_sync();
+            }
+            if (left > 8) {
+                for (int i = 0; i < n8; ++i) {
+#pragma clang fp contract(fast)
+                    const double2 p = s_xy[8 * i + q];
+                    const double v = s_v[8 * i + q];
+                    const double ax = t0.x - p.x, ay = t0.y - p.y;
+                    const double bx = t1.x - p.x, by = t1.y - p.y;
+                    a0 += log64(ax * ax + (ay * ay + EPS_REG), sh.logtab) * v;
+                    a1 += log64(bx * bx + (by * by + EPS_REG), sh.logtab) * v;
+                }
+            } else {
+                for (int i = 0; i < n8; ++i) {
+#pragma clang fp contract(fast)
+                    const double2 p = s_xy[8 * i + q];
+                    const double ax = t0.x - p.x, ay = t0.y - p.y;
+                    a0 += log64(ax * ax + (ay * ay + EPS_REG), sh.logtab) * s_v[8 * i + q];
+                }
+            }
+        }
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) {
+            a0 += __shfl_xor(a0, off, 64);
+            a1 += __shfl_xor(a1, off, 64);
+        }
+        if (q == 0) {
+            s_res[b + row] = a0;
+            s_res[b + 8 + row] = a1;
+        }
+    }
+    tc_wave_sync();
+    return s_res[act ? rank : 0];
+}
+
+// One wave's traversal (EvaluatePotential::evaluate, treecode-potential.cpp:25-86)
+// of up to tpw targets tperm[k0 .. k0 + tpw - 1]; the result of a target does not
+// depend on tpw.
+template <int P, bool CNT>
+TC_DEV void potential_wave64(TcPotShared64 &sh, const TcNode *__restrict__ nodes, const double *__restrict__ exps,
+                             const double4 *__restrict__ src, const double *__restrict__ xt,
+                             const double *__restrict__ yt, const uint32_t *__restrict__ tperm,
+                             double *__restrict__ out, const double th2, const int m, int k0, int tpw,
+                             unsigned long long *counters)
+{
+    const int wid = threadIdx.x >> 6, lane = tc_lane();
+    TcStackEntry *const stk = sh.stk[wid];
+    const int k = k0 + lane;
+    const bool valid = lane < tpw && k < m;
+    const uint32_t ti = valid ? tperm[k] : 0u;
+    const double x = valid ? xt[ti] : 0.0, y = valid ? yt[ti] : 0.0;
+    const unsigned long long live = tc_ballot(valid);
+    if (!live)
+        return;
+    sh.tgt[wid][lane] = make_double2(x, y);
+    double acc = 0;
+    unsigned long long np2p = 0, ne2p = 0, nslots = 0, neslots = 0;
+    // CNT: wave clock cycles per category (direct sums, per-target multipoles) and in total
+    unsigned long long cyc0 = 0, cp2p = 0, ce2p = 0, tc0 = 0;
+    if constexpr (CNT)
+        cyc0 = tc_clock();
+    if (lane == 0)
+        stk[0] = TcStackEntry{live, 0, 0};
+    int sp = 1;
+    while (sp > 0) {
+        --sp;
+        tc_wave_sync();
+        // one LDS read, made scalar before the record's loads (see potential_wave32)
+        const uint4 top = *reinterpret_cast<const uint4 *>(&stk[sp]);
+        const int id = tc_uniform((int)top.z);
+        const unsigned long long mask =
+            ((unsigned long long)(unsigned)tc_uniform((int)top.y) << 32) | (unsigned)tc_uniform((int)top.x);
+        const TcNode nd = nodes[id];
+        const bool nonempty = nd.s != nd.e;
+        const double dx = x - nd.xcom, dy = y - nd.ycom;
+        const double r2 = dx * dx + dy * dy;
+        const unsigned long long amask = tc_ballot(nd.rr < th2 * r2) & mask & (nonempty ? ~0ull : 0ull);
+        if constexpr (CNT)
+            tc0 = tc_clock();
+        if (__builtin_amdgcn_inverse_ballot_w64(amask))
+            acc += e2p_pot64<P>(dx, dy, nd.mass, exps + (size_t)2 * P * id, sh.logtab);
+        if constexpr (CNT) {
+            ne2p += __popcll(amask);
+            neslots += amask ? 64ull : 0ull;
+            if (amask)
+                ce2p += tc_clock() - tc0;
+        }
+        const unsigned long long omask = nonempty ? mask & ~amask : 0ull;
+        if (!omask)
+            continue;
+        if (nd.child == 0) {
+            if constexpr (CNT) {
+                tc0 = tc_clock();
+                const unsigned long long nact = __popcll(omask), nsrc = nd.e - nd.s;
+                np2p += nact * nsrc;
+                nslots += ((nact + 7) >> 3 << 3) * ((nsrc + 7) >> 3 << 3);
+            }
+            const double leafsum = p2p_leaf64(sh, src, nd.s, nd.e, omask);
+            if (__builtin_amdgcn_inverse_ballot_w64(omask))
+                acc += leafsum * 0.5;
+            if constexpr (CNT)
+                cp2p += tc_clock() - tc0;
+        } else {
+            // children pushed in order 0..3, popped 3..0 (treecode-potential.cpp:76-79)
+            if (lane < 4)
+                stk[sp + lane] = TcStackEntry{omask, nd.child + lane, 0};
+            sp += 4;
+        }
+    }
+    // log64 and the reciprocal are for finite arguments: NaN where a squared distance
+    // may have overflowed (or a coordinate is not finite)
+    {
+        const TcNode root = nodes[0];
+        const double dx = x - root.xcom, dy = y - root.ycom;
+        if (!(dx * dx + dy * dy + root.rr < 1e300))
+            acc = __longlong_as_double(0x7FF8000000000000ll);
+    }
+    if (valid)
+        out[ti] = acc;
+    if (CNT && lane == 0) {
+        atomicAdd(&counters[TC_CNT_P2P], np2p);
+        atomicAdd(&counters[TC_CNT_E2P], ne2p);
+        atomicAdd(&counters[TC_CNT_P2P_SLOTS], nslots);
+        atomicAdd(&counters[TC_CNT_E2P_SLOTS], neslots);
+        atomicAdd(&counters[TC_CNT_CYC_P2P], cp2p);
+        atomicAdd(&counters[TC_CNT_CYC_E2P], ce2p);
+        atomicAdd(&counters[TC_CNT_CYC_TOTAL], tc_clock() - cyc0);
+    }
+}
+
 // (separate kernel arguments rather than a TcPotReq: a by-value struct
 // argument costs this kernel registers and occupancy)
+// tpw: targets per wave (FP64 only; FP32 waves hold 64).
 template <int P, bool F32, bool CNT>
 __global__ __launch_bounds__(256) void k_potential(const TcNode *__restrict__ nodes, const double *__restrict__ exps,
                                                    const float2 *__restrict__ exps32,
@@ -706,12 +870,15 @@ __global__ __launch_bounds__(256) void k_potential(const TcNode *__restrict__ no
                                                    const float4 *__restrict__ src32, const double *__restrict__ xt,
                                                    const double *__restrict__ yt, const uint32_t *__restrict__ tperm,
                                                    int m, double th2, double *__restrict__ out,
-                                                   unsigned long long *counters, int xcd_lc)
+                                                   unsigned long long *counters, int xcd_lc, int tpw)
 {
-    __shared__ TcPotShared<P, F32> sh;
-    potential_shared_init<P, F32>(sh);
-    potential_wave<P, F32, CNT>(sh, nodes, exps, exps32, src, src32, xt, yt, tperm, out, th2, m,
-                                (tc_xcd_chunk_block(xcd_lc) * 4 + (threadIdx.x >> 6)) * 64, counters);
+    __shared__ std::conditional_t<F32, TcPotShared32<P>, TcPotShared64> sh;
+    sh.init();
+    const int w = tc_xcd_chunk_block(xcd_lc) * 4 + (threadIdx.x >> 6);
+    if constexpr (F32)
+        potential_wave32<P, CNT>(sh, nodes, exps32, src32, xt, yt, tperm, out, th2, m, w * 64, counters);
+    else
+        potential_wave64<P, CNT>(sh, nodes, exps, src, xt, yt, tperm, out, th2, m, w * tpw, tpw, counters);
 }
 
 // Cross-request traversal: a persistent grid drains the target waves of all
@@ -729,8 +896,8 @@ template <int P, bool F32, bool CNT>
 __global__ __launch_bounds__(256) void k_potential_batch(const TcPotReq *__restrict__ reqs, int *meta,
                                                          unsigned long long *counters)
 {
-    __shared__ TcPotShared<P, F32> sh;
-    potential_shared_init<P, F32>(sh);
+    __shared__ std::conditional_t<F32, TcPotShared32<P>, TcPotShared64> sh;
+    sh.init();
     const int nreq = meta[0], nwaves = meta[1];
     for (;;) {
         int g = 0;
@@ -756,13 +923,20 @@ __global__ __launch_bounds__(256) void k_potential_batch(const TcPotReq *__restr
             const gptr q = (gptr)(tc_uniform64((unsigned long long)p));
             return (const void *)q;
         };
-        potential_wave<P, F32, CNT>(
-            sh, static_cast<const TcNode *>(up(rq.nodes)), static_cast<const double *>(up(rq.exps)),
-            static_cast<const float2 *>(up(rq.exps32)), static_cast<const double4 *>(up(rq.src)),
-            static_cast<const float4 *>(up(rq.src32)), static_cast<const double *>(up(rq.xt)),
-            static_cast<const double *>(up(rq.yt)), static_cast<const uint32_t *>(up(rq.tperm)),
-            const_cast<double *>(static_cast<const double *>(up(rq.out))), tc_uniform(rq.th2), tc_uniform(rq.m),
-            (g - tc_uniform(rq.wave0)) * 64, counters);
+        const TcNode *nodes = static_cast<const TcNode *>(up(rq.nodes));
+        const double *xt = static_cast<const double *>(up(rq.xt)), *yt = static_cast<const double *>(up(rq.yt));
+        const uint32_t *tperm = static_cast<const uint32_t *>(up(rq.tperm));
+        double *out = const_cast<double *>(static_cast<const double *>(up(rq.out)));
+        const double th2 = tc_uniform(rq.th2);
+        const int m = tc_uniform(rq.m), k0 = (g - tc_uniform(rq.wave0)) * 64;
+        if constexpr (F32)
+            potential_wave32<P, CNT>(sh, nodes, static_cast<const float2 *>(up(rq.exps32)),
+                                     static_cast<const float4 *>(up(rq.src32)), xt, yt, tperm, out, th2, m, k0,
+                                     counters);
+        else
+            potential_wave64<P, CNT>(sh, nodes, static_cast<const double *>(up(rq.exps)),
+                                     static_cast<const double4 *>(up(rq.src)), xt, yt, tperm, out, th2, m, k0, 64,
+                                     counters);
     }
 }
 
@@ -1790,16 +1964,30 @@ TcPotReq potential_req(const TcTree &t, double th2, const double *xt, const doub
     return rq;
 }
 
+// Targets per wave of the FP64 potential: fewer where m targets would leave
+// SIMDs without a wave.  The direct sums' cost per target does not depend on it
+// (batches of 8 or 16 targets), the walk's and the multipoles' does, so full waves
+// from 2^17 targets on.  Whole solves (order 12 / leaf 512; 9 / 64, theta 0.3) with
+// 64 / 32 / 16 / 8 targets per wave: 4,000 targets 305 / 213 / 172 / 158 us and
+// 452 / 341 / 275 / 265, 32,000: 724 / 470 / 362 / 354 and 551 / 499 / 495 / 546,
+// 64,000: 600 / 474 / 416 / 477 and 603 / 570 / 615 / 817, 256,000: 849 / 844 / 934 /
+// 1271 and 870 / 1087 / 1524 / 2256.
+int pot_targets_per_wave(int m)
+{
+    return m <= 8192 ? 8 : (m <= 49152 ? 16 : (m <= 131072 ? 32 : 64));
+}
+
 template <int P>
 void launch_potential(const TcTree &t, double th2, const double *xt, const double *yt, const uint32_t *tperm,
                       int m, double *out, int precision, unsigned long long *counters, hipStream_t st,
                       int xcd_lc = TC_XCD_CHUNK_LOG2)
 {
-    const int grid = tiles_of(m, 256);
+    const int tpw = precision == 1 ? 64 : pot_targets_per_wave(m);
+    const int grid = tiles_of(m, 4 * tpw);
     const TcPotReq q = potential_req(t, th2, xt, yt, tperm, m, out, precision, 0);
     auto go = [&](auto kern) {
         kern<<<grid, 256, 0, st>>>(q.nodes, q.exps, q.exps32, q.src, q.src32, q.xt, q.yt, q.tperm, q.m, q.th2, q.out,
-                                   counters, xcd_lc);
+                                   counters, xcd_lc, tpw);
     };
     if (precision == 1 && counters)
         go(k_potential<P, true, true>);
@@ -1943,6 +2131,21 @@ void tc_upload_binomials_eval(hipStream_t st)
             tab[k * 64 + n] = (double)r;
         }
     TC_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_binomT), tab.data(), sizeof(double) * tab.size(), 0,
+                                  hipMemcpyHostToDevice, st));
+    // log64's table: interval i of z starts at the double with high word LOG_OFF + i 2^12
+    std::vector<double2> lt(LOG_TAB);
+    auto from_high = [](uint32_t hi) {
+        const uint64_t b = (uint64_t)hi << 32;
+        double d;
+        std::memcpy(&d, &b, sizeof d);
+        return d;
+    };
+    for (uint32_t i = 0; i < LOG_TAB; ++i) {
+        const double a = from_high(LOG_OFF + (i << 12)), b = from_high(LOG_OFF + ((i + 1) << 12));
+        const double c = a == 1.0 || b == 1.0 ? 1.0 : 1.0 / (0.5 * (a + b));
+        lt[i] = make_double2(c, c == 1.0 ? 0.0 : (double)-std::log((long double)c));
+    }
+    TC_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_logtab), lt.data(), sizeof(double2) * lt.size(), 0,
                                   hipMemcpyHostToDevice, st));
     TC_HIP(hipStreamSynchronize(st));
 }

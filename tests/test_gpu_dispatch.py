@@ -47,3 +47,44 @@ def test_sort_variants(pkg, oracle, wl, n):
     assert np.array_equal(box.numpy()[:3], obox)
     assert np.array_equal(keys.numpy(), oks) and np.array_equal(perm.numpy(), operm)
     ctx.close()
+
+
+# FP64 potential: 8, 16, 32, 64 targets per wave, whatever the wave the same bits; leaves of one
+# and of several source tiles, full and ragged; 1 to 64 active lanes a leaf
+@pytest.mark.parametrize("m", [1, 7, 8192, 8193, 49152, 49153, 131072, 131073])
+@pytest.mark.parametrize("order,leaf", [(9, 33), (12, 500)])
+def test_fp64_targets_per_wave(pkg, oracle, wl, m, order, leaf):
+    xs, ys, vs, *_ = wl.mixed_plummer_potential(30011, seed=m % 89)
+    st = wl.Stream(m)
+    xt, yt = st.uniform(m, -0.2, 1.2), st.uniform(m, -0.2, 1.2)
+    ctx = pkg.Context(pot_order=order, pot_leaf=leaf, counters=True)
+    out = ctx.potential(0.5, xs, ys, vs, xt, yt)
+    cnt = ctx.stats()["counters"]
+    idx = np.sort(np.random.default_rng(m).choice(m, min(m, 2000), replace=False))
+    ot = oracle.Tree(xs, ys, vs, leaf, order)
+    ref, rc = ot.potential(0.5, xt[idx], yt[idx])
+    assert rel_l2(out[idx], ref) <= 1e-12
+    if len(idx) == m:
+        assert (cnt["p2p"], cnt["e2p"]) == (rc[0], rc[1])
+    for part in (idx, idx[:9], idx[-1:]):
+        assert np.array_equal(ctx.potential_resident(0.5, xt[part], yt[part]), out[part])
+    ctx.close()
+
+
+def test_fp64_potential_nonfinite_and_huge(pkg):
+    # log64 takes finite positive arguments; what overflows a squared distance is NaN, as log is there
+    ctx = pkg.Context()
+    xs, ys, vs = np.array([0.0, 1.0]), np.array([0.0, 1.0]), np.array([1.0, -2.0])
+    x = np.array([0.5, 1e200, np.inf, np.nan, -1e160, 0.0])
+    y = np.array([0.5, 0.0, 0.0, 0.0, 1e160, 0.0])
+    d = [ctx.to_device(a) for a in (xs, ys, vs, x, y)]
+    out = ctx.empty(len(x))
+    ctx.potential(0.0, *d, out=out, device=True)
+    ctx.synchronize()
+    o = out.numpy()
+    assert np.isnan(o[[1, 2, 3, 4]]).all() and np.isfinite(o[[0, 5]]).all()
+    eps = 10 * np.finfo(float).eps
+    want = [sum(v * 0.5 * np.log((a - s) ** 2 + (b - t) ** 2 + eps) for s, t, v in zip(xs, ys, vs))
+            for a, b in zip(x[[0, 5]], y[[0, 5]])]
+    assert np.allclose(o[[0, 5]], want, rtol=1e-14, atol=1e-15)
+    ctx.close()
