@@ -690,6 +690,9 @@ int run_force(tc_context *ctx, double theta, const double *xs, const double *ys,
         if (rebuild)
             build(c, dxs, dys, dvs, n, TC_KIND_FORCE, ext);
         record(c, 1);
+        // (a server's shared tree was built for the request's precision)
+        if (c->precision == 0 && !ext.tree)
+            tc_tree_deriv(c->tree, c->stream);
         const TcTree &tree = ext.tree ? *ext.tree : c->tree;
         // Host outputs of at least FORCE_SPLIT_BLOCKS blocks: the blocks are
         // evaluated in up to FORCE_RANGES ranges of at least half that (each a
@@ -886,7 +889,8 @@ int tc_srv_solve(tc_context *c, const tc_request &r, TcTree &t, bool build, hipE
 size_t tc_tree_bytes(const TcTree &t)
 {
     size_t b = 0;
-    for (const DevBuf *d : {&t.keys, &t.perm, &t.src, &t.src32, &t.nodes, &t.exps, &t.exps32, &t.nodew, &t.selfid,
+    for (const DevBuf *d : {&t.keys, &t.perm, &t.src, &t.src32, &t.nodes, &t.exps, &t.dexps, &t.exps32, &t.nodew,
+                            &t.selfid,
                             &t.box_d})
         b += d->cap;
     return b;

@@ -1032,8 +1032,8 @@ template <int NV> TC_DEV double wave_reduce_scatter(double *v)
 template <int P>
 __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, const int2 *se, const int *level,
                                                       const int2 *cell, const double4 *src, const double *box,
-                                                      int nnodes, TcNode *nodes, double *exps, double4 *nodew,
-                                                      float4 *src32)
+                                                      int nnodes, TcNode *nodes, double *exps, double *dexps,
+                                                      double4 *nodew, float4 *src32)
 {
     const int id = tc_uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
     if (id >= nnodes || child[id] != 0)
@@ -1110,8 +1110,11 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
             v[k] = k < P ? re[k] : (k < 2 * P ? im[k - P] : 0.0);
         const double sum = wave_reduce_scatter<NV>(v);
         const int idx = NV == 64 ? lane : lane >> 1;
-        if (idx < 2 * P && (NV == 64 || (lane & 1) == 0))
+        if (idx < 2 * P && (NV == 64 || (lane & 1) == 0)) {
             ex[idx] = sum;
+            if (dexps)
+                dexps[(size_t)2 * P * id + idx] = (double)(idx < P ? idx + 1 : idx - P + 1) * sum;
+        }
     }
     if (lane == 0) {
         TcNode nd;
@@ -1174,7 +1177,7 @@ template <bool AGENT> TC_DEV void node_store(double *p, double v)
 // cached loads).  SHARED: another wave of this launch may read the node.
 template <int P, bool CHAIN, bool SHARED>
 TC_DEV void e2e_node(int rank, const int *selfid, const double *box, TcNode *nodes, double4 *nodew, double *exps,
-                     double2 (*s_a)[P], double *s_rec, const double *s_binom,
+                     double *dexps, double2 (*s_a)[P], double *s_rec, const double *s_binom,
                      double ninv)
 {
     constexpr int G = E2E_G<P>, NCH = 64 / G;
@@ -1323,6 +1326,10 @@ TC_DEV void e2e_node(int rank, const int *selfid, const double *box, TcNode *nod
     if (lane < P) {
         node_store<SHARED>(exps + (size_t)2 * P * id + lane, dre);
         node_store<SHARED>(exps + (size_t)2 * P * id + P + lane, dim);
+        if (dexps) {
+            dexps[(size_t)2 * P * id + lane] = (double)(lane + 1) * dre;
+            dexps[(size_t)2 * P * id + P + lane] = (double)(lane + 1) * dim;
+        }
     }
     // the record and weights, a word per lane again
     tc_wave_sync();
@@ -1358,7 +1365,7 @@ static_assert(offsetof(TcNode, mass) == 24 && offsetof(TcNode, s) == 32 && offse
 template <int P>
 __global__ __launch_bounds__(256) void k_e2e_level(const int *__restrict__ selfid, int r0, int r1,
                                                    const double *__restrict__ box, TcNode *nodes, double4 *nodew,
-                                                   double *exps)
+                                                   double *exps, double *dexps)
 {
     __shared__ double s_binom[P * P];
     __shared__ double2 s_a[4][4][P];
@@ -1367,7 +1374,7 @@ __global__ __launch_bounds__(256) void k_e2e_level(const int *__restrict__ selfi
     __syncthreads();
     const int wid = threadIdx.x >> 6, rank = tc_uniform(r0 + (int)blockIdx.x * 4 + wid);
     if (rank < r1)
-        e2e_node<P, false, false>(rank, selfid, box, nodes, nodew, exps, s_a[wid], s_rec[wid], s_binom,
+        e2e_node<P, false, false>(rank, selfid, box, nodes, nodew, exps, dexps, s_a[wid], s_rec[wid], s_binom,
                                   -(1.0 / (double)(tc_lane() % E2E_G<P> + 1)));
 }
 
@@ -1390,7 +1397,7 @@ constexpr int E2E_CHAIN_T = 4096;
 template <int P>
 __global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, const int *__restrict__ parent,
                                              uint32_t *pend, int T, int tlast, const double *__restrict__ box,
-                                             TcNode *nodes, double4 *nodew, double *exps)
+                                             TcNode *nodes, double4 *nodew, double *exps, double *dexps)
 {
     __shared__ double s_binom[P * P];
     __shared__ double2 s_a[4][4][P];
@@ -1405,7 +1412,7 @@ __global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, con
     if (!start)
         return;
     const double ninv = -(1.0 / (double)(tc_lane() % E2E_G<P> + 1));  // -1 / (this lane's coefficient index)
-    e2e_node<P, false, true>(rank, selfid, box, nodes, nodew, exps, s_a[wid], s_rec[wid], s_binom, ninv);
+    e2e_node<P, false, true>(rank, selfid, box, nodes, nodew, exps, dexps, s_a[wid], s_rec[wid], s_binom, ninv);
     while (rank != 0) {
         const int up = tc_uniform(parent[rank]);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -1417,7 +1424,7 @@ __global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, con
             break;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         rank = up;
-        e2e_node<P, true, true>(rank, selfid, box, nodes, nodew, exps, s_a[wid], s_rec[wid], s_binom, ninv);
+        e2e_node<P, true, true>(rank, selfid, box, nodes, nodew, exps, dexps, s_a[wid], s_rec[wid], s_binom, ninv);
     }
 }
 
@@ -1456,6 +1463,14 @@ __global__ __launch_bounds__(256) void k_exps32(const TcNode *nodes, const doubl
         b *= inv;
     }
     ex32[(size_t)(P + 1) * id + k] = make_float2((float)a, (float)b);
+}
+
+// k a_k of every node, for a force tree that was built with FP32 mirrors alone.
+__global__ __launch_bounds__(256) void k_deriv(const double *__restrict__ exps, size_t total, int p,
+                                               double *__restrict__ dexps)
+{
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256)
+        dexps[i] = (double)((int)(i % (size_t)p) + 1) * exps[i];
 }
 
 int tiles_of(int n, int t) { return (n + t - 1) / t; }
@@ -1607,8 +1622,9 @@ static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, cons
                           const int *parent, uint32_t *pend, bool fp32, bool deriv, hipStream_t st)
 {
     const double *box = t.box_d.as<double>();
+    double *dexps = t.has_deriv ? t.dexps.as<double>() : nullptr;
     k_leaf_upward<P><<<tiles_of(t.nnodes, 4), 256, 0, st>>>(child, se, lev, cell, t.src.as<double4>(), box,
-                                                             t.nnodes, t.nodes.as<TcNode>(), t.exps.as<double>(),
+                                                             t.nnodes, t.nodes.as<TcNode>(), t.exps.as<double>(), dexps,
                                                              t.nodew.as<double4>(),
                                                              fp32 ? t.src32.as<float4>() : nullptr);
     TC_HIP(hipGetLastError());
@@ -1620,7 +1636,7 @@ static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, cons
         const int r0 = t.level_start[L], r1 = t.level_start[L + 1];
         if (r1 > r0) {
             k_e2e_level<P><<<tiles_of(r1 - r0, 4), 256, 0, st>>>(t.selfid.as<int>(), r0, r1, box, t.nodes.as<TcNode>(),
-                                                                  t.nodew.as<double4>(), t.exps.as<double>());
+                                                                  t.nodew.as<double4>(), t.exps.as<double>(), dexps);
             TC_HIP(hipGetLastError());
         }
     }
@@ -1628,7 +1644,7 @@ static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, cons
         const int T = t.level_start[lt];
         k_e2e<P><<<tiles_of(T, 4), 256, 0, st>>>(t.selfid.as<int>(), parent, pend, T,
                                                  lt < TC_LMAX ? t.level_start[lt - 1] : T, box, t.nodes.as<TcNode>(),
-                                                 t.nodew.as<double4>(), t.exps.as<double>());
+                                                 t.nodew.as<double4>(), t.exps.as<double>(), dexps);
         TC_HIP(hipGetLastError());
     }
     if (fp32) {
@@ -1640,7 +1656,7 @@ static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, cons
 }
 
 void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v, int n, int leafcap, int order,
-                   bool fp32, bool deriv32, TcScratch &ws, hipStream_t st, const hipEvent_t *ev,
+                   bool fp32, bool deriv, TcScratch &ws, hipStream_t st, const hipEvent_t *ev,
                    const std::function<void()> *at_census)
 {
     if (n <= 0)
@@ -1655,7 +1671,8 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     t.order = order;
     t.leafcap = leafcap;
     t.has_fp32 = fp32;
-    t.deriv32 = fp32 && deriv32;
+    t.deriv32 = fp32 && deriv;
+    t.has_deriv = !fp32 && deriv;
     t.box_d.reserve(sizeof(double) * 4);
     t.keys.reserve(sizeof(uint32_t) * (size_t)n);
     t.perm.reserve(sizeof(uint32_t) * (size_t)n);
@@ -1706,6 +1723,8 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
 
     t.nodes.reserve(sizeof(TcNode) * (size_t)nn);
     t.exps.reserve(sizeof(double) * 2 * (size_t)order * nn);
+    if (t.has_deriv)
+        t.dexps.reserve(sizeof(double) * 2 * (size_t)order * nn);
     t.nodew.reserve(sizeof(double4) * (size_t)nn);
     t.selfid.reserve(sizeof(int) * (size_t)(T + 1));
     if (fp32)
@@ -1739,12 +1758,24 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
 
     switch (order) {
 #define TC_CASE(P) \
-    case P: upward_launch<P>(t, child, se, lev, cell, ws.ilevel.as<int>(), pend, fp32, deriv32, st); break;
+    case P: upward_launch<P>(t, child, se, lev, cell, ws.ilevel.as<int>(), pend, fp32, deriv, st); break;
         TC_ORDERS(TC_CASE)
 #undef TC_CASE
     }
     if (ev)
         TC_HIP(hipEventRecord(ev[3], st));
+}
+
+void tc_tree_deriv(TcTree &t, hipStream_t st)
+{
+    if (t.has_deriv)
+        return;
+    const size_t total = 2 * (size_t)t.order * t.nnodes;
+    t.dexps.reserve(sizeof(double) * total);
+    k_deriv<<<(int)std::min<size_t>((total + 255) / 256, 4096), 256, 0, st>>>(t.exps.as<double>(), total, t.order,
+                                                                           t.dexps.as<double>());
+    TC_HIP(hipGetLastError());
+    t.has_deriv = true;
 }
 
 const uint32_t *tc_targets_bad_flag(TcScratch &ws, int m) { return tc_bbox_bad_flag(ws, m); }

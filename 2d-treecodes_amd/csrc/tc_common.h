@@ -6,7 +6,8 @@
 //   permutation      uint32  sorted -> input index 4 B/source
 //   nodes            TcNode (64 B), breadth-first ids: root 0, children of the
 //                    k-th internal node (level, Morton order) at 1 + 4k + c
-//   expansions       double[2p] per node: [Re a_1..a_p][Im a_1..a_p]
+//   expansions       double[2p] per node: [Re a_1..a_p][Im a_1..a_p]; FP64 force
+//                    trees also k a_k in the same layout (the derivative series)
 //   FP32 mirrors     float4 {x-xc, y-yc, v, 0} per source (leaf-relative) and
 //                    float2[p] per node of scaled coefficients a_j / r^j
 //                    (j a_j / r^j for force trees)
@@ -285,16 +286,17 @@ struct TcTree {
     double box[4] = {0, 0, 0, 0};        // xmin, ymin, ext, scale (host copy)
     bool has_fp32 = false;
     bool deriv32 = false;  // FP32 coefficient mirror holds k b_k
-    DevBuf keys, perm, src, src32, nodes, exps, exps32, nodew, selfid;
+    bool has_deriv = false;  // dexps holds k a_k (FP64 force trees)
+    DevBuf keys, perm, src, src32, nodes, exps, dexps, exps32, nodew, selfid;
     DevBuf box_d;
     void release()
     {
-        for (DevBuf *b : {&keys, &perm, &src, &src32, &nodes, &exps, &exps32, &nodew, &selfid, &box_d})
+        for (DevBuf *b : {&keys, &perm, &src, &src32, &nodes, &exps, &dexps, &exps32, &nodew, &selfid, &box_d})
             b->release();
     }
     void bind(TcArena *a)
     {
-        for (DevBuf *b : {&keys, &perm, &src, &src32, &nodes, &exps, &exps32, &nodew, &selfid, &box_d})
+        for (DevBuf *b : {&keys, &perm, &src, &src32, &nodes, &exps, &dexps, &exps32, &nodew, &selfid, &box_d})
             b->bind(a);
     }
 };
@@ -370,15 +372,17 @@ void tc_sort_points(const double *x, const double *y, const double *v, int n, do
 void tc_morton_sort(const double *x, const double *y, const double *v, int n, const double *box_d,
                     uint32_t *keys_out, uint32_t *perm_out, double4 *packed, TcScratch &ws, hipStream_t st,
                     bool hilbert, const hipEvent_t *ev, uint32_t *lb);
-// fp32: also build the FP32 mirrors; deriv32: the coefficient mirror holds
-// k b_k (force trees) instead of b_k (potential trees).
+// fp32: also build the FP32 mirrors; deriv: a force tree, whose coefficient
+// mirror holds k b_k instead of b_k, and which without mirrors (FP64) keeps k a_k.
 // ev (optional, four events): recorded after the Morton keys, the sorted
 // records, the topology and the upward pass (the build's phase boundaries).
 // at_census (optional): called once the census readback is queued, before the
 // host waits for it (the caller can queue independent work on another stream).
 void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v, int n, int leafcap, int order,
-                   bool fp32, bool deriv32, TcScratch &ws, hipStream_t st, const hipEvent_t *ev = nullptr,
+                   bool fp32, bool deriv, TcScratch &ws, hipStream_t st, const hipEvent_t *ev = nullptr,
                    const std::function<void()> *at_census = nullptr);
+// Adds k a_k to a force tree that has none (one built for FP32), for an FP64 evaluation of it.
+void tc_tree_deriv(TcTree &t, hipStream_t st);
 void tc_sort_targets(const double *xt, const double *yt, int m, TcScratch &ws, hipStream_t st);
 // Several target sets of at most TC_SORT_SMALL_MAX targets each sorted in one
 // launch: tc_sort_targets_desc reserves ws's target buffers for m targets (as

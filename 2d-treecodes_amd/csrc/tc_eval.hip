@@ -40,19 +40,9 @@ __constant__ double c_binomT[TC_MAXORDER * 64];  // c_binomT[k*64 + n] = C(n, k)
 TC_DEV float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 TC_DEV float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// 1/d to ~1 ulp for positive normal d: hardware estimate + two Newton steps.
+// 1/d to ~1 ulp for positive normal d: hardware estimate and one third-order step,
+// r (1 + e + e^2): three FMAs on an estimate good to 2^-22 or better.
 TC_DEV double rcp64(double d)
-{
-    double r = __builtin_amdgcn_rcp(d);
-    double e = fma(-d, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-d, r, 1.0);
-    return fma(r, e, r);
-}
-
-// The same by one third-order step, r (1 + e + e^2): three FMAs on an
-// estimate good to 2^-22 or better.
-TC_DEV double rcp64_3(double d)
 {
     const double r = __builtin_amdgcn_rcp(d);
     const double e = fma(-d, r, 1.0);
@@ -102,7 +92,7 @@ template <int P>
 TC_DEV double e2p_pot64(double rz, double iz, double mass, const double *__restrict__ ex, const double2 *logtab)
 {
     const double r2 = fma(rz, rz, iz * iz);
-    const double inv = rcp64_3(r2);
+    const double inv = rcp64(r2);
     const double ur = rz * inv, ui = -iz * inv;
     double ar = ex[P - 1], ai = ex[2 * P - 1];
 #pragma unroll
@@ -136,19 +126,20 @@ TC_DEV float e2p_pot32(float rz, float iz, const float2 *__restrict__ ex)
 }
 
 // force_e2p_8x8 (force-kernels.m4:57-98) for one target: dphi/dz =
-// Q u - sum_k k a_k u^(k+1) = u (Q - u T), T = sum_k k a_k u^(k-1) by Horner;
+// Q u - sum_k k a_k u^(k+1) = u (Q - u T), T = sum_k k a_k u^(k-1) by Horner on
+// the derivative coefficients ex = k a_k (a force tree keeps them beside the a_k:
+// forming them here cost a multiplication for every two FMAs);
 // fx += Re dphi/dz, fy -= Im dphi/dz.
 template <int P>
 TC_DEV void e2p_force64(double rz, double iz, double mass, const double *__restrict__ ex, double &fx, double &fy)
 {
-    const double inv = 1.0 / fma(rz, rz, iz * iz);
+    const double inv = rcp64(fma(rz, rz, iz * iz));
     const double ur = rz * inv, ui = -iz * inv;
-    double ar = (double)P * ex[P - 1], ai = (double)P * ex[2 * P - 1];
+    double ar = ex[P - 1], ai = ex[2 * P - 1];
 #pragma unroll
     for (int j = P - 2; j >= 0; --j) {
-        const double k = (double)(j + 1);
-        const double tr = fma(ur, ar, fma(-ui, ai, k * ex[j]));
-        const double ti = fma(ur, ai, fma(ui, ar, k * ex[P + j]));
+        const double tr = fma(ur, ar, fma(-ui, ai, ex[j]));
+        const double ti = fma(ur, ai, fma(ui, ar, ex[P + j]));
         ar = tr;
         ai = ti;
     }
@@ -683,13 +674,16 @@ TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ no
 // One lane per target over all sources, with a 30-operation log: 12.7 -> 8.6 ms
 // at 2^22 (order 9 / leaf 64, theta 0.3; build 0.7 ms of it), 1.11 -> 0.60 ms at
 // 2^18 (12 / 512), 0.53 -> 0.28 ms at 2^16 with 32 targets a wave.
+struct TcWave64 {
+    TcStackEntry stk[TC_STACK];
+    double2 tgt[64];  // the wave's targets
+    double2 xy[64];   // source tile
+    double v[64];
+    int act[64];      // the active lanes
+};
 struct TcPotShared64 {
-    TcStackEntry stk[4][TC_STACK];
-    double2 tgt[4][64];    // the wave's targets
-    double2 xy[4][64];     // source tile
-    double v[4][64];
-    double res[4][64];     // leaf sums of the active targets
-    int act[4][64];        // the active lanes
+    TcWave64 w[4];
+    double res[4][64];  // leaf sums of the active targets
     double2 logtab[LOG_TAB];
     TC_DEV void init()
     {
@@ -698,21 +692,32 @@ struct TcPotShared64 {
     }
 };
 
-// Sum over the leaf's sources [s, e) at the targets of the lanes in omask
-// (valid in those lanes; log of the squared distance, so twice the potential).
-TC_DEV double p2p_leaf64(TcPotShared64 &sh, const double4 *__restrict__ src, int s, int e, unsigned long long omask)
+TC_DEV void acc_add(double &a, double b) { a += b; }
+TC_DEV void acc_add(double2 &a, double2 b)
 {
-    const int wid = threadIdx.x >> 6, lane = tc_lane();
-    double2 *const s_xy = sh.xy[wid], *const s_t = sh.tgt[wid];
-    double *const s_v = sh.v[wid], *const s_res = sh.res[wid];
-    int *const s_act = sh.act[wid];
+    a.x += b.x;
+    a.y += b.y;
+}
+TC_DEV double acc_shfl_xor(double a, int off) { return __shfl_xor(a, off, 64); }
+TC_DEV double2 acc_shfl_xor(double2 a, int off)
+{
+    return make_double2(__shfl_xor(a.x, off, 64), __shfl_xor(a.y, off, 64));
+}
+
+// Sum over the leaf's sources [s, e) of pair(acc, dx, dy, v), d = target -
+// source, at the targets of the lanes in omask (the sum is valid in those lanes).
+template <class Acc, class Pair>
+TC_DEV Acc p2p_leaf64(TcWave64 &w, Acc *s_res, const double4 *__restrict__ src, int s, int e,
+                      unsigned long long omask, Pair &&pair)
+{
+    const int lane = tc_lane();
     const int k = __popcll(omask), rank = __popcll(omask & tc_lanemask_lt());
     const bool act = __builtin_amdgcn_inverse_ballot_w64(omask);
     const int row = lane >> 3, q = lane & 7;
     if (act)
-        s_act[rank] = lane;
+        w.act[rank] = lane;
     for (int b = 0; b < k; b += 16) {
-        double a0 = 0, a1 = 0;
+        Acc a0{}, a1{};
         const int left = k - b;
         // lanes past the end repeat the last source with weight zero; a leaf of one
         // tile is staged once
@@ -721,40 +726,35 @@ TC_DEV double p2p_leaf64(TcPotShared64 &sh, const double4 *__restrict__ src, int
         if (stage)
             nx = src[min(s + lane, e - 1)];
         tc_wave_sync();
-        const double2 t0 = s_t[s_act[b + min(row, left - 1)]], t1 = s_t[s_act[b + min(row + 8, left - 1)]];
+        const double2 t0 = w.tgt[w.act[b + min(row, left - 1)]], t1 = w.tgt[w.act[b + min(row + 8, left - 1)]];
         for (int b0 = s; b0 < e; b0 += 64) {
             const int cnt = min(64, e - b0), n8 = (cnt + 7) >> 3;
             if (stage) {
                 tc_wave_sync();
-                s_xy[lane] = make_double2(nx.x, nx.y);
-                s_v[lane] = lane < cnt ? nx.z : 0.0;
+                w.xy[lane] = make_double2(nx.x, nx.y);
+                w.v[lane] = lane < cnt ? nx.z : 0.0;
                 if (b0 + 64 < e)
                     nx = src[min(b0 + 64 + lane, e - 1)];
                 tc_wave_sync();
             }
             if (left > 8) {
                 for (int i = 0; i < n8; ++i) {
-#pragma clang fp contract(fast)
-                    const double2 p = s_xy[8 * i + q];
-                    const double v = s_v[8 * i + q];
-                    const double ax = t0.x - p.x, ay = t0.y - p.y;
-                    const double bx = t1.x - p.x, by = t1.y - p.y;
-                    a0 += log64(ax * ax + (ay * ay + EPS_REG), sh.logtab) * v;
-                    a1 += log64(bx * bx + (by * by + EPS_REG), sh.logtab) * v;
+                    const double2 p = w.xy[8 * i + q];
+                    const double v = w.v[8 * i + q];
+                    pair(a0, t0.x - p.x, t0.y - p.y, v);
+                    pair(a1, t1.x - p.x, t1.y - p.y, v);
                 }
             } else {
                 for (int i = 0; i < n8; ++i) {
-#pragma clang fp contract(fast)
-                    const double2 p = s_xy[8 * i + q];
-                    const double ax = t0.x - p.x, ay = t0.y - p.y;
-                    a0 += log64(ax * ax + (ay * ay + EPS_REG), sh.logtab) * s_v[8 * i + q];
+                    const double2 p = w.xy[8 * i + q];
+                    pair(a0, t0.x - p.x, t0.y - p.y, w.v[8 * i + q]);
                 }
             }
         }
 #pragma unroll
         for (int off = 1; off < 8; off <<= 1) {
-            a0 += __shfl_xor(a0, off, 64);
-            a1 += __shfl_xor(a1, off, 64);
+            acc_add(a0, acc_shfl_xor(a0, off));
+            acc_add(a1, acc_shfl_xor(a1, off));
         }
         if (q == 0) {
             s_res[b + row] = a0;
@@ -776,7 +776,7 @@ TC_DEV void potential_wave64(TcPotShared64 &sh, const TcNode *__restrict__ nodes
                              unsigned long long *counters)
 {
     const int wid = threadIdx.x >> 6, lane = tc_lane();
-    TcStackEntry *const stk = sh.stk[wid];
+    TcStackEntry *const stk = sh.w[wid].stk;
     const int k = k0 + lane;
     const bool valid = lane < tpw && k < m;
     const uint32_t ti = valid ? tperm[k] : 0u;
@@ -784,7 +784,7 @@ TC_DEV void potential_wave64(TcPotShared64 &sh, const TcNode *__restrict__ nodes
     const unsigned long long live = tc_ballot(valid);
     if (!live)
         return;
-    sh.tgt[wid][lane] = make_double2(x, y);
+    sh.w[wid].tgt[lane] = make_double2(x, y);
     double acc = 0;
     unsigned long long np2p = 0, ne2p = 0, nslots = 0, neslots = 0;
     // CNT: wave clock cycles per category (direct sums, per-target multipoles) and in total
@@ -827,7 +827,12 @@ TC_DEV void potential_wave64(TcPotShared64 &sh, const TcNode *__restrict__ nodes
                 np2p += nact * nsrc;
                 nslots += ((nact + 7) >> 3 << 3) * ((nsrc + 7) >> 3 << 3);
             }
-            const double leafsum = p2p_leaf64(sh, src, nd.s, nd.e, omask);
+            // twice the potential: the log of the squared distance
+            const double leafsum = p2p_leaf64(sh.w[wid], sh.res[wid], src, nd.s, nd.e, omask,
+                                              [&](double &a, double dx, double dy, double v) {
+#pragma clang fp contract(fast)
+                                                  a += log64(dx * dx + (dy * dy + EPS_REG), sh.logtab) * v;
+                                              });
             if (__builtin_amdgcn_inverse_ballot_w64(omask))
                 acc += leafsum * 0.5;
             if constexpr (CNT)
@@ -862,7 +867,8 @@ TC_DEV void potential_wave64(TcPotShared64 &sh, const TcNode *__restrict__ nodes
 
 // (separate kernel arguments rather than a TcPotReq: a by-value struct
 // argument costs this kernel registers and occupancy)
-// tpw: targets per wave (FP64 only; FP32 waves hold 64).
+// tpw: targets per wave (FP64 only; FP32 waves hold 64, since an FP32 result's
+// rounding depends on its wave).
 template <int P, bool F32, bool CNT>
 __global__ __launch_bounds__(256) void k_potential(const TcNode *__restrict__ nodes, const double *__restrict__ exps,
                                                    const float2 *__restrict__ exps32,
@@ -1157,7 +1163,7 @@ TC_DEV void stage_rows(const int *list, int b0, int cnt, const void *base, void 
 // force-kernels.m4:57-98), E2P_QB nodes per staged batch.
 template <int P, bool F32>
 TC_DEV void force_flush_e2p(const int *list, int n, const TcNode *__restrict__ nodes,
-                            const double *__restrict__ exps, const float2 *__restrict__ exps32, double4 *buf,
+                            const double *__restrict__ dexps, const float2 *__restrict__ exps32, double4 *buf,
                             double xb, double yb, int ix, int iy, double h, double &fx, double &fy)
 {
     constexpr int QB = ForceCfg<P, F32>::E2P_QB;
@@ -1169,7 +1175,7 @@ TC_DEV void force_flush_e2p(const int *list, int n, const TcNode *__restrict__ n
         if (F32)
             stage_rows<8 * (P + 1), 4, QB>(list, b0, cnt, exps32, co);
         else
-            stage_rows<16 * P, 16, QB>(list, b0, cnt, exps, co);
+            stage_rows<16 * P, 16, QB>(list, b0, cnt, dexps, co);
         vm_wait_all();
         tc_wave_sync();
         for (int t = 0; t < cnt; ++t) {
@@ -1450,6 +1456,7 @@ TC_DEV void force_skip_p2p(const int *list, int n, int &skip, const TcNode *__re
 // CNT: the instance launched with counters, which also times the categories
 template <int P, bool F32, bool NEAR, bool CNT>
 __global__ __launch_bounds__(256, 4) void k_force(const TcNode *__restrict__ nodes, const double *__restrict__ exps,
+                                               const double *__restrict__ dexps,
                                                const float2 *__restrict__ exps32, const double4 *__restrict__ src,
                                                const float4 *__restrict__ src32, const double *__restrict__ x0s,
                                                const double *__restrict__ y0s, const double *__restrict__ hs,
@@ -1578,7 +1585,7 @@ __global__ __launch_bounds__(256, 4) void k_force(const TcNode *__restrict__ nod
                 ne2p += 64ull * ne;
                 if (timing)
                     tc0 = tc_clock();
-                force_flush_e2p<P, F32>(lst_e, ne, nodes, exps, exps32, s_buf[wid], xb, yb, ix, iy, h, fx, fy);
+                force_flush_e2p<P, F32>(lst_e, ne, nodes, dexps, exps32, s_buf[wid], xb, yb, ix, iy, h, fx, fy);
                 if (timing)
                     ce2p += tc_clock() - tc0;
                 ne = 0;
@@ -1628,7 +1635,7 @@ __global__ __launch_bounds__(256, 4) void k_force(const TcNode *__restrict__ nod
             ne2p += 64ull * ne;
             if (timing)
                 tc0 = tc_clock();
-            force_flush_e2p<P, F32>(lst_e, ne, nodes, exps, exps32, s_buf[wid], xb, yb, ix, iy, h, fx, fy);
+            force_flush_e2p<P, F32>(lst_e, ne, nodes, dexps, exps32, s_buf[wid], xb, yb, ix, iy, h, fx, fy);
             if (timing)
                 ce2p += tc_clock() - tc0;
         }
@@ -1770,57 +1777,66 @@ __global__ __launch_bounds__(256) void k_force_combine(const double *__restrict_
 // rejects non-block targets for velocities).  Same masked wave traversal as
 // k_potential -- per-target accept test r^2 < theta^2 d^2 -- with the force
 // E2P (force-kernels.m4:57-98 per target) and the force P2P pair term
-// (force-kernels.m4:46-52).
+// (force-kernels.m4:46-52).  tpw targets per wave; a target's result does not
+// depend on it.  FP64 direct sums in 8 x 8 arrangements (p2p_leaf64); FP32 ones
+// by one lane per target over LDS tiles, flushed into FP64 per tile.
+// Order 24 / leaf 192, 200,000 sources, the whole solve: 100,003 targets 808 -> 536
+// us, 1,000 scattered ones 3070 -> 594 (FP32 2069 -> 759).
+template <bool F32> struct TcForceTgtShared {
+    TcWave64 w[4];
+    double2 res[4][F32 ? 1 : 64];
+};
 template <int P, bool F32>
 __global__ __launch_bounds__(256) void k_force_targets(const TcNode *__restrict__ nodes,
-                                                       const double *__restrict__ exps,
+                                                       const double *__restrict__ dexps,
                                                        const float2 *__restrict__ exps32,
                                                        const double4 *__restrict__ src,
                                                        const float4 *__restrict__ src32,
                                                        const double *__restrict__ xt, const double *__restrict__ yt,
                                                        const uint32_t *__restrict__ tperm, int m, double th2,
                                                        double *__restrict__ xres, double *__restrict__ yres,
-                                                       unsigned long long *counters)
+                                                       unsigned long long *counters, int tpw)
 {
-    __shared__ int s_node[4][TC_STACK];
-    __shared__ unsigned long long s_mask[4][TC_STACK];
-    __shared__ double4 s_src[4][64];
+    __shared__ TcForceTgtShared<F32> sh;
     const int wid = threadIdx.x >> 6, lane = tc_lane();
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    const bool valid = k < m;
+    TcWave64 &w = sh.w[wid];
+    const int k = (tc_xcd_chunk_block(TC_XCD_CHUNK_LOG2) * 4 + wid) * tpw + lane;
+    const bool valid = lane < tpw && k < m;
     const uint32_t ti = valid ? tperm[k] : 0u;
     const double x = valid ? xt[ti] : 0.0, y = valid ? yt[ti] : 0.0;
     const unsigned long long live = tc_ballot(valid);
     if (!live)
         return;
+    w.tgt[lane] = make_double2(x, y);
     double fx = 0, fy = 0;
     unsigned long long np2p = 0, ne2p = 0, nslots = 0, neslots = 0;
-    s_node[wid][0] = 0;
-    s_mask[wid][0] = live;
+    if (lane == 0)
+        w.stk[0] = TcStackEntry{live, 0, 0};
     int sp = 1;
     while (sp > 0) {
         --sp;
         tc_wave_sync();
-        const int id = tc_uniform(s_node[wid][sp]);
-        const unsigned long long mask = tc_uniform64(s_mask[wid][sp]);
+        // one LDS read, made scalar before the record's loads (see potential_wave32)
+        const uint4 top = *reinterpret_cast<const uint4 *>(&w.stk[sp]);
+        const int id = tc_uniform((int)top.z);
+        const unsigned long long mask =
+            ((unsigned long long)(unsigned)tc_uniform((int)top.y) << 32) | (unsigned)tc_uniform((int)top.x);
         // no early exit for empty nodes: all fields of the record are needed
         // before any branch, so they arrive in one round of scalar loads (an
         // empty node leaves no lane accepting or opening it)
         const TcNode nd = nodes[id];
         const bool nonempty = nd.s != nd.e;
-        const bool in = ((mask >> lane) & 1ull) && nonempty;
         const double dx = x - nd.xcom, dy = y - nd.ycom;
         const double r2 = dx * dx + dy * dy;
-        const bool acc_ok = in && (nd.r * nd.r < th2 * r2);
-        const unsigned long long amask = tc_ballot(acc_ok);
-        if (acc_ok) {
+        const unsigned long long amask = tc_ballot(nd.rr < th2 * r2) & mask & (nonempty ? ~0ull : 0ull);
+        if (__builtin_amdgcn_inverse_ballot_w64(amask)) {
             if (F32) {
                 float gx, gy;
                 e2p_force32<P>((float)dx, (float)dy, exps32 + (size_t)(P + 1) * id, gx, gy);
                 fx += (double)gx;
                 fy += (double)gy;
             } else {
-                e2p_force64<P>(dx, dy, nd.mass, exps + (size_t)2 * P * id, fx, fy);
+                e2p_force64<P>(dx, dy, nd.mass, dexps + (size_t)2 * P * id, fx, fy);
             }
         }
         ne2p += __popcll(amask);
@@ -1829,12 +1845,13 @@ __global__ __launch_bounds__(256) void k_force_targets(const TcNode *__restrict_
         if (!omask)
             continue;
         if (nd.child == 0) {
-            const bool act = (omask >> lane) & 1ull;
-            np2p += (unsigned long long)__popcll(omask) * (unsigned long long)(nd.e - nd.s);
-            nslots += 64ull * (unsigned long long)(nd.e - nd.s);
-            if (F32) {
+            const bool act = __builtin_amdgcn_inverse_ballot_w64(omask);
+            const unsigned long long nact = __popcll(omask), nsrc = nd.e - nd.s;
+            np2p += nact * nsrc;
+            nslots += F32 ? 64ull * nsrc : ((nact + 7) >> 3 << 3) * ((nsrc + 7) >> 3 << 3);
+            if constexpr (F32) {
                 const float tx = (float)(x - nd.xcom), ty = (float)(y - nd.ycom);
-                float4 *tile = reinterpret_cast<float4 *>(&s_src[wid][0]);
+                float4 *tile = reinterpret_cast<float4 *>(w.xy);
                 for (int b0 = nd.s; b0 < nd.e; b0 += 64) {
                     const int cnt = min(64, nd.e - b0);
                     if (lane < cnt)
@@ -1856,29 +1873,21 @@ __global__ __launch_bounds__(256) void k_force_targets(const TcNode *__restrict_
                     tc_wave_sync();
                 }
             } else {
-                for (int b0 = nd.s; b0 < nd.e; b0 += 64) {
-                    const int cnt = min(64, nd.e - b0);
-                    if (lane < cnt)
-                        s_src[wid][lane] = src[b0 + lane];
-                    tc_wave_sync();
-                    if (act) {
+                const double2 f = p2p_leaf64(w, sh.res[wid], src, nd.s, nd.e, omask,
+                                             [](double2 &a, double dx, double dy, double v) {
 #pragma clang fp contract(fast)
-                        for (int j = 0; j < cnt; ++j) {
-                            const double4 q = s_src[wid][j];
-                            const double ddx = x - q.x, ddy = y - q.y;
-                            const double f = q.z * rcp64(ddx * ddx + (ddy * ddy + EPS_REG));
-                            fx += ddx * f;
-                            fy += ddy * f;
-                        }
-                    }
-                    tc_wave_sync();
+                                                 const double g = v * rcp64(dx * dx + (dy * dy + EPS_REG));
+                                                 a.x += dx * g;
+                                                 a.y += dy * g;
+                                             });
+                if (act) {
+                    fx += f.x;
+                    fy += f.y;
                 }
             }
         } else {
-            if (lane < 4) {
-                s_node[wid][sp + lane] = nd.child + lane;
-                s_mask[wid][sp + lane] = omask;
-            }
+            if (lane < 4)
+                w.stk[sp + lane] = TcStackEntry{omask, nd.child + lane, 0};
             sp += 4;
         }
     }
@@ -1964,25 +1973,25 @@ TcPotReq potential_req(const TcTree &t, double th2, const double *xt, const doub
     return rq;
 }
 
-// Targets per wave of the FP64 potential: fewer where m targets would leave
-// SIMDs without a wave.  The direct sums' cost per target does not depend on it
-// (batches of 8 or 16 targets), the walk's and the multipoles' does, so full waves
-// from 2^17 targets on.  Whole solves (order 12 / leaf 512; 9 / 64, theta 0.3) with
-// 64 / 32 / 16 / 8 targets per wave: 4,000 targets 305 / 213 / 172 / 158 us and
-// 452 / 341 / 275 / 265, 32,000: 724 / 470 / 362 / 354 and 551 / 499 / 495 / 546,
-// 64,000: 600 / 474 / 416 / 477 and 603 / 570 / 615 / 817, 256,000: 849 / 844 / 934 /
-// 1271 and 870 / 1087 / 1524 / 2256.
-int pot_targets_per_wave(int m)
-{
-    return m <= 8192 ? 8 : (m <= 49152 ? 16 : (m <= 131072 ? 32 : 64));
-}
+// Targets per wave of the FP64 potential and the force at targets: fewer where m
+// targets would leave SIMDs without a wave.  The FP64 direct sums' cost per target
+// does not depend on it (batches of 8 or 16 targets), the walk's and the
+// multipoles' does, so full waves from about 10^5 targets on.  Whole solves with 64 /
+// 32 / 16 / 8 targets per wave, potential 12 / 512; potential 9 / 64, theta 0.3;
+// force 24 / 192, 200,000 sources:
+//     4,000 targets  305 / 213 / 172 / 158  452 / 341 / 275 / 265   757 / 600 / 516 / 462 us
+//    32,000          724 / 470 / 362 / 354  551 / 499 / 495 / 546   560 / 491 / 458 / 520
+//    64,000          600 / 474 / 416 / 477  603 / 570 / 615 / 817   504 / 481 / 530 / 712
+//   128,000          622 / 551 / 573 / 703  682 / 715 / 920 / 1311  520 / 566 / 741 / 1017
+//   256,000          849 / 844 / 934 / 1271 870 / 1087 / 1524 / 2256 636 / 806 / 1064 / 1654
+int targets_per_wave(int m) { return m <= 8192 ? 8 : (m <= 49152 ? 16 : (m <= 98304 ? 32 : 64)); }
 
 template <int P>
 void launch_potential(const TcTree &t, double th2, const double *xt, const double *yt, const uint32_t *tperm,
                       int m, double *out, int precision, unsigned long long *counters, hipStream_t st,
                       int xcd_lc = TC_XCD_CHUNK_LOG2)
 {
-    const int tpw = precision == 1 ? 64 : pot_targets_per_wave(m);
+    const int tpw = precision == 1 ? 64 : targets_per_wave(m);
     const int grid = tiles_of(m, 4 * tpw);
     const TcPotReq q = potential_req(t, th2, xt, yt, tperm, m, out, precision, 0);
     auto go = [&](auto kern) {
@@ -2005,16 +2014,16 @@ void launch_force_targets(const TcTree &t, double th2, const double *xt, const d
                           int m, double *xr, double *yr, int precision, unsigned long long *counters,
                           hipStream_t st)
 {
-    const int grid = tiles_of(m, 256);
+    const int tpw = targets_per_wave(m);
+    const int grid = tiles_of(m, 4 * tpw);
     if (precision == 1)
-        k_force_targets<P, true><<<grid, 256, 0, st>>>(t.nodes.as<TcNode>(), t.exps.as<double>(),
-                                                       t.exps32.as<float2>(), t.src.as<double4>(),
-                                                       t.src32.as<float4>(), xt, yt, tperm, m, th2, xr, yr,
-                                                       counters);
+        k_force_targets<P, true><<<grid, 256, 0, st>>>(t.nodes.as<TcNode>(), nullptr, t.exps32.as<float2>(),
+                                                       t.src.as<double4>(), t.src32.as<float4>(), xt, yt, tperm, m,
+                                                       th2, xr, yr, counters, tpw);
     else
-        k_force_targets<P, false><<<grid, 256, 0, st>>>(t.nodes.as<TcNode>(), t.exps.as<double>(), nullptr,
+        k_force_targets<P, false><<<grid, 256, 0, st>>>(t.nodes.as<TcNode>(), t.dexps.as<double>(), nullptr,
                                                         t.src.as<double4>(), nullptr, xt, yt, tperm, m, th2, xr,
-                                                        yr, counters);
+                                                        yr, counters, tpw);
     TC_HIP(hipGetLastError());
 }
 
@@ -2045,6 +2054,7 @@ void launch_force_pass(const TcTree &t, double theta, const double *x0s, const d
 {
     const TcNode *nodes = t.nodes.as<TcNode>();
     const double *exps = t.exps.as<double>();
+    const double *dexps = F32 ? nullptr : t.dexps.as<double>();
     const float2 *exps32 = F32 ? t.exps32.as<float2>() : nullptr;
     const double4 *src = t.src.as<double4>();
     const float4 *src32 = F32 ? t.src32.as<float4>() : nullptr;
@@ -2052,21 +2062,21 @@ void launch_force_pass(const TcTree &t, double theta, const double *x0s, const d
     tc_fill_u32(nl.ctr, 0u, FN_NCTR, st);
     if (counters) {
         const int grid = std::min(tiles_of(nb, 4), resident_blocks<k_force<P, F32, false, true>>(device));
-        k_force<P, F32, false, true><<<grid, 256, 0, st>>>(nodes, exps, exps32, src, src32, x0s, y0s, hs, first, nb,
+        k_force<P, F32, false, true><<<grid, 256, 0, st>>>(nodes, exps, dexps, exps32, src, src32, x0s, y0s, hs, first, nb,
                                                            theta, xr, yr, counters, work, nl);
     } else {
         const int grid = std::min(tiles_of(nb, 4), resident_blocks<k_force<P, F32, false, false>>(device));
-        k_force<P, F32, false, false><<<grid, 256, 0, st>>>(nodes, exps, exps32, src, src32, x0s, y0s, hs, first,
+        k_force<P, F32, false, false><<<grid, 256, 0, st>>>(nodes, exps, dexps, exps32, src, src32, x0s, y0s, hs, first,
                                                             nb, theta, xr, yr, counters, work, nl);
     }
     // the chunk and overflow counts are on the device: persistent grids
     k_force_chunks<F32><<<512, 256, 0, st>>>(nodes, src, src32, x0s, y0s, hs, first, nl, counters);
     k_force_combine<<<64, 256, 0, st>>>(x0s, y0s, hs, first, nl, xr, yr);
     if (counters)
-        k_force<P, F32, true, true><<<256, 256, 0, st>>>(nodes, exps, exps32, src, src32, x0s, y0s, hs, first, nb,
+        k_force<P, F32, true, true><<<256, 256, 0, st>>>(nodes, exps, dexps, exps32, src, src32, x0s, y0s, hs, first, nb,
                                                          theta, xr, yr, counters, work, nl);
     else
-        k_force<P, F32, true, false><<<256, 256, 0, st>>>(nodes, exps, exps32, src, src32, x0s, y0s, hs, first, nb,
+        k_force<P, F32, true, false><<<256, 256, 0, st>>>(nodes, exps, dexps, exps32, src, src32, x0s, y0s, hs, first, nb,
                                                           theta, xr, yr, counters, work, nl);
     TC_HIP(hipGetLastError());
 }

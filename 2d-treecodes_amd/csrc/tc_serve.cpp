@@ -80,7 +80,8 @@ size_t tree_estimate(const tc_request &r)
     const size_t n = pos(r.n);
     const size_t p = (size_t)req_order(r);
     const size_t nodes = 4 * (15 * n / (size_t)req_leaf(r) + 1) + 1;
-    const size_t per_node = 64 + 16 * p + 32 + 4 + (r.precision ? 8 * (p + 1) : 0);
+    const size_t per_node = 64 + 16 * p + 32 + 4 +
+                            (r.precision ? 8 * (p + 1) : (r.kind == TC_REQ_FORCE ? 16 * p : 0));
     return n * (4 + 4 + 32 + (r.precision ? 16 : 0)) + nodes * per_node + (64u << 10);
 }
 

@@ -51,7 +51,7 @@ def test_sort_variants(pkg, oracle, wl, n):
 
 # FP64 potential: 8, 16, 32, 64 targets per wave, whatever the wave the same bits; leaves of one
 # and of several source tiles, full and ragged; 1 to 64 active lanes a leaf
-@pytest.mark.parametrize("m", [1, 7, 8192, 8193, 49152, 49153, 131072, 131073])
+@pytest.mark.parametrize("m", [1, 7, 8192, 8193, 49152, 49153, 98304, 98305])
 @pytest.mark.parametrize("order,leaf", [(9, 33), (12, 500)])
 def test_fp64_targets_per_wave(pkg, oracle, wl, m, order, leaf):
     xs, ys, vs, *_ = wl.mixed_plummer_potential(30011, seed=m % 89)
@@ -87,4 +87,36 @@ def test_fp64_potential_nonfinite_and_huge(pkg):
     want = [sum(v * 0.5 * np.log((a - s) ** 2 + (b - t) ** 2 + eps) for s, t, v in zip(xs, ys, vs))
             for a, b in zip(x[[0, 5]], y[[0, 5]])]
     assert np.allclose(o[[0, 5]], want, rtol=1e-14, atol=1e-15)
+    ctx.close()
+
+
+# force at targets: the same rule; a target's result is the same alone and among others
+@pytest.mark.parametrize("m", [1, 9, 8192, 8193, 49153, 98305])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_force_targets_per_wave(pkg, oracle, wl, m, precision):
+    xs, ys, vs, *_ = wl.gaussian4_force(20011, seed=m % 83)
+    st = wl.Stream(m)
+    xt, yt = st.uniform(m), st.uniform(m)
+    ctx = pkg.Context(precision=precision, force_order=12, force_leaf=70)
+    fx, fy = ctx.force_targets(0.5, xs, ys, vs, xt, yt)
+    idx = np.sort(np.random.default_rng(m).choice(m, min(m, 500), replace=False))
+    rx, ry, _ = oracle.force_targets(0.5, xs, ys, vs, xt[idx], yt[idx], order=12, leafcap=70)
+    tol = 1e-5 if precision else 1e-12
+    assert rel_l2(fx[idx], rx) <= tol and rel_l2(fy[idx], ry) <= tol
+    gx, gy = ctx.force_targets(0.5, xs, ys, vs, xt[idx[:17]], yt[idx[:17]])
+    assert np.array_equal(gx, fx[idx[:17]]) and np.array_equal(gy, fy[idx[:17]])
+    ctx.close()
+
+
+def test_fp64_force_on_fp32_tree(pkg, wl):
+    # a tree built for FP32 keeps no k a_k of its own: an FP64 evaluation of it adds them
+    xs, ys, vs, x0s, y0s, hs = wl.gaussian4_force(30000, seed=5, nbx=4, h=1.0 / 128)
+    ctx = pkg.Context(precision=pkg.FP64, force_order=10, force_leaf=64)
+    want = ctx.force(0.5, xs, ys, vs, x0s, y0s, hs)
+    ctx.set(pkg.OPT_PRECISION, pkg.FP32)
+    ctx.force(0.5, xs, ys, vs, x0s, y0s, hs)
+    ctx.set(pkg.OPT_PRECISION, pkg.FP64)
+    for _ in range(2):
+        got = ctx.force_resident(0.5, x0s, y0s, hs)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     ctx.close()
