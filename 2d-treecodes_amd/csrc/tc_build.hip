@@ -837,7 +837,7 @@ __global__ __launch_bounds__(SCAN_NT) void k_census(const uint32_t *cnt, uint32_
 
 template <int IT>
 __global__ __launch_bounds__(256) void k_int_emit(const uint32_t *keys, int n, int cap, const uint32_t *offs,
-                                                   int stride, int *istart, int *ilevel)
+                                                   int stride, int tmax, int *istart, int *ilevel)
 {
     __shared__ uint32_t s_cnt[4][TC_LMAX];
     const int wid = threadIdx.x >> 6;
@@ -863,8 +863,10 @@ __global__ __launch_bounds__(256) void k_int_emit(const uint32_t *keys, int n, i
             const unsigned long long b = tc_ballot(f);
             if (f) {
                 const uint32_t r = c[L] + __popcll(b & tc_lanemask_lt());
-                istart[r] = base + 64 * j + tc_lane();
-                ilevel[r] = L;
+                if (r < (uint32_t)tmax) {
+                    istart[r] = base + 64 * j + tc_lane();
+                    ilevel[r] = L;
+                }
             }
             c[L] += __popcll(b);
         }
@@ -872,14 +874,11 @@ __global__ __launch_bounds__(256) void k_int_emit(const uint32_t *keys, int n, i
 }
 
 constexpr int NODES_WAVE_T = 16384;
-
-// The root of a tree without internal nodes (one leaf).
-__global__ void k_topo_leaf(uint32_t *child, int n, int2 *se, int *level, int2 *cell)
+// Internal nodes of the tree being built, from its census record; the buffers hold
+// tmax.  None where the sort failed (bit 1 of the flag): the keys are then in no order.
+TC_DEV int census_nodes(const int *__restrict__ info, int tmax)
 {
-    child[0] = 0u;
-    se[0] = make_int2(0, n);
-    level[0] = 0;
-    cell[0] = make_int2(0, 0);
+    return info[TC_LMAX + 1] & 2 ? 0 : min(info[TC_LMAX], tmax);
 }
 
 // First position in [lo, hi) where pred is false (pred holds on a prefix of
@@ -918,10 +917,18 @@ template <int G, class Pred> TC_DEV int group_partition(int lo, int hi, Pred &&p
 template <int G>
 __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ keys, int n, int cap,
                                                     const int *__restrict__ istart, int *ilevel,
-                                                    const int *__restrict__ info, int T, int *__restrict__ selfid,
+                                                    const int *__restrict__ info, int tmax, int *__restrict__ selfid,
                                                     uint32_t *pend, uint32_t *child, int2 *se, int *level, int2 *cell)
 {
     const int r = blockIdx.x * (256 / G) + threadIdx.x / G, lane = threadIdx.x % G;
+    const int T = census_nodes(info, tmax);
+    if (T == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+        // a tree of one leaf
+        child[0] = 0u;
+        se[0] = make_int2(0, n);
+        level[0] = 0;
+        cell[0] = make_int2(0, 0);
+    }
     if (r >= T)
         return;
     const int L = ilevel[r], i = istart[r];
@@ -1032,11 +1039,11 @@ template <int NV> TC_DEV double wave_reduce_scatter(double *v)
 template <int P>
 __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, const int2 *se, const int *level,
                                                       const int2 *cell, const double4 *src, const double *box,
-                                                      int nnodes, TcNode *nodes, double *exps, double *dexps,
+                                                      const int *__restrict__ info, int tmax, TcNode *nodes, double *exps, double *dexps,
                                                       double4 *nodew, float4 *src32)
 {
     const int id = tc_uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    if (id >= nnodes || child[id] != 0)
+    if (id > 4 * census_nodes(info, tmax) || child[id] != 0)
         return;
     const int lane = tc_lane();
     const int2 r = se[id];
@@ -1394,9 +1401,15 @@ __global__ __launch_bounds__(256) void k_e2e_level(const int *__restrict__ selfi
 // 142 -> 90 at 2^23 (order 8), 45 -> 17 at 2^16 (order 12), 71 -> 37 at 10,000
 // (order 24).
 constexpr int E2E_CHAIN_T = 4096;
+// A build whose node bound is at most this is queued without waiting for its census
+// (tc_build_tree): bounded by the chained launch, whose waves are started at the
+// bound, and by the memory that nodes short of it leave unused.
+constexpr long long AHEAD_NODES = 16384;
+constexpr size_t AHEAD_BYTES = size_t(48) << 20;
 template <int P>
 __global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, const int *__restrict__ parent,
-                                             uint32_t *pend, int T, int tlast, const double *__restrict__ box,
+                                             uint32_t *pend, const int *__restrict__ info, int tmax, int tlast,
+                                             const double *__restrict__ box,
                                              TcNode *nodes, double4 *nodew, double *exps, double *dexps)
 {
     __shared__ double s_binom[P * P];
@@ -1404,7 +1417,7 @@ __global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, con
     __shared__ double s_rec[4][48];
     const int wid = threadIdx.x >> 6;
     int rank = tc_uniform((int)(blockIdx.x * 4 + wid));
-    const bool start = rank < T && (rank >= tlast || (pend[rank] >> 8) == 0);
+    const bool start = rank < census_nodes(info, tmax) && (rank >= tlast || (pend[rank] >> 8) == 0);
     if (!__syncthreads_or(start))
         return;
     e2e_binom<P>(s_binom);
@@ -1436,15 +1449,15 @@ __global__ __launch_bounds__(256) void k_e2e(const int *__restrict__ selfid, con
 // node's p + 1 records holds the E2P constants (s, Q ln2/2) for potential
 // trees (the FP32 E2P works with log2) and (s, Q) for force trees.
 template <int P>
-__global__ __launch_bounds__(256) void k_exps32(const TcNode *nodes, const double *exps, int nnodes, int deriv,
-                                                float2 *ex32)
+__global__ __launch_bounds__(256) void k_exps32(const TcNode *nodes, const double *exps, const int *__restrict__ info,
+                                                int tmax, int deriv, float2 *ex32)
 {
     // G lanes per node (p + 1 records each), 64 / G nodes per wave
     constexpr int G = P + 1 <= 16 ? 16 : (P + 1 <= 32 ? 32 : 64);
     const int lane = tc_lane();
     const int id = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / G) + lane / G;
     const int k = lane % G;
-    if (id >= nnodes || k > P)
+    if (id > 4 * census_nodes(info, tmax) || k > P)
         return;
     const double r = nodes[id].r;
     const double sc = r > 1e-30 ? r : 1e-30;
@@ -1617,42 +1630,63 @@ void tc_morton_sort(const double *x, const double *y, const double *v, int n, co
     }
 }
 
+// info, tmax: the tree's internal nodes as the kernels read them (at most tmax);
+// starts: its level starts, or null where the host does not have them yet (all
+// levels then go in the chained launch).
 template <int P>
 static void upward_launch(TcTree &t, const uint32_t *child, const int2 *se, const int *lev, const int2 *cell,
-                          const int *parent, uint32_t *pend, bool fp32, bool deriv, hipStream_t st)
+                          const int *parent, uint32_t *pend, bool fp32, bool deriv, const int *info, int tmax,
+                          const int *starts, hipStream_t st)
 {
     const double *box = t.box_d.as<double>();
     double *dexps = t.has_deriv ? t.dexps.as<double>() : nullptr;
-    k_leaf_upward<P><<<tiles_of(t.nnodes, 4), 256, 0, st>>>(child, se, lev, cell, t.src.as<double4>(), box,
-                                                             t.nnodes, t.nodes.as<TcNode>(), t.exps.as<double>(), dexps,
-                                                             t.nodew.as<double4>(),
-                                                             fp32 ? t.src32.as<float4>() : nullptr);
+    const int nn = 1 + 4 * tmax;
+    k_leaf_upward<P><<<tiles_of(nn, 4), 256, 0, st>>>(child, se, lev, cell, t.src.as<double4>(), box, info, tmax,
+                                                      t.nodes.as<TcNode>(), t.exps.as<double>(), dexps,
+                                                      t.nodew.as<double4>(), fp32 ? t.src32.as<float4>() : nullptr);
     TC_HIP(hipGetLastError());
     // levels lt and below one launch each, the levels above in one
-    int lt = TC_LMAX;
-    while (t.level_start[lt] > E2E_CHAIN_T)
-        --lt;
-    for (int L = TC_LMAX - 1; L >= lt; --L) {
-        const int r0 = t.level_start[L], r1 = t.level_start[L + 1];
-        if (r1 > r0) {
-            k_e2e_level<P><<<tiles_of(r1 - r0, 4), 256, 0, st>>>(t.selfid.as<int>(), r0, r1, box, t.nodes.as<TcNode>(),
-                                                                  t.nodew.as<double4>(), t.exps.as<double>(), dexps);
-            TC_HIP(hipGetLastError());
+    int top = tmax, last = INT_MAX;
+    if (starts) {
+        int lt = TC_LMAX;
+        while (starts[lt] > E2E_CHAIN_T)
+            --lt;
+        for (int L = TC_LMAX - 1; L >= lt; --L) {
+            const int r0 = starts[L], r1 = starts[L + 1];
+            if (r1 > r0) {
+                k_e2e_level<P><<<tiles_of(r1 - r0, 4), 256, 0, st>>>(t.selfid.as<int>(), r0, r1, box,
+                                                                      t.nodes.as<TcNode>(), t.nodew.as<double4>(),
+                                                                      t.exps.as<double>(), dexps);
+                TC_HIP(hipGetLastError());
+            }
         }
+        top = starts[lt];
+        if (lt < TC_LMAX)
+            last = starts[lt - 1];
     }
-    if (t.ninternal > 0) {
-        const int T = t.level_start[lt];
-        k_e2e<P><<<tiles_of(T, 4), 256, 0, st>>>(t.selfid.as<int>(), parent, pend, T,
-                                                 lt < TC_LMAX ? t.level_start[lt - 1] : T, box, t.nodes.as<TcNode>(),
-                                                 t.nodew.as<double4>(), t.exps.as<double>(), dexps);
+    if (top > 0) {
+        k_e2e<P><<<tiles_of(top, 4), 256, 0, st>>>(t.selfid.as<int>(), parent, pend, info, top, last, box,
+                                                   t.nodes.as<TcNode>(), t.nodew.as<double4>(), t.exps.as<double>(),
+                                                   dexps);
         TC_HIP(hipGetLastError());
     }
     if (fp32) {
         constexpr int per_wave = P + 1 <= 16 ? 4 : (P + 1 <= 32 ? 2 : 1);
-        k_exps32<P><<<tiles_of(t.nnodes, 4 * per_wave), 256, 0, st>>>(t.nodes.as<TcNode>(), t.exps.as<double>(),
-                                                                        t.nnodes, deriv ? 1 : 0, t.exps32.as<float2>());
+        k_exps32<P><<<tiles_of(nn, 4 * per_wave), 256, 0, st>>>(t.nodes.as<TcNode>(), t.exps.as<double>(), info, tmax,
+                                                                 deriv ? 1 : 0, t.exps32.as<float2>());
         TC_HIP(hipGetLastError());
     }
+}
+
+// Most internal nodes that n sources with this leaf capacity can have: the
+// cells of a level are disjoint and hold more than leafcap sources each.
+static long long internal_bound(int n, int leafcap)
+{
+    const long long per_level = (long long)n / ((long long)leafcap + 1);
+    long long t = 0;
+    for (int L = 0; L < TC_LMAX; ++L)
+        t += std::min(per_level, 1ll << (2 * L));
+    return t;
 }
 
 void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v, int n, int leafcap, int order,
@@ -1702,24 +1736,46 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     static_assert(INFO_BYTES <= sizeof(int) * 32 && INFO_BYTES <= TcScratch::PINNED_BYTES, "census record size");
     char *hp = static_cast<char *>(ws.host_pinned());
     TC_HIP(hipMemcpyAsync(hp, info, INFO_BYTES, hipMemcpyDeviceToHost, st));
+    // Where the bound on the node count fits a modest buffer, the rest of the
+    // build is queued behind the census at that bound (its kernels read the count on the
+    // device), and the host waits for the record while they run: queued after the
+    // readback instead, they start one host round trip and launch after the
+    // other with the GPU idle in between.  AHEAD_TIMES
+    const size_t per_node = sizeof(TcNode) + sizeof(double4) + 24 + 16 * (size_t)order * (t.has_deriv ? 2 : 1) +
+                            (fp32 ? 8 * ((size_t)order + 1) : 0);
+    const long long bound = internal_bound(n, leafcap);
+    const bool ahead = !t.nodes.arena && bound <= AHEAD_NODES && (1 + 4 * (size_t)bound) * per_node <= AHEAD_BYTES;
+    if (ahead)
+        TC_HIP(hipEventRecord(ws.census_event(), st));
     if (at_census)
         (*at_census)();  // work queued elsewhere fills the GPU while the host waits
-    TC_HIP(hipStreamSynchronize(st));
-    int hinfo[TC_LMAX + 2];
-    std::memcpy(hinfo, hp, sizeof(hinfo));
-    std::memcpy(t.box, hp + sizeof(int) * INFO_BOX, sizeof(t.box));
-    if (hinfo[TC_LMAX + 1] & 2)
-        throw TcError(-9, "treecode: the source sort did not complete (a radix pass timed out)");
-    if (hinfo[TC_LMAX + 1])
-        throw TcError(-4, "treecode: non-finite source coordinate");
-    const int T = hinfo[TC_LMAX];
-    for (int L = 0; L < TC_LMAX; ++L)
-        t.level_start[L] = hinfo[L];
-    t.level_start[TC_LMAX] = T;
-    t.level_start[TC_LMAX + 1] = T;
-    t.ninternal = T;
-    t.nnodes = 1 + 4 * T;
-    const int nn = t.nnodes;
+    int T = (int)std::min<long long>(bound, INT_MAX / 8), hinfo[TC_LMAX + 2];
+    const int *starts = nullptr;
+    auto census = [&] {
+        if (ahead)
+            TC_HIP(hipEventSynchronize(ws.census_event()));
+        else
+            TC_HIP(hipStreamSynchronize(st));
+        std::memcpy(hinfo, hp, sizeof(hinfo));
+        std::memcpy(t.box, hp + sizeof(int) * INFO_BOX, sizeof(t.box));
+        if (hinfo[TC_LMAX + 1]) {
+            TC_HIP(hipStreamSynchronize(st));  // no kernel of a failed build outlives the call
+            if (hinfo[TC_LMAX + 1] & 2)
+                throw TcError(-9, "treecode: the source sort did not complete (a radix pass timed out)");
+            throw TcError(-4, "treecode: non-finite source coordinate");
+        }
+        for (int L = 0; L <= TC_LMAX; ++L)
+            t.level_start[L] = hinfo[L];
+        t.level_start[TC_LMAX + 1] = hinfo[TC_LMAX];
+        t.ninternal = hinfo[TC_LMAX];
+        t.nnodes = 1 + 4 * t.ninternal;
+    };
+    if (!ahead) {
+        census();
+        T = t.ninternal;
+        starts = t.level_start;
+    }
+    const int nn = 1 + 4 * T;
 
     t.nodes.reserve(sizeof(TcNode) * (size_t)nn);
     t.exps.reserve(sizeof(double) * 2 * (size_t)order * nn);
@@ -1739,31 +1795,29 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     int *lev = reinterpret_cast<int *>(se + nn);
     int2 *cell = reinterpret_cast<int2 *>(lev + ((nn + 1) & ~1));
 
-    if (T > 0) {
-        if (few)
-            k_int_emit<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, ws.istart.as<int>(),
-                                                           ws.ilevel.as<int>());
-        else
-            k_int_emit<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, ws.istart.as<int>(),
-                                                     ws.ilevel.as<int>());
-        const auto nodes_kernel = T <= NODES_WAVE_T ? k_int_nodes<64> : k_int_nodes<16>;
-        nodes_kernel<<<T <= NODES_WAVE_T ? tiles_of(T, 4) : tiles_of(T, 16), 256, 0, st>>>(keys, n, leafcap, ws.istart.as<int>(), ws.ilevel.as<int>(), info,
-                                                    T, t.selfid.as<int>(), pend, child, se, lev, cell);
-    } else {
-        k_topo_leaf<<<1, 1, 0, st>>>(child, n, se, lev, cell);
-    }
+    int *istart = ws.istart.as<int>(), *ilevel = ws.ilevel.as<int>();
+    if (T > 0 && few)
+        k_int_emit<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, T, istart, ilevel);
+    else if (T > 0)
+        k_int_emit<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, T, istart, ilevel);
+    const bool by_wave = T <= NODES_WAVE_T;
+    const auto nodes_kernel = by_wave ? k_int_nodes<64> : k_int_nodes<16>;
+    nodes_kernel<<<std::max(1, tiles_of(T, by_wave ? 4 : 16)), 256, 0, st>>>(
+        keys, n, leafcap, istart, ilevel, info, T, t.selfid.as<int>(), pend, child, se, lev, cell);
     TC_HIP(hipGetLastError());
     if (ev)
         TC_HIP(hipEventRecord(ev[2], st));
 
     switch (order) {
 #define TC_CASE(P) \
-    case P: upward_launch<P>(t, child, se, lev, cell, ws.ilevel.as<int>(), pend, fp32, deriv, st); break;
+    case P: upward_launch<P>(t, child, se, lev, cell, ilevel, pend, fp32, deriv, info, T, starts, st); break;
         TC_ORDERS(TC_CASE)
 #undef TC_CASE
     }
     if (ev)
         TC_HIP(hipEventRecord(ev[3], st));
+    if (ahead)
+        census();
 }
 
 void tc_tree_deriv(TcTree &t, hipStream_t st)

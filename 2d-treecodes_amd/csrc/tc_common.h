@@ -315,8 +315,18 @@ struct TcScratch {
             TC_HIP(hipHostMalloc(&pinned, PINNED_BYTES, hipHostMallocDefault));
         return pinned;
     }
+    hipEvent_t census_ev = nullptr;
+    hipEvent_t census_event()
+    {
+        if (!census_ev)
+            TC_HIP(hipEventCreateWithFlags(&census_ev, hipEventDisableTiming));
+        return census_ev;
+    }
     void release()
     {
+        if (census_ev)
+            (void)hipEventDestroy(census_ev);
+        census_ev = nullptr;
         for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
                           &bbox_part, &ints, &packed, &work, &flist})
             b->release();
@@ -378,6 +388,8 @@ void tc_morton_sort(const double *x, const double *y, const double *v, int n, co
 // records, the topology and the upward pass (the build's phase boundaries).
 // at_census (optional): called once the census readback is queued, before the
 // host waits for it (the caller can queue independent work on another stream).
+// Returns with the build queued on st and the tree's counts known; a non-finite
+// source throws.
 void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v, int n, int leafcap, int order,
                    bool fp32, bool deriv, TcScratch &ws, hipStream_t st, const hipEvent_t *ev = nullptr,
                    const std::function<void()> *at_census = nullptr);
