@@ -16,6 +16,7 @@
 #include "../../include/float/2d-treecodes-potential.h"
 #endif
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -26,6 +27,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 void tc_upload_binomials_eval(hipStream_t st);
@@ -92,6 +94,8 @@ struct tc_context {
     static constexpr int FORCE_RANGES = 4;
     hipEvent_t range_ev[FORCE_RANGES] = {};
     DevBuf io, cnt;
+    double *io_d = nullptr;  // the last host-array call's device copies: doubles,
+    float *io_f = nullptr;   // and for float arrays their float images
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     // build phase boundaries: after the keys, the sorted records, the topology, the upward pass
     hipEvent_t bev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -180,12 +184,11 @@ void par_memcpy(void *dst, const void *src, size_t bytes)
         t.join();
 }
 
-// Host array -> device, ordered on stream st.  Large copies go through the
+// Host memory -> device, ordered on stream st.  Large copies go through the
 // pinned staging buffers of sg in 16 MiB chunks: the CPU fills one buffer
 // while the DMA engine drains the other.
-void copy_in(TcStager &sg, hipStream_t st, const double *h, double *d, long long n)
+void copy_in(TcStager &sg, hipStream_t st, const void *h, void *d, size_t bytes)
 {
-    const size_t bytes = sizeof(double) * (size_t)(n > 0 ? n : 0);
     if (!bytes)
         return;
     if (bytes < STAGE_MIN) {
@@ -204,11 +207,10 @@ void copy_in(TcStager &sg, hipStream_t st, const double *h, double *d, long long
     }
 }
 
-// Device -> host array through the staging buffers of sg on stream st;
+// Device -> host memory through the staging buffers of sg on stream st;
 // returns with the data in h (synchronises st).
-void copy_out(TcStager &sg, hipStream_t st, const double *d, double *h, long long n)
+void copy_out(TcStager &sg, hipStream_t st, const void *d, void *h, size_t bytes)
 {
-    const size_t bytes = sizeof(double) * (size_t)(n > 0 ? n : 0);
     if (bytes < STAGE_MIN) {
         if (bytes)
             TC_HIP(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, st));
@@ -240,33 +242,73 @@ void copy_out(TcStager &sg, hipStream_t st, const double *d, double *h, long lon
     TC_HIP(hipStreamSynchronize(st));
 }
 
-void copy_out(tc_context *c, const double *d, double *h, long long n) { copy_out(c->stg, c->stream, d, h, n); }
+template <class T> size_t arr_bytes(long long n) { return sizeof(T) * (size_t)(n > 0 ? n : 0); }
 
-struct HostIn {
-    const double *h;
+// The device copies of a call's host arrays: n doubles in the io buffer and, for
+// float arrays, as many floats behind them.  Floats cross the link as they are
+// and are converted on the GPU: converted on the host they cost twice the link's bytes
+// and, in freshly allocated double arrays, their page faults (a 200,003-source,
+// 150,001-target solve 843 us, so 547).
+template <class T> double *io_reserve(tc_context *c, size_t n)
+{
+    const size_t nd = (n + 1) & ~size_t(1);
+    c->io.reserve(sizeof(double) * nd + (sizeof(T) < sizeof(double) ? sizeof(T) * n : 0));
+    c->io_d = c->io.as<double>();
+    c->io_f = reinterpret_cast<float *>(c->io_d + nd);
+    return c->io_d;
+}
+inline double *host_image(tc_context *, double *d, double) { return d; }
+inline float *host_image(tc_context *c, double *d, float) { return c->io_f + (d - c->io_d); }
+inline void from_image(tc_context *, double *, size_t, hipStream_t, double) {}
+inline void from_image(tc_context *c, double *d, size_t n, hipStream_t st, float)
+{
+    tc_widen(host_image(c, d, 0.f), d, n, st);
+}
+inline void to_image(tc_context *, double *, size_t, hipStream_t, double) {}
+inline void to_image(tc_context *c, double *d, size_t n, hipStream_t st, float)
+{
+    tc_narrow(d, host_image(c, d, 0.f), n, st);
+}
+
+// One host array -> its n doubles at d in the io buffer, on stream st.
+template <class T> void copy_in(tc_context *c, TcStager &sg, hipStream_t st, const T *h, double *d, long long n)
+{
+    copy_in(sg, st, h, host_image(c, d, T()), arr_bytes<T>(n));
+    if (n > 0)
+        from_image(c, d, (size_t)n, st, T());
+}
+
+// n doubles at d in the io buffer -> host array, on stream st (synchronised).
+template <class T> void copy_out(tc_context *c, TcStager &sg, hipStream_t st, double *d, T *h, long long n)
+{
+    if (n > 0)
+        to_image(c, d, (size_t)n, st, T());
+    copy_out(sg, st, host_image(c, d, T()), h, arr_bytes<T>(n));
+}
+
+template <class T> struct HostIn {
+    const T *h;
     long long n;
 };
-struct HostOut {
-    double *h;
+template <class T> struct HostOut {
+    T *h;
     long long n;
 };
-
-inline size_t arr_bytes(long long n) { return sizeof(double) * (size_t)(n > 0 ? n : 0); }
 
 // Host arrays whose device copies lie back to back from d (in the io buffer).
 // Together up to one staging buffer, they are packed into pinned memory and
 // sent with one DMA (a copy from pageable memory costs a staged transfer of
 // its own); larger sets go array by array.
-void copy_in_all(tc_context *c, double *d, std::initializer_list<HostIn> arrs)
+template <class T> void copy_in_all(tc_context *c, double *d, std::initializer_list<HostIn<T>> arrs)
 {
     size_t total = 0;
-    for (const HostIn &a : arrs)
-        total += arr_bytes(a.n);
+    for (const HostIn<T> &a : arrs)
+        total += arr_bytes<T>(a.n);
     if (!total)
         return;
     if (total > STAGE_BYTES) {
-        for (const HostIn &a : arrs) {
-            copy_in(c->stg, c->stream, a.h, d, a.n);
+        for (const HostIn<T> &a : arrs) {
+            copy_in(c, c->stg, c->stream, a.h, d, a.n);
             d += a.n > 0 ? a.n : 0;
         }
         return;
@@ -274,26 +316,27 @@ void copy_in_all(tc_context *c, double *d, std::initializer_list<HostIn> arrs)
     c->stg.ready();
     c->stg.wait(0);
     char *s = static_cast<char *>(c->stg.buf[0]);
-    for (const HostIn &a : arrs) {
-        par_memcpy(s, a.h, arr_bytes(a.n));
-        s += arr_bytes(a.n);
+    for (const HostIn<T> &a : arrs) {
+        par_memcpy(s, a.h, arr_bytes<T>(a.n));
+        s += arr_bytes<T>(a.n);
     }
-    TC_HIP(hipMemcpyAsync(d, c->stg.buf[0], total, hipMemcpyHostToDevice, c->stream));
+    TC_HIP(hipMemcpyAsync(host_image(c, d, T()), c->stg.buf[0], total, hipMemcpyHostToDevice, c->stream));
     TC_HIP(hipEventRecord(c->stg.ev[0], c->stream));
     c->stg.busy[0] = true;
+    from_image(c, d, total / sizeof(T), c->stream, T());
 }
 
-// Device block from d (arrays back to back) -> host arrays; returns with the
-// data in place (synchronises the stream).  Up to one staging buffer in total
-// it is one DMA into pinned memory.
-void copy_out_all(tc_context *c, const double *d, std::initializer_list<HostOut> arrs)
+// Device block from d (arrays back to back, in the io buffer) -> host arrays;
+// returns with the data in place (synchronises the stream).  Up to one staging
+// buffer in total it is one DMA into pinned memory.
+template <class T> void copy_out_all(tc_context *c, double *d, std::initializer_list<HostOut<T>> arrs)
 {
     size_t total = 0;
-    for (const HostOut &a : arrs)
-        total += arr_bytes(a.n);
+    for (const HostOut<T> &a : arrs)
+        total += arr_bytes<T>(a.n);
     if (total > STAGE_BYTES || !total) {
-        for (const HostOut &a : arrs) {
-            copy_out(c, d, a.h, a.n);
+        for (const HostOut<T> &a : arrs) {
+            copy_out(c, c->stg, c->stream, d, a.h, a.n);
             d += a.n > 0 ? a.n : 0;
         }
         TC_HIP(hipStreamSynchronize(c->stream));
@@ -301,12 +344,13 @@ void copy_out_all(tc_context *c, const double *d, std::initializer_list<HostOut>
     }
     c->stg.ready();
     c->stg.wait(0);
-    TC_HIP(hipMemcpyAsync(c->stg.buf[0], d, total, hipMemcpyDeviceToHost, c->stream));
+    to_image(c, d, total / sizeof(T), c->stream, T());
+    TC_HIP(hipMemcpyAsync(c->stg.buf[0], host_image(c, d, T()), total, hipMemcpyDeviceToHost, c->stream));
     TC_HIP(hipStreamSynchronize(c->stream));
     const char *s = static_cast<const char *>(c->stg.buf[0]);
-    for (const HostOut &a : arrs) {
-        par_memcpy(a.h, s, arr_bytes(a.n));
-        s += arr_bytes(a.n);
+    for (const HostOut<T> &a : arrs) {
+        par_memcpy(a.h, s, arr_bytes<T>(a.n));
+        s += arr_bytes<T>(a.n);
     }
 }
 
@@ -428,10 +472,20 @@ void eval_potential_ext(tc_context *c, const TcTree &t, const ExtTree &ext, doub
     record(c, 3);
 }
 
-int run_potential(tc_context *ctx, double theta, const double *xs, const double *ys, const double *vs, int n,
-                  const double *xt, const double *yt, int m, double *out, int device_ptrs, bool rebuild,
-                  const ExtTree &ext = ExtTree())
+inline const double *dev_ptr(const double *p) { return p; }
+inline double *dev_ptr(double *p) { return p; }
+inline const double *dev_ptr(const float *) { return nullptr; }
+inline double *dev_ptr(float *) { return nullptr; }
+
+// T: element type of host arrays; device arrays (device_ptrs) are double.
+template <class T>
+int run_potential(tc_context *ctx, double theta, const T *xs, const T *ys, const T *vs, int n, const T *xt,
+                  const T *yt, int m, T *out, int device_ptrs, bool rebuild, const ExtTree &ext = ExtTree())
 {
+    if (device_ptrs && !std::is_same<T, double>::value) {
+        set_error("treecode: device arrays are double");
+        return -3;
+    }
     return guarded(ctx, [&] {
         tc_context *c = ctx;
         c->ev_valid = false;
@@ -441,7 +495,7 @@ int run_potential(tc_context *ctx, double theta, const double *xs, const double 
             if (device_ptrs)
                 TC_HIP(hipMemsetAsync(out, 0, sizeof(double) * (size_t)m, c->stream));
             else
-                std::memset(out, 0, sizeof(double) * (size_t)m);
+                std::memset(out, 0, sizeof(T) * (size_t)m);
             c->tree_kind = TC_KIND_NONE;
             return;
         }
@@ -451,27 +505,26 @@ int run_potential(tc_context *ctx, double theta, const double *xs, const double 
         }
         if (!rebuild && ext.tree && ext.ready)
             TC_HIP(hipStreamWaitEvent(c->stream, ext.ready, 0));
-        const double *dxs = xs, *dys = ys, *dvs = vs, *dxt = xt, *dyt = yt;
-        double *dout = out;
+        const double *dxs = dev_ptr(xs), *dys = dev_ptr(ys), *dvs = dev_ptr(vs), *dxt = dev_ptr(xt), *dyt = dev_ptr(yt);
+        double *dout = dev_ptr(out);
         // host target arrays of 4 MiB or more (512 Ki targets) are uploaded by a
         // helper thread, through their own staging buffers on the second
         // stream, while the source tree builds (the build waits on the host only
         // for its census): the upload then overlaps the build instead of
         // preceding it
-        const bool overlap = !device_ptrs && rebuild && arr_bytes(m) >= STAGE_BYTES / 4;
+        const bool overlap = !device_ptrs && rebuild && arr_bytes<T>(m) >= STAGE_BYTES / 4;
         if (!device_ptrs) {
             const size_t ns = rebuild ? (size_t)n : 0;
-            c->io.reserve(sizeof(double) * (3 * ns + 3 * (size_t)m));
-            double *base = c->io.as<double>();
+            double *base = io_reserve<T>(c, 3 * ns + 3 * (size_t)m);
             double *bxs = base, *bys = base + ns, *bvs = base + 2 * ns;
             double *bxt = base + 3 * ns, *byt = bxt + m;
             dout = byt + m;
             if (overlap)
-                copy_in_all(c, bxs, {{xs, n}, {ys, n}, {vs, n}});
+                copy_in_all<T>(c, bxs, {{xs, n}, {ys, n}, {vs, n}});
             else if (rebuild)
-                copy_in_all(c, bxs, {{xs, n}, {ys, n}, {vs, n}, {xt, m}, {yt, m}});
+                copy_in_all<T>(c, bxs, {{xs, n}, {ys, n}, {vs, n}, {xt, m}, {yt, m}});
             else
-                copy_in_all(c, bxt, {{xt, m}, {yt, m}});
+                copy_in_all<T>(c, bxt, {{xt, m}, {yt, m}});
             dxs = bxs; dys = bys; dvs = bvs; dxt = bxt; dyt = byt;
         }
         unsigned long long *cnt = prepare_counters(c);
@@ -486,8 +539,8 @@ int run_potential(tc_context *ctx, double theta, const double *xs, const double 
                 up = std::thread([&] {
                     try {
                         TC_HIP(hipSetDevice(c->device));
-                        copy_in(c->tstg, c->tstream, xt, const_cast<double *>(dxt), m);
-                        copy_in(c->tstg, c->tstream, yt, const_cast<double *>(dyt), m);
+                        copy_in(c, c->tstg, c->tstream, xt, const_cast<double *>(dxt), m);
+                        copy_in(c, c->tstg, c->tstream, yt, const_cast<double *>(dyt), m);
                         tc_sort_targets(dxt, dyt, m, c->tws, c->tstream);
                     } catch (...) {
                         up_err = std::current_exception();
@@ -553,7 +606,7 @@ int run_potential(tc_context *ctx, double theta, const double *xs, const double 
             uint32_t *bad = static_cast<uint32_t *>(c->tws.host_pinned());
             TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->tws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
                                   c->stream));
-            copy_out_all(c, dout, {{out, m}});
+            copy_out_all<T>(c, dout, {{out, m}});
             if (*bad & 2)
                 throw TcError(-9, "treecode_potential: the target sort did not complete (a radix pass timed out)");
             if (*bad)
@@ -639,10 +692,14 @@ int run_potential_noalloc(tc_context *ctx, double theta, const double *xs, const
 }
 #endif
 
-int run_force(tc_context *ctx, double theta, const double *xs, const double *ys, const double *vs, int n,
-              const double *x0s, const double *y0s, const double *hs, int nb, double *xr, double *yr,
-              int device_ptrs, bool rebuild, const ExtTree &ext = ExtTree())
+template <class T>
+int run_force(tc_context *ctx, double theta, const T *xs, const T *ys, const T *vs, int n, const T *x0s, const T *y0s,
+              const T *hs, int nb, T *xr, T *yr, int device_ptrs, bool rebuild, const ExtTree &ext = ExtTree())
 {
+    if (device_ptrs && !std::is_same<T, double>::value) {
+        set_error("treecode: device arrays are double");
+        return -3;
+    }
     return guarded(ctx, [&] {
         tc_context *c = ctx;
         c->ev_valid = false;
@@ -654,8 +711,8 @@ int run_force(tc_context *ctx, double theta, const double *xs, const double *ys,
                 TC_HIP(hipMemsetAsync(xr, 0, sizeof(double) * nt, c->stream));
                 TC_HIP(hipMemsetAsync(yr, 0, sizeof(double) * nt, c->stream));
             } else {
-                std::memset(xr, 0, sizeof(double) * nt);
-                std::memset(yr, 0, sizeof(double) * nt);
+                std::memset(xr, 0, sizeof(T) * nt);
+                std::memset(yr, 0, sizeof(T) * nt);
             }
             c->tree_kind = TC_KIND_NONE;
             return;
@@ -666,23 +723,23 @@ int run_force(tc_context *ctx, double theta, const double *xs, const double *ys,
         }
         if (!rebuild && ext.tree && ext.ready)
             TC_HIP(hipStreamWaitEvent(c->stream, ext.ready, 0));
-        const double *dxs = xs, *dys = ys, *dvs = vs, *dx0 = x0s, *dy0 = y0s, *dh = hs;
-        double *dxr = xr, *dyr = yr;
+        const double *dxs = dev_ptr(xs), *dys = dev_ptr(ys), *dvs = dev_ptr(vs), *dx0 = dev_ptr(x0s),
+                     *dy0 = dev_ptr(y0s), *dh = dev_ptr(hs);
+        double *dxr = dev_ptr(xr), *dyr = dev_ptr(yr);
         if (!device_ptrs) {
             for (int i = 0; i < nb; ++i)
                 if (!std::isfinite(x0s[i]) || !std::isfinite(y0s[i]) || !std::isfinite(hs[i]))
                     throw TcError(-4, "treecode_force_mrag: non-finite block origin or spacing");
             const size_t ns = rebuild ? (size_t)n : 0;
-            c->io.reserve(sizeof(double) * (3 * ns + 3 * (size_t)nb + 2 * nt));
-            double *base = c->io.as<double>();
+            double *base = io_reserve<T>(c, 3 * ns + 3 * (size_t)nb + 2 * nt);
             double *bxs = base, *bys = base + ns, *bvs = base + 2 * ns;
             double *bx0 = base + 3 * ns, *by0 = bx0 + nb, *bh = by0 + nb;
             dxr = bh + nb;
             dyr = dxr + nt;
             if (rebuild)
-                copy_in_all(c, bxs, {{xs, n}, {ys, n}, {vs, n}, {x0s, nb}, {y0s, nb}, {hs, nb}});
+                copy_in_all<T>(c, bxs, {{xs, n}, {ys, n}, {vs, n}, {x0s, nb}, {y0s, nb}, {hs, nb}});
             else
-                copy_in_all(c, bx0, {{x0s, nb}, {y0s, nb}, {hs, nb}});
+                copy_in_all<T>(c, bx0, {{x0s, nb}, {y0s, nb}, {hs, nb}});
             dxs = bxs; dys = bys; dvs = bvs; dx0 = bx0; dy0 = by0; dh = bh;
         }
         unsigned long long *cnt = prepare_counters(c);
@@ -711,7 +768,7 @@ int run_force(tc_context *ctx, double theta, const double *xs, const double *ys,
             c->ev_valid = c->profile;
             c->eval_has_tsort = false;
             if (!device_ptrs)
-                copy_out_all(c, dxr, {{xr, (long long)nt}, {yr, (long long)nt}});
+                copy_out_all<T>(c, dxr, {{xr, (long long)nt}, {yr, (long long)nt}});
             return;
         }
         const int pool = c->force_chunks > 0 ? c->force_chunks : std::max(4096, std::min(nb * 16, 1 << 20) / 4);
@@ -730,8 +787,8 @@ int run_force(tc_context *ctx, double theta, const double *xs, const double *ys,
             const long long len = (long long)std::min(per, nb - b0) * 1024;
             const size_t o = (size_t)b0 * 1024;
             TC_HIP(hipStreamWaitEvent(c->tstream, c->range_ev[k], 0));
-            copy_out(c->tstg, c->tstream, dxr + o, xr + o, len);
-            copy_out(c->tstg, c->tstream, dyr + o, yr + o, len);
+            copy_out(c, c->tstg, c->tstream, dxr + o, xr + o, len);
+            copy_out(c, c->tstg, c->tstream, dyr + o, yr + o, len);
         }
     });
 }
@@ -758,27 +815,44 @@ int run_force_targets(tc_context *ctx, double theta, const double *xs, const dou
         const double *dxs = xs, *dys = ys, *dvs = vs, *dxt = xt, *dyt = yt;
         double *dxr = xr, *dyr = yr;
         if (!device_ptrs) {
-            c->io.reserve(sizeof(double) * (3 * (size_t)n + 4 * (size_t)m));
-            double *base = c->io.as<double>();
+            double *base = io_reserve<double>(c, 3 * (size_t)n + 4 * (size_t)m);
             double *bxs = base, *bys = base + n, *bvs = base + 2 * (size_t)n;
             double *bxt = base + 3 * (size_t)n, *byt = bxt + m;
             dxr = byt + m;
             dyr = dxr + m;
-            copy_in_all(c, bxs, {{xs, n}, {ys, n}, {vs, n}, {xt, m}, {yt, m}});
+            copy_in_all<double>(c, bxs, {{xs, n}, {ys, n}, {vs, n}, {xt, m}, {yt, m}});
             dxs = bxs; dys = bys; dvs = bvs; dxt = bxt; dyt = byt;
         }
         unsigned long long *cnt = prepare_counters(c);
         record(c, 0);
-        build(c, dxs, dys, dvs, n, TC_KIND_FORCE, ExtTree());
+        // the targets are sorted on the second stream beside the source build (see run_potential)
+        TC_HIP(hipEventRecord(c->fork_ev, c->stream));
+        TC_HIP(hipStreamWaitEvent(c->tstream, c->fork_ev, 0));
+        const std::function<void()> tsort = [&] {
+            try {
+                tc_sort_targets(dxt, dyt, m, c->tws, c->tstream);
+            } catch (...) {
+                (void)hipEventRecord(c->join_ev, c->tstream);
+                throw;
+            }
+            TC_HIP(hipEventRecord(c->join_ev, c->tstream));
+        };
+        try {
+            build(c, dxs, dys, dvs, n, TC_KIND_FORCE, ExtTree(), &tsort);
+        } catch (...) {
+            (void)hipStreamWaitEvent(c->stream, c->join_ev, 0);
+            throw;
+        }
         record(c, 1);
-        tc_eval_force_targets(c->tree, theta, dxt, dyt, m, dxr, dyr, c->precision, cnt, c->ws, c->stream,
+        TC_HIP(hipStreamWaitEvent(c->stream, c->join_ev, 0));
+        tc_eval_force_targets(c->tree, theta, dxt, dyt, m, dxr, dyr, c->precision, cnt, c->tws, c->stream,
                               c->profile ? c->ev[2] : nullptr, c->profile ? c->ev[3] : nullptr);
         c->ev_valid = c->profile;
         if (!device_ptrs) {
-            uint32_t *bad = static_cast<uint32_t *>(c->ws.host_pinned());
-            TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->ws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
+            uint32_t *bad = static_cast<uint32_t *>(c->tws.host_pinned());
+            TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->tws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
                                   c->stream));
-            copy_out_all(c, dxr, {{xr, m}, {yr, m}});
+            copy_out_all<double>(c, dxr, {{xr, m}, {yr, m}});
             if (*bad & 2)
                 throw TcError(-9, "treecode_force: the target sort did not complete (a radix pass timed out)");
             if (*bad)
@@ -806,14 +880,6 @@ tc_context *default_context_f32()
     return g_default_f32;
 }
 
-std::vector<double> widen(const float *p, size_t n)
-{
-    std::vector<double> v(n);
-    for (size_t i = 0; i < n; ++i)
-        v[i] = (double)p[i];
-    return v;
-}
-
 void report_dropin_failure(const char *fn)
 {
     static bool printed = false;
@@ -824,25 +890,22 @@ void report_dropin_failure(const char *fn)
 }
 
 // The float drop-in pair (the reference's real=float build, libraries.Makefile:13):
-// float arrays are widened, solved on the FP32-bulk path of a second default
-// context, and narrowed back.
+// float arrays are widened on the GPU, solved on the FP32-bulk path of a second
+// default context, and narrowed back.
 void dropin_potential_f32(const char *fn, const float theta, const float *const xsources,
                           const float *const ysources, const float *const sourcevalues, const int nsources,
                           const float *const xtargets, const float *const ytargets, const int ntargets,
                           float *const targetvalues)
 {
     std::lock_guard<std::mutex> lk(g_default_mu);
-    const size_t n = nsources > 0 ? (size_t)nsources : 0, m = ntargets > 0 ? (size_t)ntargets : 0;
-    std::vector<double> xs = widen(xsources, n), ys = widen(ysources, n), vs = widen(sourcevalues, n);
-    std::vector<double> xt = widen(xtargets, m), yt = widen(ytargets, m), out(m);
     tc_context *c = default_context_f32();
-    int rc = c ? tc_potential(c, (double)theta, xs.data(), ys.data(), vs.data(), nsources, xt.data(), yt.data(),
-                              ntargets, out.data(), 0)
-               : -1;
-    if (rc)
+    const int rc = c ? run_potential(c, (double)theta, xsources, ysources, sourcevalues, nsources, xtargets, ytargets,
+                                     ntargets, targetvalues, 0, true)
+                     : -1;
+    if (rc) {
         report_dropin_failure(fn);
-    for (size_t i = 0; i < m; ++i)
-        targetvalues[i] = rc ? std::numeric_limits<float>::quiet_NaN() : (float)out[i];
+        std::fill(targetvalues, targetvalues + std::max(0, ntargets), std::numeric_limits<float>::quiet_NaN());
+    }
 }
 
 void dropin_force_f32(const char *fn, const float theta, const float *const xsources, const float *const ysources,
@@ -851,19 +914,15 @@ void dropin_force_f32(const char *fn, const float theta, const float *const xsou
                       float *const yresults)
 {
     std::lock_guard<std::mutex> lk(g_default_mu);
-    const size_t n = nsources > 0 ? (size_t)nsources : 0, nb = nblocks > 0 ? (size_t)nblocks : 0;
-    std::vector<double> xs = widen(xsources, n), ys = widen(ysources, n), vs = widen(sourcevalues, n);
-    std::vector<double> bx = widen(x0s, nb), by = widen(y0s, nb), bh = widen(hs, nb);
-    std::vector<double> xr(nb * 1024), yr(nb * 1024);
     tc_context *c = default_context_f32();
-    int rc = c ? tc_force_mrag(c, (double)theta, xs.data(), ys.data(), vs.data(), nsources, bx.data(), by.data(),
-                               bh.data(), nblocks, xr.data(), yr.data(), 0)
-               : -1;
-    if (rc)
+    const int rc = c ? run_force(c, (double)theta, xsources, ysources, sourcevalues, nsources, x0s, y0s, hs, nblocks,
+                                 xresults, yresults, 0, true)
+                     : -1;
+    if (rc) {
         report_dropin_failure(fn);
-    for (size_t i = 0; i < nb * 1024; ++i) {
-        xresults[i] = rc ? std::numeric_limits<float>::quiet_NaN() : (float)xr[i];
-        yresults[i] = rc ? std::numeric_limits<float>::quiet_NaN() : (float)yr[i];
+        const size_t nt = 1024 * (size_t)std::max(0, nblocks);
+        std::fill(xresults, xresults + nt, std::numeric_limits<float>::quiet_NaN());
+        std::fill(yresults, yresults + nt, std::numeric_limits<float>::quiet_NaN());
     }
 }
 
@@ -1075,7 +1134,7 @@ TC_API int tc_potential(tc_context *c, double theta, const double *xs, const dou
 TC_API int tc_potential_resident(tc_context *c, double theta, const double *xt, const double *yt, int m,
                                  double *out, int device_ptrs)
 {
-    return run_potential(c, theta, nullptr, nullptr, nullptr, 0, xt, yt, m, out, device_ptrs, false);
+    return run_potential<double>(c, theta, nullptr, nullptr, nullptr, 0, xt, yt, m, out, device_ptrs, false);
 }
 
 TC_API int tc_potential_batch_resident(tc_context *const *ctxs, int k, const double *theta,
@@ -1170,7 +1229,7 @@ TC_API int tc_force_mrag(tc_context *c, double theta, const double *xs, const do
 TC_API int tc_force_mrag_resident(tc_context *c, double theta, const double *x0s, const double *y0s,
                                   const double *hs, int nblocks, double *xr, double *yr, int device_ptrs)
 {
-    return run_force(c, theta, nullptr, nullptr, nullptr, 0, x0s, y0s, hs, nblocks, xr, yr, device_ptrs, false);
+    return run_force<double>(c, theta, nullptr, nullptr, nullptr, 0, x0s, y0s, hs, nblocks, xr, yr, device_ptrs, false);
 }
 
 TC_API int tc_force_targets(tc_context *c, double theta, const double *xs, const double *ys, const double *vs,

@@ -1740,7 +1740,8 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     // build is queued behind the census at that bound (its kernels read the count on the
     // device), and the host waits for the record while they run: queued after the
     // readback instead, they start one host round trip and launch after the
-    // other with the GPU idle in between.  AHEAD_TIMES
+    // other with the GPU idle in between. 4 to 5% of a 0.3 to 0.5 ms
+    // solve (65,536-point FP64 potential 288 -> 278 us).
     const size_t per_node = sizeof(TcNode) + sizeof(double4) + 24 + 16 * (size_t)order * (t.has_deriv ? 2 : 1) +
                             (fp32 ? 8 * ((size_t)order + 1) : 0);
     const long long bound = internal_bound(n, leafcap);

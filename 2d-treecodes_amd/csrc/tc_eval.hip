@@ -1946,6 +1946,13 @@ __global__ __launch_bounds__(256) void k_direct(const double *__restrict__ xs, c
 
 // Plain 16-byte-per-thread copy: the reference kernel for scaling HBM counters
 // (FETCH_SIZE / WRITE_SIZE of a copy of known size).
+template <class S, class D>
+__global__ __launch_bounds__(256) void k_convert(const S *__restrict__ src, D *__restrict__ dst, size_t n)
+{
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
+        dst[i] = (D)src[i];
+}
+
 __global__ __launch_bounds__(256) void k_copy16(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n)
 {
     for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
@@ -2158,6 +2165,18 @@ void tc_upload_binomials_eval(hipStream_t st)
     TC_HIP(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_logtab), lt.data(), sizeof(double2) * lt.size(), 0,
                                   hipMemcpyHostToDevice, st));
     TC_HIP(hipStreamSynchronize(st));
+}
+
+void tc_widen(const float *src, double *dst, size_t n, hipStream_t st)
+{
+    k_convert<<<(int)std::min<size_t>((n + 255) / 256, 4096), 256, 0, st>>>(src, dst, n);
+    TC_HIP(hipGetLastError());
+}
+
+void tc_narrow(const double *src, float *dst, size_t n, hipStream_t st)
+{
+    k_convert<<<(int)std::min<size_t>((n + 255) / 256, 4096), 256, 0, st>>>(src, dst, n);
+    TC_HIP(hipGetLastError());
 }
 
 void tc_copy16(const void *src, void *dst, size_t bytes, hipStream_t st)
@@ -2428,7 +2447,6 @@ void tc_eval_force_targets(const TcTree &t, double theta, const double *xt, cons
         return;
     if (precision == 1 && !t.has_fp32)
         throw TcError(-3, "tc_eval_force_targets: tree was built without FP32 mirrors");
-    tc_sort_targets(xt, yt, m, ws, st);
     const double th2 = theta * theta;
     const uint32_t *tperm = ws.tperm.as<uint32_t>();
     if (ev0)

@@ -120,3 +120,28 @@ def test_fp64_force_on_fp32_tree(pkg, wl):
         got = ctx.force_resident(0.5, x0s, y0s, hs)
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     ctx.close()
+
+
+# float arrays are converted on the GPU: packed (one transfer), array by array, and with targets
+# uploaded beside the build; forces in one piece and in ranges
+@pytest.mark.parametrize("n,m", [(5, 3), (1001, 777), (1 << 20, 70001), (100001, 1 << 20)])
+def test_float_arrays_equal_double_arrays(pkg, wl, n, m):
+    st = wl.Stream(n + m)
+    a = [st.uniform(n).astype(np.float32), st.uniform(n).astype(np.float32), st.uniform(n, -1, 1).astype(np.float32),
+         st.uniform(m).astype(np.float32), st.uniform(m).astype(np.float32)]
+    out = pkg.treecode_potential_float(0.5, *a)
+    ctx = pkg.Context(precision=pkg.FP32)
+    ref = ctx.potential(float(np.float32(0.5)), *[v.astype(np.float64) for v in a])
+    assert out.dtype == np.float32 and np.array_equal(out, ref.astype(np.float32))
+    ctx.close()
+
+
+@pytest.mark.parametrize("nb", [1, 33, 2050])
+def test_float_forces_equal_double_forces(pkg, wl, nb):
+    xs, ys, vs, x0s, y0s, hs = wl.gaussian4_force(20000, seed=nb)
+    a = [v.astype(np.float32) for v in (xs, ys, vs, x0s[:nb], y0s[:nb], hs[:nb])]
+    fx, fy = pkg.treecode_force_mrag_float(0.5, *a)
+    ctx = pkg.Context(precision=pkg.FP32)
+    rx, ry = ctx.force(0.5, *[v.astype(np.float64) for v in a])
+    assert np.array_equal(fx, rx.astype(np.float32)) and np.array_equal(fy, ry.astype(np.float32))
+    ctx.close()
