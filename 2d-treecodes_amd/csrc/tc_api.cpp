@@ -396,7 +396,7 @@ struct ExtTree {
 // at_census (optional): work to queue once the build's census readback is
 // queued (see tc_build_tree).
 void build(tc_context *c, const double *xs, const double *ys, const double *vs, int n, int kind, const ExtTree &ext,
-           const std::function<void()> *at_census = nullptr)
+           const std::function<void()> *at_census = nullptr, TcJointTargets *targets = nullptr)
 {
     if (ext.tree) {
         const int order = kind == TC_KIND_POTENTIAL ? c->pot_order : c->force_order;
@@ -404,7 +404,7 @@ void build(tc_context *c, const double *xs, const double *ys, const double *vs, 
         ext.tree->nnodes = 0;
         ext.tree->has_fp32 = false;
         tc_build_tree(*ext.tree, xs, ys, vs, n, leaf, order, c->precision == 1, kind == TC_KIND_FORCE, c->ws,
-                      c->stream, nullptr, at_census);
+                      c->stream, nullptr, at_census, targets);
         if (ext.ready)
             TC_HIP(hipEventRecord(ext.ready, c->stream));
         return;
@@ -420,7 +420,7 @@ void build(tc_context *c, const double *xs, const double *ys, const double *vs, 
     c->tree.has_fp32 = false;
     c->bev_valid = false;
     tc_build_tree(c->tree, xs, ys, vs, n, leaf, order, c->precision == 1, kind == TC_KIND_FORCE, c->ws, c->stream,
-                  c->profile ? c->bev : nullptr, at_census);
+                  c->profile ? c->bev : nullptr, at_census, targets);
     c->bev_valid = c->profile;
     c->tree_kind = kind;
     c->tree_precision = c->precision;
@@ -528,7 +528,18 @@ int run_potential(tc_context *ctx, double theta, const T *xs, const T *ys, const
             dxs = bxs; dys = bys; dvs = bvs; dxt = bxt; dyt = byt;
         }
         unsigned long long *cnt = prepare_counters(c);
-        if (rebuild) {
+        // small and middling targets are sorted by the source sort's launches
+        const bool joint = rebuild && !overlap && tc_sorts_jointly(n, m);
+        TcJointTargets jt{dxt, dyt, m, &c->tws, 0};
+        if (joint) {
+            record(c, 0);
+            build(c, dxs, dys, dvs, n, TC_KIND_POTENTIAL, ext, nullptr, &jt);
+            record(c, 1);
+            if (ext.tree)
+                eval_potential_ext(c, *ext.tree, ext, theta, dxt, dyt, m, dout, cnt, false);
+            else
+                eval_potential(c, theta, dxt, dyt, m, dout, cnt, false);
+        } else if (rebuild) {
             // the target sort (one workgroup for small m) runs beside the
             // source build; the evaluation waits for both
             TC_HIP(hipEventRecord(c->fork_ev, c->stream));
@@ -603,9 +614,10 @@ int run_potential(tc_context *ctx, double theta, const T *xs, const T *ys, const
         c->eval_has_tsort = true;
         if (!device_ptrs) {
             // the target sort's bounding-box pass flags non-finite coordinates
-            uint32_t *bad = static_cast<uint32_t *>(c->tws.host_pinned());
-            TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->tws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                  c->stream));
+            uint32_t *bad = joint ? &jt.bad : static_cast<uint32_t *>(c->tws.host_pinned());
+            if (!joint)
+                TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->tws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                      c->stream));
             copy_out_all<T>(c, dout, {{out, m}});
             if (*bad & 2)
                 throw TcError(-9, "treecode_potential: the target sort did not complete (a radix pass timed out)");
@@ -825,33 +837,41 @@ int run_force_targets(tc_context *ctx, double theta, const double *xs, const dou
         }
         unsigned long long *cnt = prepare_counters(c);
         record(c, 0);
-        // the targets are sorted on the second stream beside the source build (see run_potential)
-        TC_HIP(hipEventRecord(c->fork_ev, c->stream));
-        TC_HIP(hipStreamWaitEvent(c->tstream, c->fork_ev, 0));
-        const std::function<void()> tsort = [&] {
+        // the targets are sorted by the source sort's launches or beside the build (see run_potential)
+        const bool joint = tc_sorts_jointly(n, m);
+        TcJointTargets jt{dxt, dyt, m, &c->tws, 0};
+        if (joint) {
+            build(c, dxs, dys, dvs, n, TC_KIND_FORCE, ExtTree(), nullptr, &jt);
+            record(c, 1);
+        } else {
+            TC_HIP(hipEventRecord(c->fork_ev, c->stream));
+            TC_HIP(hipStreamWaitEvent(c->tstream, c->fork_ev, 0));
+            const std::function<void()> tsort = [&] {
+                try {
+                    tc_sort_targets(dxt, dyt, m, c->tws, c->tstream);
+                } catch (...) {
+                    (void)hipEventRecord(c->join_ev, c->tstream);
+                    throw;
+                }
+                TC_HIP(hipEventRecord(c->join_ev, c->tstream));
+            };
             try {
-                tc_sort_targets(dxt, dyt, m, c->tws, c->tstream);
+                build(c, dxs, dys, dvs, n, TC_KIND_FORCE, ExtTree(), &tsort);
             } catch (...) {
-                (void)hipEventRecord(c->join_ev, c->tstream);
+                (void)hipStreamWaitEvent(c->stream, c->join_ev, 0);
                 throw;
             }
-            TC_HIP(hipEventRecord(c->join_ev, c->tstream));
-        };
-        try {
-            build(c, dxs, dys, dvs, n, TC_KIND_FORCE, ExtTree(), &tsort);
-        } catch (...) {
-            (void)hipStreamWaitEvent(c->stream, c->join_ev, 0);
-            throw;
+            record(c, 1);
+            TC_HIP(hipStreamWaitEvent(c->stream, c->join_ev, 0));
         }
-        record(c, 1);
-        TC_HIP(hipStreamWaitEvent(c->stream, c->join_ev, 0));
         tc_eval_force_targets(c->tree, theta, dxt, dyt, m, dxr, dyr, c->precision, cnt, c->tws, c->stream,
                               c->profile ? c->ev[2] : nullptr, c->profile ? c->ev[3] : nullptr);
         c->ev_valid = c->profile;
         if (!device_ptrs) {
-            uint32_t *bad = static_cast<uint32_t *>(c->tws.host_pinned());
-            TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->tws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                  c->stream));
+            uint32_t *bad = joint ? &jt.bad : static_cast<uint32_t *>(c->tws.host_pinned());
+            if (!joint)
+                TC_HIP(hipMemcpyAsync(bad, tc_targets_bad_flag(c->tws, m), sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                      c->stream));
             copy_out_all<double>(c, dxr, {{xr, m}, {yr, m}});
             if (*bad & 2)
                 throw TcError(-9, "treecode_force: the target sort did not complete (a radix pass timed out)");
@@ -960,7 +980,7 @@ size_t tc_srv_context_bytes(tc_context *c)
     size_t b = tc_tree_bytes(c->tree) + c->io.cap + c->cnt.cap;
     for (const TcScratch *w : {&c->ws, &c->tws})
         for (const DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->istart, &w->ilevel, &w->info,
-                                &w->tkeys, &w->tperm, &w->tsorted, &w->bbox_part, &w->ints, &w->packed, &w->work,
+                                &w->tkeys, &w->tperm, &w->bbox_part, &w->ints, &w->packed, &w->work,
                                 &w->flist})
             b += d->cap;
     return b;
@@ -976,7 +996,7 @@ void tc_srv_context_trim(tc_context *c)
     c->io.release();
     for (TcScratch *w : {&c->ws, &c->tws})
         for (DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->istart, &w->ilevel, &w->info,
-                          &w->tkeys, &w->tperm, &w->tsorted, &w->bbox_part, &w->ints, &w->packed, &w->work,
+                          &w->tkeys, &w->tperm, &w->bbox_part, &w->ints, &w->packed, &w->work,
                           &w->flist})
             d->release();
 }
@@ -1406,7 +1426,7 @@ TC_API int tc_morton_sort_device(tc_context *c, const double *x, const double *y
     return guarded(c, [&] {
         if (n <= 0)
             throw TcError(-3, "tc_morton_sort_device: n must be positive");
-        tc_sort_points(x, y, nullptr, n, box, keys, perm, nullptr, c->ws, c->stream, false);
+        tc_morton_sort(x, y, n, box, keys, perm, c->ws, c->stream);
     });
 }
 

@@ -75,21 +75,43 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, size_t n)
         p[i] = v;
 }
 
+// ------------------------------------------------------------------ sorts of one or two point sets
+// One point set of a sort and its device memory.  A solve's sources and targets
+// are sorted by the same launches where both are small or middling (a launch
+// costs the host about 4 us, a pass of few tiles fills a fraction of the CUs):
+// workgroups [0, first set's) take the first set, the rest the second.
+struct SortSet {
+    const double *x, *y, *v;  // v: sources (Morton keys, records packed); else targets (Hilbert keys)
+    double *box;              // {xmin, ymin, ext, scale} out
+    uint32_t *keys, *perm;    // out
+    uint32_t *k2, *v2;        // scratch of n words each
+    double4 *packed;          // source records in input order
+    double4 *part;            // bounding-box partials
+    uint32_t *bad, *pbad;     // non-finite flag (bit 1: a pass gave up); per-workgroup flags
+    uint32_t *lb;             // digit totals, tickets, published counts (lb_words)
+    int n, np, ntiles, kgrid, kstep;
+};
+struct SortSets {
+    SortSet s[2];
+};
+
 // ------------------------------------------------------------------ bbox
 // sort-sources.cpp:44-82 with upward-common.ispc:126-150's accumulators:
-// min starts at 1e13, max at 0.  Non-finite coordinates are ORed into *bad
-// (cleared before), or with pbad recorded per workgroup in pbad[blockIdx.x].
-// Also zeroes zero[0 .. nzero) (the one-launch radix passes' counters, used
-// after this kernel).
-__global__ __launch_bounds__(256) void k_bbox_partial(const double *x, const double *y, int n, double4 *part,
-                                                       uint32_t *bad, uint32_t *pbad, uint32_t *zero, int nzero)
+// min starts at 1e13, max at 0.  Non-finite coordinates are recorded per
+// workgroup in pbad.  Also zeroes the lb words (used after this kernel).
+__global__ __launch_bounds__(256) void k_bbox_partial(SortSets sets, int nlb0, int nlb1)
 {
     __shared__ double4 s[4];
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < nzero; i += gridDim.x * 256)
-        zero[i] = 0u;
+    const bool second = (int)blockIdx.x >= sets.s[0].np;
+    const SortSet &t = second ? sets.s[1] : sets.s[0];
+    const int bi = blockIdx.x - (second ? sets.s[0].np : 0), nb = t.np, nlb = second ? nlb1 : nlb0;
+    const double *x = t.x, *y = t.y;
+    const int n = t.n;
+    for (int i = bi * 256 + threadIdx.x; i < nlb; i += nb * 256)
+        t.lb[i] = 0u;
     double xmi = 1e13, ymi = 1e13, xma = 0, yma = 0;
     bool nonfinite = false;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    for (int i = bi * 256 + threadIdx.x; i < n; i += nb * 256) {
         const double a = x[i], b = y[i];
         nonfinite |= !isfinite(a) || !isfinite(b);
         xmi = a < xmi ? a : xmi;
@@ -109,12 +131,8 @@ __global__ __launch_bounds__(256) void k_bbox_partial(const double *x, const dou
     if (threadIdx.x == 0)
         s_bad = 0u;
     __syncthreads();
-    if (tc_ballot(nonfinite) && tc_lane() == 0) {
-        if (pbad)
-            s_bad = 1u;
-        else
-            atomicOr(bad, 1u);
-    }
+    if (tc_ballot(nonfinite) && tc_lane() == 0)
+        s_bad = 1u;
     const int wid = threadIdx.x >> 6;
     if (tc_lane() == 0)
         s[wid] = make_double4(xmi, xma, ymi, yma);
@@ -127,9 +145,8 @@ __global__ __launch_bounds__(256) void k_bbox_partial(const double *x, const dou
             r.z = s[w].z < r.z ? s[w].z : r.z;
             r.w = r.w < s[w].w ? s[w].w : r.w;
         }
-        part[blockIdx.x] = r;
-        if (pbad)
-            pbad[blockIdx.x] = s_bad;
+        t.part[bi] = r;
+        t.pbad[bi] = s_bad;
     }
 }
 
@@ -352,16 +369,23 @@ static size_t lb_words(int ntiles) { return (size_t)LB_HIST + LB_TICKETS + (size
 // unpublished for RS_SPIN_MAX polls sets bit 1 of *err (reported by the host
 // as a failed sort) and ends the walk.
 template <int NT>
-__global__ __launch_bounds__(NT) void k_rs_pass_lb(const uint32_t *kin, const uint32_t *vin, uint32_t *kout,
-                                                       uint32_t *vout, int n, int shift, const uint32_t *hist,
-                                                       unsigned long long *flags, uint32_t *ticket, uint32_t *err)
+__global__ __launch_bounds__(NT) void k_rs_pass_lb(SortSets sets, int pass)
 {
     __shared__ int s_tile;
+    const SortSet &t = (int)blockIdx.x < sets.s[0].ntiles ? sets.s[0] : sets.s[1];
+    const uint32_t *const hist = t.lb + RS_BINS * pass;
+    uint32_t *const err = t.bad;
+    unsigned long long *const flags =
+        reinterpret_cast<unsigned long long *>(t.lb + LB_HIST + LB_TICKETS) + (size_t)RS_BINS * t.ntiles * pass;
+    // ping-pong out -> scratch -> out -> scratch -> out; the first pass makes the indices
+    const bool odd = pass & 1;
+    const uint32_t *const kin = odd ? t.k2 : t.keys, *const vin = pass == 0 ? nullptr : (odd ? t.v2 : t.perm);
+    uint32_t *const kout = odd ? t.keys : t.k2, *const vout = odd ? t.perm : t.v2;
     if (threadIdx.x == 0)
-        s_tile = (int)atomicAdd(ticket, 1u);
+        s_tile = (int)atomicAdd(t.lb + LB_HIST + pass, 1u);
     __syncthreads();
     const int tile = s_tile;
-    rs_tile<NT>(kin, vin, kout, vout, n, shift, tile, [&](uint32_t tot, uint32_t *s_w) {
+    rs_tile<NT>(kin, vin, kout, vout, t.n, 8 * pass, tile, [&](uint32_t tot, uint32_t *s_w) {
         const int d = threadIdx.x;
         const bool digit = NT == RS_BINS || d < RS_BINS;
         unsigned long long *fd = flags + (digit ? d : 0);  // fd[t * RS_BINS]: digit d of tile t
@@ -370,24 +394,24 @@ __global__ __launch_bounds__(NT) void k_rs_pass_lb(const uint32_t *kin, const ui
                                __HIP_MEMORY_SCOPE_AGENT);
         uint32_t pre = 0;
         bool done = tile == 0 || !digit;
-        int t = tile;  // tiles t .. tile-1 are summed
+        int u = tile;  // tiles u .. tile-1 are summed
         while (!done) {
-            // the counts of tiles t-1, t-2, ..., RS_LB_BATCH loads in flight at once
-            const int nt = min(RS_LB_BATCH, t);
+            // the counts of tiles u-1, u-2, ..., RS_LB_BATCH loads in flight at once
+            const int nt = min(RS_LB_BATCH, u);
             unsigned long long c[RS_LB_BATCH];
 #pragma unroll
             for (int j = 0; j < RS_LB_BATCH; ++j)
-                c[j] = j < nt ? __hip_atomic_load(&fd[(size_t)(t - 1 - j) * RS_BINS], __ATOMIC_RELAXED,
+                c[j] = j < nt ? __hip_atomic_load(&fd[(size_t)(u - 1 - j) * RS_BINS], __ATOMIC_RELAXED,
                                                   __HIP_MEMORY_SCOPE_AGENT)
                               : 0ull;
 #pragma unroll
             for (int j = 0; j < RS_LB_BATCH; ++j) {
                 if (!done && j < nt) {
                     unsigned long long w = c[j];
-                    // tile t-1-j has not published yet: wait for it
+                    // tile u-1-j has not published yet: wait for it
                     for (int spin = 0; !(w >> 32) && spin < RS_SPIN_MAX; ++spin) {
                         __builtin_amdgcn_s_sleep(2);
-                        w = __hip_atomic_load(&fd[(size_t)(t - 1 - j) * RS_BINS], __ATOMIC_RELAXED,
+                        w = __hip_atomic_load(&fd[(size_t)(u - 1 - j) * RS_BINS], __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT);
                     }
                     if (!(w >> 32))
@@ -396,7 +420,7 @@ __global__ __launch_bounds__(NT) void k_rs_pass_lb(const uint32_t *kin, const ui
                     done = (w & LB_INC) || !(w >> 32);
                 }
             }
-            t -= nt;
+            u -= nt;
         }
         if (tile && digit)
             __hip_atomic_store(&fd[(size_t)tile * RS_BINS], LB_INC | (pre + tot), __ATOMIC_RELAXED,
@@ -408,49 +432,61 @@ __global__ __launch_bounds__(NT) void k_rs_pass_lb(const uint32_t *kin, const ui
 // Keys of the points: sources by sort-sources.cpp:87-110 (quantise +
 // interleave, x in even bits), with `packed` also the source record
 // {x, y, v, 0} in input order, so the gather after the sort reads one 32-byte
-// record per source; targets (HILBERT) by hilbert15.  Tiles of RS_TILE points
-// are taken in turn by at most KH_GRID workgroups, and each workgroup adds the
-// digit totals of all four passes into hist4 (zeroed before) once.  step points (a
-// multiple of 256) per workgroup and turn.  Each
+// record per source; targets by hilbert15.  Steps of kstep points (a multiple of
+// 1,024) are taken in turn by a set's kgrid workgroups, and each workgroup adds the
+// digit totals of all four passes into lb (zeroed before) once.  Each
 // workgroup finishes the bounding box from k_bbox_partial's np partials and
-// per-workgroup flags itself (workgroup 0 writes it and the non-finite flag to
-// box_out and bad_out).
-template <bool HILBERT>
-__global__ __launch_bounds__(256) void k_keys_hist(const double *x, const double *y, const double *v, int n,
-                                                    const double4 *part, const uint32_t *pbad, int np,
-                                                    double *box_out, uint32_t *bad_out, uint32_t *keys,
-                                                    double4 *packed, uint32_t *hist4, int step)
+// per-workgroup flags itself (a set's first one writes it and the non-finite flag).
+__global__ __launch_bounds__(256) void k_keys_hist(SortSets sets)
 {
     __shared__ uint32_t h[4 * RS_BINS];
     __shared__ double s_box[4];
+    const bool second = (int)blockIdx.x >= sets.s[0].kgrid;
+    const SortSet &t = second ? sets.s[1] : sets.s[0];
+    const int bi = blockIdx.x - (second ? sets.s[0].kgrid : 0), n = t.n, step = t.kstep;
+    const double *x = t.x, *y = t.y, *v = t.v;
     for (int i = threadIdx.x; i < 4 * RS_BINS; i += 256)
         h[i] = 0;
     if (threadIdx.x < 64)
-        bbox_finish(part, np, s_box);
+        bbox_finish(t.part, t.np, s_box);
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x < 64) {
+    if (bi == 0 && threadIdx.x < 64) {
         uint32_t b = 0;
-        for (int i = threadIdx.x; i < np; i += 64)
-            b |= pbad[i];
+        for (int i = threadIdx.x; i < t.np; i += 64)
+            b |= t.pbad[i];
         b = tc_ballot(b != 0) ? 1u : 0u;
         if (threadIdx.x == 0) {
             for (int q = 0; q < 4; ++q)
-                box_out[q] = s_box[q];
-            *bad_out = b;
+                t.box[q] = s_box[q];
+            *t.bad = b;
         }
     }
     const double xmin = s_box[0], ymin = s_box[1], scale = s_box[3];
-    for (long long base = (long long)blockIdx.x * step; base < n; base += (long long)gridDim.x * step) {
-#pragma unroll 4
-        for (int j = 0; j < step; j += 256) {
-            const long long i = base + j + threadIdx.x;
-            if (i < n) {
-                const double xi = x[i], yi = y[i];
-                const uint32_t qx = quantise(xi, xmin, scale), qy = quantise(yi, ymin, scale);
-                const uint32_t k = HILBERT ? hilbert15(qx, qy) : (tc_spread15(qx) | (tc_spread15(qy) << 1));
-                keys[i] = k;
-                if (!HILBERT && packed)
-                    packed[i] = make_double4(xi, yi, v[i], 0.0);
+    // four points a turn, loaded before the first is stored (the compiler cannot
+    // tell the arrays apart)
+    constexpr int U = 4;
+    static_assert(KH_TILE_MIN % (256 * U) == 0 && RS_TILE % (256 * U) == 0, "whole turns");
+    for (long long base = (long long)bi * step; base < n; base += (long long)t.kgrid * step) {
+        for (int j = 0; j < step; j += 256 * U) {
+            const long long i0 = base + j + threadIdx.x;
+            double xi[U], yi[U], vi[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long long i = i0 + 256 * u;
+                xi[u] = i < n ? x[i] : 0.0;
+                yi[u] = i < n ? y[i] : 0.0;
+                vi[u] = i < n && t.packed ? v[i] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long long i = i0 + 256 * u;
+                if (i >= n)
+                    break;
+                const uint32_t qx = quantise(xi[u], xmin, scale), qy = quantise(yi[u], ymin, scale);
+                const uint32_t k = v ? tc_spread15(qx) | (tc_spread15(qy) << 1) : hilbert15(qx, qy);
+                t.keys[i] = k;
+                if (t.packed)
+                    t.packed[i] = make_double4(xi[u], yi[u], vi[u], 0.0);
                 atomicAdd(&h[k & 255u], 1u);
                 atomicAdd(&h[RS_BINS + ((k >> 8) & 255u)], 1u);
                 atomicAdd(&h[2 * RS_BINS + ((k >> 16) & 255u)], 1u);
@@ -461,7 +497,7 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double *x, const double
     __syncthreads();
     for (int i = threadIdx.x; i < 4 * RS_BINS; i += 256)
         if (h[i])
-            atomicAdd(&hist4[i], h[i]);
+            atomicAdd(&t.lb[i], h[i]);
 }
 
 // ------------------------------------------------------------------ small sorts
@@ -469,8 +505,9 @@ __global__ __launch_bounds__(256) void k_keys_hist(const double *x, const double
 // bbox_finish semantics), keys (Morton or Hilbert as k_keys_hist), the same
 // stable 4-pass LSD radix sort as above with the keys in registers and each
 // pass's scatter in LDS, and for sources the gather of the sorted records.
-// One launch instead of seven, which is what a small solve is made of.  IT keys
-// per thread, the least power of two that holds the points: the ranking (8
+// One launch instead of seven (and for two sets instead of fourteen), which is what
+// a small solve is made of.  IT keys
+// per thread, the least of 1, 2, 4, 8, 12, 16 that holds the points: the ranking (8
 // ballots per key slot and pass) is what the kernel spends its time on, and
 // with 16 slots for every n it took 48 us at 1,000 points and 79 us at 10,000,
 // with the points on one wave instead of 16; 15 us now at 1,000 points, and back
@@ -479,17 +516,20 @@ constexpr int SS_NT = 1024, SS_MAX_IT = 16, SS_N = SS_NT * SS_MAX_IT;
 static_assert(SS_N == TC_SORT_SMALL_MAX, "one-workgroup sort size");
 
 // The one-workgroup sort of one point set (the body of k_sort_small and of
-// k_sort_small_batch's workgroups).
-template <bool HILBERT, int IT>
-TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ v,
-                       int n, double *__restrict__ box_out, uint32_t *__restrict__ bad_out,
+// k_sort_small_batch's workgroups); the sorted keys stay in lds.k.
+template <int IT> struct SortSmallLds {
+    uint32_t k[SS_NT * IT], v[SS_NT * IT], wrun[SS_NT / 64][RS_BINS];
+};
+template <int IT>
+TC_DEV void sort_small(SortSmallLds<IT> &lds, bool hilbert, const double *__restrict__ x,
+                       const double *__restrict__ y, const double *__restrict__ v, int n,
+                       double *__restrict__ box_out, uint32_t *__restrict__ bad_out,
                        uint32_t *__restrict__ keys_out, uint32_t *__restrict__ perm_out,
                        double4 *__restrict__ src_out)
 {
     constexpr int NW = SS_NT / 64, WITEMS = 64 * IT;
-    __shared__ uint32_t s_k[SS_NT * IT];
-    __shared__ uint32_t s_v[SS_NT * IT];
-    __shared__ uint32_t s_wrun[NW][RS_BINS];
+    uint32_t *const s_k = lds.k, *const s_v = lds.v;
+    uint32_t(*const s_wrun)[RS_BINS] = lds.wrun;
     __shared__ uint32_t s_w[NW + 1];
     __shared__ double4 s_red[NW];
     __shared__ double s_box[4];
@@ -565,7 +605,7 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
     for (int j = 0; j < IT; ++j) {
         const int i = wid * WITEMS + j * 64 + lane;
         const uint32_t qx = quantise(xr[j], xmin, scale), qy = quantise(yr[j], ymin, scale);
-        k[j] = i < n ? (HILBERT ? hilbert15(qx, qy) : (tc_spread15(qx) | (tc_spread15(qy) << 1))) : 0u;
+        k[j] = i < n ? (hilbert ? hilbert15(qx, qy) : (tc_spread15(qx) | (tc_spread15(qy) << 1))) : 0u;
         vi[j] = (uint32_t)i;
     }
 
@@ -639,21 +679,13 @@ TC_DEV void sort_small(const double *__restrict__ x, const double *__restrict__ 
     }
 }
 
-template <bool HILBERT, int IT>
-__global__ __launch_bounds__(SS_NT) void k_sort_small(const double *__restrict__ x, const double *__restrict__ y,
-                                                      const double *__restrict__ v, int n, double *__restrict__ box_out,
-                                                      uint32_t *__restrict__ bad_out, uint32_t *__restrict__ keys_out,
-                                                      uint32_t *__restrict__ perm_out, double4 *__restrict__ src_out)
-{
-    sort_small<HILBERT, IT>(x, y, v, n, box_out, bad_out, keys_out, perm_out, src_out);
-}
-
 // Target orders of several requests at once: workgroup b sorts desc[b]'s
-// targets as k_sort_small<true> does alone (the order does not depend on IT).
+// targets as k_sort_small does alone (the order does not depend on IT).
 template <int IT> __global__ __launch_bounds__(SS_NT) void k_sort_small_batch(const TcSortDesc *__restrict__ desc)
 {
+    __shared__ SortSmallLds<IT> lds;
     const TcSortDesc &d = desc[blockIdx.x];
-    sort_small<true, IT>(d.x, d.y, nullptr, d.n, d.box, d.bad, d.keys, d.perm, nullptr);
+    sort_small<IT>(lds, true, d.x, d.y, nullptr, d.n, d.box, d.bad, d.keys, d.perm, nullptr);
 }
 
 // f(std::integral_constant<int, IT>) with the least IT whose SS_NT IT slots hold n points.
@@ -667,6 +699,8 @@ template <class F> void small_items(int n, F &&f)
         f(std::integral_constant<int, 4>());
     else if (n <= 8 * SS_NT)
         f(std::integral_constant<int, 8>());
+    else if (n <= 12 * SS_NT)
+        f(std::integral_constant<int, 12>());
     else
         f(std::integral_constant<int, SS_MAX_IT>());
 }
@@ -695,6 +729,12 @@ __global__ __launch_bounds__(256) void k_gather_src(const double4 *packed, const
 // short.  Count and emission at 65,536 positions, key by key with IT = 16: 11 +
 // 16 us, with IT = 4: 5 + 6 us; at 2^24 positions 49 + 73 us, with IT = 16: 30 + 60 us.
 constexpr int TB_IT_SMALL = 4, TB_IT = 16, TB_SMALL_N = 1 << 20;
+
+// Census record: level starts, internal count, non-finite flags of the sources and of
+// targets sorted with them (info in device memory), and at int offset INFO_BOX the
+// bounding box; the kernels write it to pinned host memory too, so no copy is queued.
+constexpr int INFO_BOX = 20;
+constexpr size_t INFO_BYTES = sizeof(int) * INFO_BOX + sizeof(double) * 4;
 
 // Internal levels [lo, hi] of the cells starting at this lane's positions
 // (none where hi < lo).
@@ -752,11 +792,6 @@ __global__ __launch_bounds__(256) void k_int_count(const uint32_t *keys, int n, 
             s_cnt[0][threadIdx.x] + s_cnt[1][threadIdx.x] + s_cnt[2][threadIdx.x] + s_cnt[3][threadIdx.x];
 }
 
-// Census record read back by the host in one copy: level starts, internal
-// count, non-finite flag, then (at int offset INFO_BOX) the bounding box.
-constexpr int INFO_BOX = 20;
-constexpr size_t INFO_BYTES = sizeof(int) * INFO_BOX + sizeof(double) * 4;
-
 // The census in one workgroup: cnt holds TC_LMAX rows (levels) of nblk counts,
 // `stride` (a multiple of 4) apart; wave L sums, then scans row L, 1,024 counts
 // a step, so the rows run side by side, each step is one round of wide loads
@@ -765,7 +800,8 @@ constexpr size_t INFO_BYTES = sizeof(int) * INFO_BOX + sizeof(double) * 4;
 // 4,096 blocks (2^24 positions): 11 us; the scan over all rows as one array
 // took 25 us in four launches.
 __global__ __launch_bounds__(SCAN_NT) void k_census(const uint32_t *cnt, uint32_t *offs, int nblk, int stride,
-                                                     const uint32_t *bad, const double *box, int *info)
+                                                     const uint32_t *bad, const uint32_t *tbad, const double *box,
+                                                     int *info, int *hinfo)
 {
     static_assert(TC_LMAX < SCAN_NT / 64, "one wave per level");
     __shared__ uint32_t s_tot[SCAN_NT / 64];
@@ -800,13 +836,20 @@ __global__ __launch_bounds__(SCAN_NT) void k_census(const uint32_t *cnt, uint32_
     for (int q = 0; q < L; ++q)
         start += s_tot[q];
     if (lane == 0) {
+        auto put = [&](int at, int v) {
+            info[at] = v;
+            __hip_atomic_store(hinfo + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        };
         if (L <= TC_LMAX)
-            info[L] = (int)start;  // row TC_LMAX: the total
-        if (L == 0)
-            info[TC_LMAX + 1] = (int)*bad;
+            put(L, (int)start);  // row TC_LMAX: the total
+        if (L == 0) {
+            put(TC_LMAX + 1, (int)*bad);
+            put(TC_LMAX + 2, tbad ? (int)*tbad : 0);
+        }
     }
     if (threadIdx.x >= 32 && threadIdx.x < 36)
-        reinterpret_cast<double *>(info + INFO_BOX)[threadIdx.x - 32] = box[threadIdx.x - 32];
+        __hip_atomic_store(reinterpret_cast<double *>(hinfo + INFO_BOX) + (threadIdx.x - 32), box[threadIdx.x - 32],
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (L >= TC_LMAX)
         return;
     for (int b0 = 0; b0 < nblk; b0 += 1024) {
@@ -985,6 +1028,179 @@ __global__ __launch_bounds__(256) void k_int_nodes(const uint32_t *__restrict__ 
     const uint32_t ni = (uint32_t)group_count<G>(inner);
     if (lane == 0)
         pend[r] = ni << 8 | ni;
+}
+
+// The whole topology of a small tree by the workgroup that sorted its keys, from
+// the keys in LDS (count, census, emission and nodes of the kernels above, which
+// take larger trees): a launch each costs the host more than this takes.
+// At most tmax <= SMALL_TOPO_T internal nodes, a thread per node: a search is a
+// chain of LDS reads, about 50 ns each.  With the joint
+// sorts, 1,000 points drop-in: 138 -> 105 us; 31,623 on host arrays 388 -> 329 us.
+constexpr int SMALL_TOPO_T = SS_NT;
+struct SmallTopo {
+    int cap, tmax;  // tmax 0: no topology
+    int *info, *hinfo, *selfid, *parent;
+    uint32_t *pend, *child;
+    int2 *se;
+    int *level;
+    int2 *cell;
+};
+
+template <int IT>
+TC_DEV void small_topology(SortSmallLds<IT> &lds, const SmallTopo &tp, int n, const double *box, const uint32_t *bad)
+{
+    constexpr int NW = SS_NT / 64;
+    static_assert(SS_N <= 1 << 14 && TC_LMAX < 16, "position and level share a word");
+    const int tid = threadIdx.x, lane = tc_lane(), wid = tid >> 6, cap = tp.cap;
+    const uint32_t *const key = lds.k;
+    uint32_t *const ist = lds.v;             // position | level << 14 by breadth-first rank
+    uint32_t(*const cnt)[RS_BINS] = lds.wrun;  // [wave][level], then first ranks
+    __shared__ int s_start[TC_LMAX + 1];
+    __syncthreads();  // the sort's last reads of lds.v and lds.wrun
+    int lo[IT], hi[IT];
+    uint32_t c[TC_LMAX];
+#pragma unroll
+    for (int L = 0; L < TC_LMAX; ++L)
+        c[L] = 0;
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const int i = wid * 64 * IT + 64 * j + lane;
+        const uint32_t k = i < n ? key[i] : 0u;
+        lo[j] = i >= n ? 1 : (i == 0 ? 0 : tc_common_level(key[i - 1], k) + 1);
+        hi[j] = i >= n ? 0 : (i + cap < n ? min(TC_LMAX - 1, tc_common_level(k, key[i + cap])) : -1);
+        if (!tc_ballot(hi[j] >= lo[j]))
+            continue;
+#pragma unroll
+        for (int L = 0; L < TC_LMAX; ++L)
+            c[L] += __popcll(tc_ballot(L >= lo[j] && L <= hi[j]));
+    }
+    if (lane == 0)
+#pragma unroll
+        for (int L = 0; L < TC_LMAX; ++L)
+            cnt[wid][L] = c[L];
+    __syncthreads();
+    if (wid == 0) {
+        // lane L: level L's count, its first rank, and each wave's
+        uint32_t w[NW], tot = 0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            w[q] = lane < TC_LMAX ? cnt[q][lane] : 0u;
+            tot += w[q];
+        }
+        uint32_t x = tot;
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            const uint32_t y = __shfl_up(x, off, 64);
+            if (lane >= off)
+                x += y;
+        }
+        uint32_t start = x - tot;
+        if (lane <= TC_LMAX) {
+            s_start[lane] = min((int)start, tp.tmax);
+            tp.info[lane] = (int)start;
+            __hip_atomic_store(tp.hinfo + lane, (int)start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (lane < TC_LMAX)
+#pragma unroll
+            for (int q = 0; q < NW; ++q) {
+                cnt[q][lane] = start;
+                start += w[q];
+            }
+        if (lane == 0) {
+            tp.info[TC_LMAX + 1] = (int)*bad;
+            __hip_atomic_store(tp.hinfo + TC_LMAX + 1, (int)*bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (lane >= 32 && lane < 36)
+            __hip_atomic_store(reinterpret_cast<double *>(tp.hinfo + INFO_BOX) + (lane - 32), box[lane - 32],
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int L = 0; L < TC_LMAX; ++L)
+        c[L] = cnt[wid][L];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        if (!tc_ballot(hi[j] >= lo[j]))
+            continue;
+#pragma unroll
+        for (int L = 0; L < TC_LMAX; ++L) {
+            const bool f = L >= lo[j] && L <= hi[j];
+            const unsigned long long b = tc_ballot(f);
+            const uint32_t r = c[L] + __popcll(b & tc_lanemask_lt());
+            if (f && r < (uint32_t)tp.tmax)
+                ist[r] = (uint32_t)(wid * 64 * IT + 64 * j + lane) | (uint32_t)L << 14;
+            c[L] += __popcll(b);
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        // the root; without internal nodes a leaf
+        tp.se[0] = make_int2(0, n);
+        tp.level[0] = 0;
+        tp.cell[0] = make_int2(0, 0);
+        if (s_start[TC_LMAX] == 0)
+            tp.child[0] = 0u;
+    }
+    const int r = tid;
+    if (r >= s_start[TC_LMAX])
+        return;
+    // first position in [a, b) where pred is false
+    auto partition = [](int a, int b, auto pred) {
+        while (a < b) {
+            const int mid = (a + b) >> 1;
+            if (pred(mid))
+                a = mid + 1;
+            else
+                b = mid;
+        }
+        return a;
+    };
+    const int L = (int)(ist[r] >> 14), i = (int)(ist[r] & 0x3fffu);
+    const int sh = 2 * (TC_LMAX - L), csh = sh - 2;
+    const uint32_t prefix = key[i] >> sh;
+    int self = 0, up = 0, e = n;
+    if (L > 0) {
+        up = partition(s_start[L - 1], s_start[L], [&](int p) { return (int)(ist[p] & 0x3fffu) <= i; }) - 1;
+        self = 1 + 4 * up + (int)(prefix & 3u);
+        e = partition(i + cap + 1, n, [&](int p) { return (key[p] >> sh) == prefix; });
+    }
+    tp.selfid[r] = self;
+    tp.parent[r] = up;
+    tp.child[self] = (uint32_t)(1 + 4 * r);
+    uint32_t inner = 0;
+    int a = i;
+    const int cx = 2 * (int)tc_compact15(prefix), cy = 2 * (int)tc_compact15(prefix >> 1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t next = ((prefix << 2) | (uint32_t)(q + 1)) << csh;
+        const int b = q == 3 ? e : partition(a, e, [&](int p) { return key[p] < next; });
+        const int k = 1 + 4 * r + q;
+        tp.se[k] = make_int2(a, b);
+        tp.level[k] = L + 1;
+        tp.cell[k] = make_int2(cx + (q & 1), cy + (q >> 1));
+        if (b - a > cap && L + 1 < TC_LMAX)
+            ++inner;
+        else
+            tp.child[k] = 0u;
+        a = b;
+    }
+    tp.pend[r] = inner << 8 | inner;
+}
+
+// One workgroup per set (one or two): the sort and, for the first set's keys, the topology.
+template <int IT>
+__global__ __launch_bounds__(SS_NT) void k_sort_small(SortSets sets, double4 *__restrict__ src_out, SmallTopo tp)
+{
+    __shared__ SortSmallLds<IT> lds;
+    const SortSet &t = blockIdx.x ? sets.s[1] : sets.s[0];
+    sort_small<IT>(lds, t.v == nullptr, t.x, t.y, t.v, t.n, t.box, t.bad, t.keys, t.perm, blockIdx.x ? nullptr : src_out);
+    if (tp.tmax) {
+        __syncthreads();  // the box and flag written by thread 0 of this workgroup
+        if (blockIdx.x == 0)
+            small_topology<IT>(lds, tp, t.n, t.box, t.bad);
+        else if (threadIdx.x == 0)
+            __hip_atomic_store(tp.hinfo + TC_LMAX + 2, (int)*t.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // Reduce-scatter form of the pairwise lane tree: at offsets 32, 16, ..., 1 a
@@ -1523,38 +1739,58 @@ static const uint32_t *tc_bbox_bad_flag(TcScratch &ws, int n)
     return reinterpret_cast<const uint32_t *>(ws.bbox_part.as<double4>() + np);
 }
 
-// Bounding-box partials of a sort with one-launch passes: np partials, the
-// non-finite flag where tc_bbox_bad_flag finds it, per-workgroup flags after it.
-struct LbBox {
-    double4 *part;
-    uint32_t *bad, *pbad;
-    int np;
-};
-static LbBox lb_box(TcScratch &ws, int n)
+// A set's device memory for a sort with one-launch passes (small: one-workgroup
+// sort): np bounding-box partials, the non-finite flag where tc_bbox_bad_flag finds
+// it, per-workgroup flags after it.
+static SortSet sort_set(const double *x, const double *y, const double *v, int n, double *box, uint32_t *keys,
+                        uint32_t *perm, bool records, TcScratch &ws, bool small)
 {
-    const int np = std::max(1, std::min(1024, tiles_of(n, 256 * 8)));
-    ws.bbox_part.reserve(sizeof(double4) * (size_t)np + 256 + sizeof(uint32_t) * (size_t)np);
-    LbBox b;
-    b.part = ws.bbox_part.as<double4>();
-    b.bad = reinterpret_cast<uint32_t *>(b.part + np);
-    b.pbad = b.bad + 64;
-    b.np = np;
-    return b;
+    SortSet t = {};
+    t.x = x;
+    t.y = y;
+    t.v = v;
+    t.n = n;
+    t.box = box;
+    t.keys = keys;
+    t.perm = perm;
+    t.np = std::max(1, std::min(1024, tiles_of(n, 256 * 8)));
+    if (small) {
+        ws.bbox_part.reserve(sizeof(double4) * (size_t)t.np + 256);
+        t.bad = const_cast<uint32_t *>(tc_bbox_bad_flag(ws, n));
+        return t;
+    }
+    ws.bbox_part.reserve(sizeof(double4) * (size_t)t.np + 256 + sizeof(uint32_t) * (size_t)t.np);
+    t.part = ws.bbox_part.as<double4>();
+    t.bad = const_cast<uint32_t *>(tc_bbox_bad_flag(ws, n));
+    t.pbad = t.bad + 64;
+    t.ntiles = tiles_of(n, RS_TILE);
+    if (lb_words(t.ntiles) > (size_t)INT_MAX)
+        throw TcError(-3, "tc_sort_points: too many points");
+    ws.hist.reserve(sizeof(uint32_t) * lb_words(t.ntiles));
+    t.lb = ws.hist.as<uint32_t>();
+    ws.k2.reserve(sizeof(uint32_t) * (size_t)n);
+    ws.v2.reserve(sizeof(uint32_t) * (size_t)n);
+    t.k2 = ws.k2.as<uint32_t>();
+    t.v2 = ws.v2.as<uint32_t>();
+    if (records) {
+        ws.packed.reserve(sizeof(double4) * (size_t)n);
+        t.packed = ws.packed.as<double4>();
+    }
+    // at most RS_TILE points a step, at least KH_TILE_MIN, about one step per CU
+    t.kstep = std::min(RS_TILE, std::max(KH_TILE_MIN, tiles_of(tiles_of(n, 1024), 256) * 1024));
+    t.kgrid = std::min(tiles_of(n, t.kstep), KH_GRID);
+    return t;
 }
 
-void tc_sort_points(const double *x, const double *y, const double *v, int n, double *box_d, uint32_t *keys_out,
-                    uint32_t *perm_out, double4 *src_out, TcScratch &ws, hipStream_t st, bool hilbert,
-                    const hipEvent_t *ev)
+// Sorts one or two sets (the second with n = 0 for one); both small or neither.
+// src_out: the first set's sorted records; tp: the first set's topology (small
+// sorts only).
+static void sort_sets(const SortSets &t, double4 *src_out, const SmallTopo &tp, hipStream_t st, const hipEvent_t *ev)
 {
-    if (n <= SS_N) {
-        ws.bbox_part.reserve(sizeof(double4) + 256);
-        uint32_t *bad = const_cast<uint32_t *>(tc_bbox_bad_flag(ws, n));
-        small_items(n, [&](auto it) {
-            constexpr int IT = decltype(it)::value;
-            if (hilbert)
-                k_sort_small<true, IT><<<1, SS_NT, 0, st>>>(x, y, v, n, box_d, bad, keys_out, perm_out, src_out);
-            else
-                k_sort_small<false, IT><<<1, SS_NT, 0, st>>>(x, y, v, n, box_d, bad, keys_out, perm_out, src_out);
+    const int sets = t.s[1].n > 0 ? 2 : 1;
+    if (t.s[0].n <= SS_N) {
+        small_items(std::max(t.s[0].n, t.s[1].n), [&](auto it) {
+            k_sort_small<decltype(it)::value><<<sets, SS_NT, 0, st>>>(t, src_out, tp);
         });
         TC_HIP(hipGetLastError());
         if (ev) {
@@ -1564,70 +1800,53 @@ void tc_sort_points(const double *x, const double *y, const double *v, int n, do
         }
         return;
     }
-    // the radix passes take one launch each; their counters are zeroed by the
-    // bounding-box kernel, whose partials the key kernel finishes
-    const size_t words = lb_words(tiles_of(n, RS_TILE));
-    if (words > (size_t)INT_MAX)
-        throw TcError(-3, "tc_sort_points: too many points");
-    ws.hist.reserve(sizeof(uint32_t) * words);
-    uint32_t *lb = ws.hist.as<uint32_t>();
-    const LbBox b = lb_box(ws, n);
-    k_bbox_partial<<<b.np, 256, 0, st>>>(x, y, n, b.part, nullptr, b.pbad, lb, (int)words);
+    // the box, the keys with all four passes' digit totals, then one launch per pass
+    const int ntiles = t.s[0].ntiles + t.s[1].ntiles;
+    k_bbox_partial<<<t.s[0].np + t.s[1].np, 256, 0, st>>>(t, (int)lb_words(t.s[0].ntiles),
+                                                          sets == 2 ? (int)lb_words(t.s[1].ntiles) : 0);
+    k_keys_hist<<<t.s[0].kgrid + t.s[1].kgrid, 256, 0, st>>>(t);
     TC_HIP(hipGetLastError());
-    double4 *packed = nullptr;
-    if (src_out) {
-        ws.packed.reserve(sizeof(double4) * (size_t)n);
-        packed = ws.packed.as<double4>();
-    }
-    tc_morton_sort(x, y, v, n, box_d, keys_out, perm_out, packed, ws, st, hilbert, ev, lb);
-    if (src_out) {
-        k_gather_src<<<tiles_of(n, 256), 256, 0, st>>>(packed, perm_out, n, src_out);
-        TC_HIP(hipGetLastError());
-    }
+    if (ev)
+        TC_HIP(hipEventRecord(ev[0], st));
+    const bool wide = ntiles <= RS_WIDE_TILES;
+    const auto pass_kernel = wide ? k_rs_pass_lb<RS_NT_WIDE> : k_rs_pass_lb<RS_NT>;
+    for (int pass = 0; pass < 4; ++pass)
+        pass_kernel<<<ntiles, wide ? RS_NT_WIDE : RS_NT, 0, st>>>(t, pass);
+    if (src_out)
+        k_gather_src<<<tiles_of(t.s[0].n, 256), 256, 0, st>>>(t.s[0].packed, t.s[0].perm, t.s[0].n, src_out);
+    TC_HIP(hipGetLastError());
     if (ev)
         TC_HIP(hipEventRecord(ev[1], st));
 }
 
-void tc_morton_sort(const double *x, const double *y, const double *v, int n, const double *box_d,
-                    uint32_t *keys_out, uint32_t *perm_out, double4 *packed, TcScratch &ws, hipStream_t st,
-                    bool hilbert, const hipEvent_t *ev, uint32_t *lb)
+void tc_morton_sort(const double *x, const double *y, int n, double *box_d, uint32_t *keys, uint32_t *perm,
+                    TcScratch &ws, hipStream_t st)
 {
-    ws.k2.reserve(sizeof(uint32_t) * (size_t)n);
-    ws.v2.reserve(sizeof(uint32_t) * (size_t)n);
-    const int ntiles = tiles_of(n, RS_TILE);
-    // ping-pong out -> scratch -> out -> scratch -> out (four 8-bit passes over 30-bit keys);
-    // the first pass generates the index payload itself
-    uint32_t *kin[4] = {keys_out, ws.k2.as<uint32_t>(), keys_out, ws.k2.as<uint32_t>()};
-    uint32_t *vin[4] = {nullptr, ws.v2.as<uint32_t>(), perm_out, ws.v2.as<uint32_t>()};
-    uint32_t *kout[4] = {ws.k2.as<uint32_t>(), keys_out, ws.k2.as<uint32_t>(), keys_out};
-    uint32_t *vout[4] = {ws.v2.as<uint32_t>(), perm_out, ws.v2.as<uint32_t>(), perm_out};
-    // the box and keys with all four passes' digit totals, then one launch per
-    // pass (the bounding-box partials and the zeroed region lb were made by the caller)
-    uint32_t *hist4 = lb, *tickets = lb + LB_HIST;
-    unsigned long long *flags = reinterpret_cast<unsigned long long *>(tickets + LB_TICKETS);
-    const LbBox b = lb_box(ws, n);
-    uint32_t *err = b.bad;
-    // at most RS_TILE points a step, at least KH_TILE_MIN, about one step per CU
-    const int step = std::min(RS_TILE, std::max(KH_TILE_MIN, tiles_of(tiles_of(n, 256), 256) * 256));
-    const int grid = std::min(tiles_of(n, step), KH_GRID);
-    if (hilbert)
-        k_keys_hist<true><<<grid, 256, 0, st>>>(x, y, nullptr, n, b.part, b.pbad, b.np, const_cast<double *>(box_d),
-                                                b.bad, keys_out, nullptr, hist4, step);
-    else
-        k_keys_hist<false><<<grid, 256, 0, st>>>(x, y, v, n, b.part, b.pbad, b.np, const_cast<double *>(box_d),
-                                                 b.bad, keys_out, packed, hist4, step);
-    TC_HIP(hipGetLastError());
-    if (ev)
-        TC_HIP(hipEventRecord(ev[0], st));
-    for (int pass = 0; pass < 4; ++pass) {
-        const bool wide = ntiles <= RS_WIDE_TILES;
-        const auto pass_kernel = wide ? k_rs_pass_lb<RS_NT_WIDE> : k_rs_pass_lb<RS_NT>;
-        pass_kernel<<<ntiles, wide ? RS_NT_WIDE : RS_NT, 0, st>>>(kin[pass], vin[pass], kout[pass], vout[pass], n,
-                                                                  8 * pass, hist4 + RS_BINS * pass,
-                                                                  flags + (size_t)RS_BINS * ntiles * pass,
-                                                                  tickets + pass, err);
-        TC_HIP(hipGetLastError());
-    }
+    SortSets t = {};
+    // (any non-null strengths make Morton keys; without records they are not read)
+    t.s[0] = sort_set(x, y, x, n, box_d, keys, perm, false, ws, n <= SS_N);
+    sort_sets(t, nullptr, SmallTopo{}, st, nullptr);
+}
+
+// Targets' buffers in ws: keys, permutation, and the box after the source box's place.
+static SortSet target_set(const double *xt, const double *yt, int m, TcScratch &ws, bool small)
+{
+    ws.tkeys.reserve(sizeof(uint32_t) * (size_t)m + 64);
+    ws.tperm.reserve(sizeof(uint32_t) * (size_t)m + 64);
+    ws.info.reserve(sizeof(int) * 32 + sizeof(double) * 4);
+    return sort_set(xt, yt, nullptr, m, reinterpret_cast<double *>(ws.info.as<char>() + 128), ws.tkeys.as<uint32_t>(),
+                    ws.tperm.as<uint32_t>(), false, ws, small);
+}
+
+// Sources and targets up to here in total go through one set of launches; beyond, the
+// GPU is filled by either, and the targets' sort runs beside the build on a stream of
+// its own.
+constexpr int SORT_JOINT_MAX = 1 << 20;
+bool tc_sorts_jointly(int n, int m)
+{
+    if (n <= 0 || m <= 0)
+        return false;
+    return n <= SS_N ? m <= SS_N : m > SS_N && (long long)n + m <= SORT_JOINT_MAX;
 }
 
 // info, tmax: the tree's internal nodes as the kernels read them (at most tmax);
@@ -1691,7 +1910,7 @@ static long long internal_bound(int n, int leafcap)
 
 void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v, int n, int leafcap, int order,
                    bool fp32, bool deriv, TcScratch &ws, hipStream_t st, const hipEvent_t *ev,
-                   const std::function<void()> *at_census)
+                   const std::function<void()> *at_census, TcJointTargets *targets)
 {
     if (n <= 0)
         throw TcError(-3, "tc_build_tree: no sources");
@@ -1716,26 +1935,20 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
 
     double *box = t.box_d.as<double>();
     uint32_t *keys = t.keys.as<uint32_t>(), *perm = t.perm.as<uint32_t>();
-    tc_sort_points(x, y, v, n, box, keys, perm, t.src.as<double4>(), ws, st, false, ev);
-
-    // census of internal cells
-    const bool few = n <= TB_SMALL_N;
-    const int nblk = tiles_of(n, 256 * (few ? TB_IT_SMALL : TB_IT));
-    const int stride = (nblk + 3) & ~3;
-    ws.part.reserve(sizeof(uint32_t) * (size_t)2 * TC_LMAX * stride);
-    uint32_t *cnt = ws.part.as<uint32_t>();
-    uint32_t *offs = cnt + (size_t)TC_LMAX * stride;
-    ws.info.reserve(sizeof(int) * 32);
+    const bool small = n <= SS_N;
+    SortSets sets = {};
+    sets.s[0] = sort_set(x, y, v, n, box, keys, perm, true, ws, small);
+    const uint32_t *tbad = nullptr;
+    if (targets) {
+        sets.s[1] = target_set(targets->x, targets->y, targets->m, *targets->ws, small);
+        tbad = sets.s[1].bad;
+    }
+    ws.info.reserve(sizeof(int) * 32 + sizeof(double) * 4);
     int *info = ws.info.as<int>();
-    if (few)
-        k_int_count<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, stride);
-    else
-        k_int_count<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, stride);
-    k_census<<<1, SCAN_NT, 0, st>>>(cnt, offs, nblk, stride, tc_bbox_bad_flag(ws, n), box, info);
-    TC_HIP(hipGetLastError());
     static_assert(INFO_BYTES <= sizeof(int) * 32 && INFO_BYTES <= TcScratch::PINNED_BYTES, "census record size");
     char *hp = static_cast<char *>(ws.host_pinned());
-    TC_HIP(hipMemcpyAsync(hp, info, INFO_BYTES, hipMemcpyDeviceToHost, st));
+    int *hrec = reinterpret_cast<int *>(hp);
+
     // Where the bound on the node count fits a modest buffer, the rest of the
     // build is queued behind the census at that bound (its kernels read the count on the
     // device), and the host waits for the record while they run: queued after the
@@ -1746,11 +1959,73 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
                             (fp32 ? 8 * ((size_t)order + 1) : 0);
     const long long bound = internal_bound(n, leafcap);
     const bool ahead = !t.nodes.arena && bound <= AHEAD_NODES && (1 + 4 * (size_t)bound) * per_node <= AHEAD_BYTES;
+    const bool topo_small = ahead && small && bound <= SMALL_TOPO_T;
+
+    int T = (int)std::min<long long>(bound, INT_MAX / 8), hinfo[TC_LMAX + 3];
+    uint32_t *child = nullptr, *pend = nullptr;
+    int2 *se = nullptr, *cell = nullptr;
+    int *lev = nullptr, *istart = nullptr, *ilevel = nullptr;
+    // buffers of a tree of at most T internal nodes
+    auto reserve_nodes = [&] {
+        const size_t nn = 1 + 4 * (size_t)T;
+        t.nodes.reserve(sizeof(TcNode) * nn);
+        t.exps.reserve(sizeof(double) * 2 * (size_t)order * nn);
+        if (t.has_deriv)
+            t.dexps.reserve(sizeof(double) * 2 * (size_t)order * nn);
+        t.nodew.reserve(sizeof(double4) * nn);
+        t.selfid.reserve(sizeof(int) * (size_t)(T + 1));
+        if (fp32)
+            t.exps32.reserve(sizeof(float2) * (size_t)(order + 1) * nn);
+        ws.istart.reserve(sizeof(int) * 2 * (size_t)(T + 1));
+        istart = ws.istart.as<int>();
+        pend = ws.istart.as<uint32_t>() + T + 1;
+        ws.ilevel.reserve(sizeof(int) * (size_t)(T + 1));
+        ilevel = ws.ilevel.as<int>();
+        // per-node topology scratch: child | se | level | cell
+        ws.ints.reserve(sizeof(int) * nn * 6 + 64);
+        child = ws.ints.as<uint32_t>();
+        se = reinterpret_cast<int2 *>(child + ((nn + 1) & ~size_t(1)));
+        lev = reinterpret_cast<int *>(se + nn);
+        cell = reinterpret_cast<int2 *>(lev + ((nn + 1) & ~size_t(1)));
+    };
+    SmallTopo tp = {};
+    if (ahead)
+        reserve_nodes();
+    if (topo_small) {
+        tp.cap = leafcap;
+        tp.tmax = std::max(1, T);
+        tp.info = info;
+        tp.hinfo = hrec;
+        tp.selfid = t.selfid.as<int>();
+        tp.parent = ilevel;
+        tp.pend = pend;
+        tp.child = child;
+        tp.se = se;
+        tp.level = lev;
+        tp.cell = cell;
+    }
+    sort_sets(sets, t.src.as<double4>(), tp, st, ev);
+
+    // census of internal cells
+    const bool few = n <= TB_SMALL_N;
+    const int nblk = tiles_of(n, 256 * (few ? TB_IT_SMALL : TB_IT));
+    const int stride = (nblk + 3) & ~3;
+    uint32_t *cnt = nullptr, *offs = nullptr;
+    if (!topo_small) {
+        ws.part.reserve(sizeof(uint32_t) * (size_t)2 * TC_LMAX * stride);
+        cnt = ws.part.as<uint32_t>();
+        offs = cnt + (size_t)TC_LMAX * stride;
+        if (few)
+            k_int_count<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, stride);
+        else
+            k_int_count<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, cnt, stride);
+        k_census<<<1, SCAN_NT, 0, st>>>(cnt, offs, nblk, stride, sets.s[0].bad, tbad, box, info, hrec);
+        TC_HIP(hipGetLastError());
+    }
     if (ahead)
         TC_HIP(hipEventRecord(ws.census_event(), st));
     if (at_census)
         (*at_census)();  // work queued elsewhere fills the GPU while the host waits
-    int T = (int)std::min<long long>(bound, INT_MAX / 8), hinfo[TC_LMAX + 2];
     const int *starts = nullptr;
     auto census = [&] {
         if (ahead)
@@ -1770,42 +2045,26 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
         t.level_start[TC_LMAX + 1] = hinfo[TC_LMAX];
         t.ninternal = hinfo[TC_LMAX];
         t.nnodes = 1 + 4 * t.ninternal;
+        if (targets)
+            targets->bad = (uint32_t)hinfo[TC_LMAX + 2];
     };
     if (!ahead) {
         census();
         T = t.ninternal;
         starts = t.level_start;
+        reserve_nodes();
     }
-    const int nn = 1 + 4 * T;
-
-    t.nodes.reserve(sizeof(TcNode) * (size_t)nn);
-    t.exps.reserve(sizeof(double) * 2 * (size_t)order * nn);
-    if (t.has_deriv)
-        t.dexps.reserve(sizeof(double) * 2 * (size_t)order * nn);
-    t.nodew.reserve(sizeof(double4) * (size_t)nn);
-    t.selfid.reserve(sizeof(int) * (size_t)(T + 1));
-    if (fp32)
-        t.exps32.reserve(sizeof(float2) * (size_t)(order + 1) * nn);
-    ws.istart.reserve(sizeof(int) * 2 * (size_t)(T + 1));
-    uint32_t *pend = ws.istart.as<uint32_t>() + T + 1;
-    ws.ilevel.reserve(sizeof(int) * (size_t)(T + 1));
-    // per-node topology scratch: child | se | level | cell
-    ws.ints.reserve(sizeof(int) * (size_t)nn * 6 + 64);
-    uint32_t *child = ws.ints.as<uint32_t>();
-    int2 *se = reinterpret_cast<int2 *>(child + ((nn + 1) & ~1));
-    int *lev = reinterpret_cast<int *>(se + nn);
-    int2 *cell = reinterpret_cast<int2 *>(lev + ((nn + 1) & ~1));
-
-    int *istart = ws.istart.as<int>(), *ilevel = ws.ilevel.as<int>();
-    if (T > 0 && few)
-        k_int_emit<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, T, istart, ilevel);
-    else if (T > 0)
-        k_int_emit<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, T, istart, ilevel);
-    const bool by_wave = T <= NODES_WAVE_T;
-    const auto nodes_kernel = by_wave ? k_int_nodes<64> : k_int_nodes<16>;
-    nodes_kernel<<<std::max(1, tiles_of(T, by_wave ? 4 : 16)), 256, 0, st>>>(
-        keys, n, leafcap, istart, ilevel, info, T, t.selfid.as<int>(), pend, child, se, lev, cell);
-    TC_HIP(hipGetLastError());
+    if (!topo_small) {
+        if (T > 0 && few)
+            k_int_emit<TB_IT_SMALL><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, T, istart, ilevel);
+        else if (T > 0)
+            k_int_emit<TB_IT><<<nblk, 256, 0, st>>>(keys, n, leafcap, offs, stride, T, istart, ilevel);
+        const bool by_wave = T <= NODES_WAVE_T;
+        const auto nodes_kernel = by_wave ? k_int_nodes<64> : k_int_nodes<16>;
+        nodes_kernel<<<std::max(1, tiles_of(T, by_wave ? 4 : 16)), 256, 0, st>>>(
+            keys, n, leafcap, istart, ilevel, info, T, t.selfid.as<int>(), pend, child, se, lev, cell);
+        TC_HIP(hipGetLastError());
+    }
     if (ev)
         TC_HIP(hipEventRecord(ev[2], st));
 
@@ -1840,18 +2099,14 @@ TcSortDesc tc_sort_targets_desc(const double *xt, const double *yt, int m, TcScr
     if (m < 1 || m > SS_N)
         throw TcError(-3, "tc_sort_targets_desc: 1 to 16384 targets");
     // the buffers and places tc_sort_targets uses for m targets
-    ws.tkeys.reserve(sizeof(uint32_t) * (size_t)m + 64);
-    ws.tperm.reserve(sizeof(uint32_t) * (size_t)m + 64);
-    ws.tsorted.reserve(sizeof(double) * 2 * (size_t)m + 64);
-    ws.info.reserve(sizeof(int) * 32 + sizeof(double) * 4);
-    ws.bbox_part.reserve(sizeof(double4) + 256);
+    const SortSet t = target_set(xt, yt, m, ws, true);
     TcSortDesc d;
     d.x = xt;
     d.y = yt;
-    d.box = reinterpret_cast<double *>(ws.info.as<char>() + 128);
-    d.bad = const_cast<uint32_t *>(tc_bbox_bad_flag(ws, m));
-    d.keys = ws.tkeys.as<uint32_t>();
-    d.perm = ws.tperm.as<uint32_t>();
+    d.box = t.box;
+    d.bad = t.bad;
+    d.keys = t.keys;
+    d.perm = t.perm;
     d.n = m;
     d.pad = 0;
     return d;
@@ -1867,12 +2122,7 @@ void tc_sort_targets_batch(const TcSortDesc *desc_dev, int k, int mmax, hipStrea
 
 void tc_sort_targets(const double *xt, const double *yt, int m, TcScratch &ws, hipStream_t st)
 {
-    ws.tkeys.reserve(sizeof(uint32_t) * (size_t)m + 64);
-    ws.tperm.reserve(sizeof(uint32_t) * (size_t)m + 64);
-    ws.tsorted.reserve(sizeof(double) * 2 * (size_t)m + 64);
-    // the target box lives after the keys' tail
-    DevBuf &boxbuf = ws.info;
-    ws.info.reserve(sizeof(int) * 32 + sizeof(double) * 4);
-    double *box = reinterpret_cast<double *>(boxbuf.as<char>() + 128);
-    tc_sort_points(xt, yt, nullptr, m, box, ws.tkeys.as<uint32_t>(), ws.tperm.as<uint32_t>(), nullptr, ws, st, true);
+    SortSets t = {};
+    t.s[0] = target_set(xt, yt, m, ws, m <= SS_N);
+    sort_sets(t, nullptr, SmallTopo{}, st, nullptr);
 }

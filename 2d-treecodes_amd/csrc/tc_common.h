@@ -303,7 +303,7 @@ struct TcTree {
 
 // Scratch reused across calls of one context.
 struct TcScratch {
-    DevBuf k2, v2, hist, part, istart, ilevel, info, tkeys, tperm, tsorted, bbox_part, ints, packed, work,
+    DevBuf k2, v2, hist, part, istart, ilevel, info, tkeys, tperm, bbox_part, ints, packed, work,
         flist;
     // pinned host memory for the per-solve readbacks (tree census, flags): a
     // copy into pageable memory costs a staged transfer of its own
@@ -327,7 +327,7 @@ struct TcScratch {
         if (census_ev)
             (void)hipEventDestroy(census_ev);
         census_ev = nullptr;
-        for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
+        for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm,
                           &bbox_part, &ints, &packed, &work, &flist})
             b->release();
         if (pinned)
@@ -338,7 +338,7 @@ struct TcScratch {
     // exist (host_pinned() at set-up), so no call made with this scratch allocates.
     void bind(TcArena *a)
     {
-        for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm, &tsorted,
+        for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm,
                           &bbox_part, &ints, &packed, &work, &flist})
             b->bind(a);
     }
@@ -368,31 +368,30 @@ size_t tc_noalloc_scratch_bytes();
 void *tc_noalloc_scratch_lookup(int device);
 
 // Internal entry points (tc_build.hip, tc_eval.hip)
-// Bounding box, keys (Morton, or Hilbert for targets) and stable sort of n
-// points; with src_out also the sorted records {x, y, v, 0}.  One workgroup
-// for n <= 16384, else a bounding-box partial kernel and tc_morton_sort.
-// ev (optional, two events): recorded after the keys and after the sorted records.
-void tc_sort_points(const double *x, const double *y, const double *v, int n, double *box_d, uint32_t *keys_out,
-                    uint32_t *perm_out, double4 *src_out, TcScratch &ws, hipStream_t st, bool hilbert,
-                    const hipEvent_t *ev = nullptr);
-// Keys and the four one-launch radix passes.  lb: the passes' digit totals,
-// tickets and published tile counts, zeroed beforehand by the bounding-box
-// partial kernel, whose partials the key kernel then finishes into box_d (as
-// tc_sort_points does).
-void tc_morton_sort(const double *x, const double *y, const double *v, int n, const double *box_d,
-                    uint32_t *keys_out, uint32_t *perm_out, double4 *packed, TcScratch &ws, hipStream_t st,
-                    bool hilbert, const hipEvent_t *ev, uint32_t *lb);
+// Bounding box, Morton keys and stable sort of n points.
+void tc_morton_sort(const double *x, const double *y, int n, double *box_d, uint32_t *keys, uint32_t *perm,
+                    TcScratch &ws, hipStream_t st);
+// Targets that a build sorts with its sources, in the same launches (where
+// tc_sorts_jointly says so), into ws as tc_sort_targets does; bad: their
+// non-finite flag, set when tc_build_tree returns.
+struct TcJointTargets {
+    const double *x, *y;
+    int m;
+    TcScratch *ws;
+    uint32_t bad;
+};
+bool tc_sorts_jointly(int n, int m);
 // fp32: also build the FP32 mirrors; deriv: a force tree, whose coefficient
 // mirror holds k b_k instead of b_k, and which without mirrors (FP64) keeps k a_k.
 // ev (optional, four events): recorded after the Morton keys, the sorted
 // records, the topology and the upward pass (the build's phase boundaries).
-// at_census (optional): called once the census readback is queued, before the
+// at_census (optional): called once the census is queued, before the
 // host waits for it (the caller can queue independent work on another stream).
 // Returns with the build queued on st and the tree's counts known; a non-finite
 // source throws.
 void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v, int n, int leafcap, int order,
                    bool fp32, bool deriv, TcScratch &ws, hipStream_t st, const hipEvent_t *ev = nullptr,
-                   const std::function<void()> *at_census = nullptr);
+                   const std::function<void()> *at_census = nullptr, TcJointTargets *targets = nullptr);
 // Adds k a_k to a force tree that has none (one built for FP32), for an FP64 evaluation of it.
 void tc_tree_deriv(TcTree &t, hipStream_t st);
 void tc_sort_targets(const double *xt, const double *yt, int m, TcScratch &ws, hipStream_t st);

@@ -31,9 +31,9 @@ def test_upward_variants(pkg, oracle, wl, n, leaf, order):
     ctx.close()
 
 
-# one-workgroup sorts with 1, 2, 4, 8, 16 keys per thread, one-launch passes with 1,024 threads a
+# one-workgroup sorts with 1, 2, 4, 8, 12, 16 keys per thread, one-launch passes with 1,024 threads a
 # tile (up to 256 tiles of 5,120 keys) and 256 beyond; many equal keys, so stability shows
-@pytest.mark.parametrize("n", [1, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 16384, 16385, 40961,
+@pytest.mark.parametrize("n", [1, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 12288, 12289, 16384, 16385, 40961,
                                256 * 5120, 256 * 5120 + 1])
 def test_sort_variants(pkg, oracle, wl, n):
     st = wl.Stream(n)
@@ -144,4 +144,36 @@ def test_float_forces_equal_double_forces(pkg, wl, nb):
     ctx = pkg.Context(precision=pkg.FP32)
     rx, ry = ctx.force(0.5, *[v.astype(np.float64) for v in a])
     assert np.array_equal(fx, rx.astype(np.float32)) and np.array_equal(fy, ry.astype(np.float32))
+    ctx.close()
+
+
+# topology by the sorting workgroup (up to 1,024 internal nodes by the bound) and by its own kernels;
+# a tree queued at its node bound and one that waits for its census; sources and targets sorted
+# together (both small, both middling) and apart
+@pytest.mark.parametrize("n,m,leaf", [(1, 1, 1), (2, 3, 1), (70, 1000, 1), (900, 16384, 64), (16384, 1, 200),
+                                      (16384, 16385, 200), (16385, 16384, 200), (12000, 9000, 8), (20000, 20001, 2),
+                                      (20000, 30000, 300), (600000, 448576, 512), (600000, 448577, 512)])
+def test_build_queueing_variants(pkg, oracle, wl, n, m, leaf):
+    xs, ys, vs, *_ = wl.mixed_plummer_potential(n, seed=leaf)
+    st = wl.Stream(m)
+    xt, yt = st.uniform(m), st.uniform(m)
+    ctx = pkg.Context(pot_order=8, pot_leaf=leaf)
+    ot = oracle.Tree(xs, ys, vs, leaf, 8)
+    idx = np.sort(np.random.default_rng(m).choice(m, min(m, 300), replace=False))
+    ref, _ = ot.potential(0.5, xt[idx], yt[idx])
+    for _ in range(2):
+        out = ctx.potential(0.5, xs, ys, vs, xt, yt)
+        assert rel_l2(out[idx], ref) <= 1e-12
+    compare_tree(ctx.tree(), ot)
+    # non-finite coordinates are reported, and the context stays usable
+    for bad in (0, n - 1):
+        b = xs.copy()
+        b[bad] = np.nan
+        with pytest.raises(pkg.TreecodeError):
+            ctx.potential(0.5, b, ys, vs, xt, yt)
+    b = xt.copy()
+    b[-1] = np.inf
+    with pytest.raises(pkg.TreecodeError):
+        ctx.potential(0.5, xs, ys, vs, b, yt)
+    assert np.array_equal(ctx.potential(0.5, xs, ys, vs, xt, yt), out)
     ctx.close()
