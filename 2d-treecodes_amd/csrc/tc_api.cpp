@@ -1089,7 +1089,7 @@ size_t tc_srv_context_bytes(tc_context *c)
     size_t b = tc_tree_bytes(c->tree) + c->io.cap + c->cnt.cap;
     for (const TcScratch *w : {&c->ws, &c->tws})
         for (const DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->istart, &w->ilevel, &w->info,
-                                &w->tkeys, &w->tperm, &w->bbox_part, &w->ints, &w->packed, &w->work,
+                                &w->tkeys, &w->tperm, &w->bbox_part, &w->ints, &w->packed,
                                 &w->flist})
             b += d->cap;
     return b;
@@ -1105,7 +1105,7 @@ void tc_srv_context_trim(tc_context *c)
     c->io.release();
     for (TcScratch *w : {&c->ws, &c->tws})
         for (DevBuf *d : {&w->k2, &w->v2, &w->hist, &w->part, &w->istart, &w->ilevel, &w->info,
-                          &w->tkeys, &w->tperm, &w->bbox_part, &w->ints, &w->packed, &w->work,
+                          &w->tkeys, &w->tperm, &w->bbox_part, &w->ints, &w->packed,
                           &w->flist})
             d->release();
 }

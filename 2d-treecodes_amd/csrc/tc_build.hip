@@ -1369,7 +1369,7 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
 // by the same operations as a child-by-child loop.
 template <int P> constexpr int E2E_G = P <= 16 ? 16 : 32;
 
-// C(l, k) at [k * P + l], k <= l < P: lane l reads consecutive words
+// C(l, k) at [k * P + l], k, l < P (0 for k > l): lane l reads consecutive words
 template <int P> TC_DEV void e2e_binom(double *s_binom)
 {
     for (int i = threadIdx.x; i < P * P; i += blockDim.x)
@@ -1512,13 +1512,16 @@ TC_DEV void e2e_node(int rank, const int *selfid, const double *box, TcNode *nod
             double rt = mq[q] * ninv;
             double it = a[0].y;
             rt = rt + a[0].x;
-#pragma unroll 4
+            // lanes past their last term keep their sums by selects, not branches, so that
+            // the LDS reads of several terms are in flight (order 24, 10,000 points:
+            // chained levels 37 -> 32 us)
+            const double *bin = s_binom + (gl < P ? gl : 0);
+#pragma unroll(P > 16 ? 8 : 4)
             for (int k = 1; k < P; ++k) {
-                if (k <= gl && gl < P) {
-                    const double bk = s_binom[k * P + gl];
-                    rt = rt + a[k].x * bk;
-                    it = it + a[k].y * bk;
-                }
+                const double bk = bin[k * P];
+                const double nr = rt + a[k].x * bk, ni = it + a[k].y * bk;
+                rt = k <= gl ? nr : rt;
+                it = k <= gl ? ni : it;
             }
             const double invz2 = zr[q] * zr[q] + zi[q] * zi[q];
             const double invinv = invz2 != 0 ? 1 / invz2 : 0;

@@ -303,7 +303,7 @@ struct TcTree {
 
 // Scratch reused across calls of one context.
 struct TcScratch {
-    DevBuf k2, v2, hist, part, istart, ilevel, info, tkeys, tperm, bbox_part, ints, packed, work,
+    DevBuf k2, v2, hist, part, istart, ilevel, info, tkeys, tperm, bbox_part, ints, packed,
         flist;
     // pinned host memory for the per-solve readbacks (tree census, flags): a
     // copy into pageable memory costs a staged transfer of its own
@@ -328,7 +328,7 @@ struct TcScratch {
             (void)hipEventDestroy(census_ev);
         census_ev = nullptr;
         for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm,
-                          &bbox_part, &ints, &packed, &work, &flist})
+                          &bbox_part, &ints, &packed, &flist})
             b->release();
         if (pinned)
             (void)hipHostFree(pinned);
@@ -339,7 +339,7 @@ struct TcScratch {
     void bind(TcArena *a)
     {
         for (DevBuf *b : {&k2, &v2, &hist, &part, &istart, &ilevel, &info, &tkeys, &tperm,
-                          &bbox_part, &ints, &packed, &work, &flist})
+                          &bbox_part, &ints, &packed, &flist})
             b->bind(a);
     }
 };

@@ -1098,7 +1098,7 @@ template <bool F32> constexpr int P2P_TILE_N = F32 ? 64 : 32;
 // in the pool is marked in pmark and listed in ovf; the NEAR instantiation of
 // k_force then repeats its traversal and sums all its P2P leaves.
 constexpr int FP2P_INLINE = 64;  // default of the inline count (TcNearLists::inl)
-enum { FN_OVF = 0, FN_CHUNKS = 1, FN_OBRICKS = 2, FN_NCTR = 4 };
+enum { FN_OVF = 0, FN_CHUNKS = 1, FN_OBRICKS = 2, FN_WORK = 64, FN_NCTR = 128 };  // FN_WORK: the brick queue, a cache line of its own, cleared with the rest
 struct TcNearLists {
     uint32_t *pmark;    // [nb] 1: the brick is listed in ovf
     int *ohead;         // [nb] first chunk of a brick listed in obricks
@@ -2056,8 +2056,8 @@ template <auto Kernel> int resident_blocks(int device)
 
 template <int P, bool F32>
 void launch_force_pass(const TcTree &t, double theta, const double *x0s, const double *y0s, const double *hs,
-                       int first, int nb, double *xr, double *yr, unsigned long long *counters, uint32_t *work,
-                       const TcNearLists &nl, int device, hipStream_t st)
+                       int first, int nb, double *xr, double *yr, unsigned long long *counters, const TcNearLists &nl,
+                       int device, hipStream_t st)
 {
     const TcNode *nodes = t.nodes.as<TcNode>();
     const double *exps = t.exps.as<double>();
@@ -2065,8 +2065,8 @@ void launch_force_pass(const TcTree &t, double theta, const double *x0s, const d
     const float2 *exps32 = F32 ? t.exps32.as<float2>() : nullptr;
     const double4 *src = t.src.as<double4>();
     const float4 *src32 = F32 ? t.src32.as<float4>() : nullptr;
-    tc_fill_u32(work, 0u, 1, st);
     tc_fill_u32(nl.ctr, 0u, FN_NCTR, st);
+    uint32_t *work = nl.ctr + FN_WORK;
     if (counters) {
         const int grid = std::min(tiles_of(nb, 4), resident_blocks<k_force<P, F32, false, true>>(device));
         k_force<P, F32, false, true><<<grid, 256, 0, st>>>(nodes, exps, dexps, exps32, src, src32, x0s, y0s, hs, first, nb,
@@ -2104,7 +2104,6 @@ void launch_force(const TcTree &t, double theta, const double *x0s, const double
     const int maxc = max_chunks > 0 ? max_chunks : std::max(4096, chunk / 4);
     const size_t part_bytes = sizeof(double2) * 64 * (size_t)maxc;
     const size_t u32s = (size_t)chunk * 4 + (size_t)maxc * (64 + 4) + FN_NCTR;
-    ws.work.reserve(256);
     ws.flist.reserve(part_bytes + sizeof(uint32_t) * u32s);
     TcNearLists nl;
     nl.cpart = ws.flist.as<double2>();
@@ -2124,13 +2123,12 @@ void launch_force(const TcTree &t, double theta, const double *x0s, const double
     nl.ctr = u;
     nl.maxc = maxc;
     nl.inl = inline_leaves > 0 ? inline_leaves : FP2P_INLINE;
-    uint32_t *work = ws.work.as<uint32_t>();
     for (int first = 0; first < nbricks; first += chunk) {
         const int nb = std::min(chunk, nbricks - first);
         if (precision == 1)
-            launch_force_pass<P, true>(t, theta, x0s, y0s, hs, first, nb, xr, yr, counters, work, nl, device, st);
+            launch_force_pass<P, true>(t, theta, x0s, y0s, hs, first, nb, xr, yr, counters, nl, device, st);
         else
-            launch_force_pass<P, false>(t, theta, x0s, y0s, hs, first, nb, xr, yr, counters, work, nl, device, st);
+            launch_force_pass<P, false>(t, theta, x0s, y0s, hs, first, nb, xr, yr, counters, nl, device, st);
     }
 }
 
