@@ -119,14 +119,7 @@ __global__ __launch_bounds__(256) void k_bbox_partial(SortSets sets, int nlb0, i
         ymi = b < ymi ? b : ymi;
         yma = yma < b ? b : yma;
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        double o;
-        o = __shfl_xor(xmi, off, 64); xmi = o < xmi ? o : xmi;
-        o = __shfl_xor(ymi, off, 64); ymi = o < ymi ? o : ymi;
-        o = __shfl_xor(xma, off, 64); xma = xma < o ? o : xma;
-        o = __shfl_xor(yma, off, 64); yma = yma < o ? o : yma;
-    }
+    tc_wave_box(xmi, ymi, xma, yma);
     __shared__ uint32_t s_bad;
     if (threadIdx.x == 0)
         s_bad = 0u;
@@ -162,14 +155,7 @@ TC_DEV void bbox_finish(const double4 *part, int np, double *box)
         ymi = r.z < ymi ? r.z : ymi;
         yma = yma < r.w ? r.w : yma;
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        double o;
-        o = __shfl_xor(xmi, off, 64); xmi = o < xmi ? o : xmi;
-        o = __shfl_xor(ymi, off, 64); ymi = o < ymi ? o : ymi;
-        o = __shfl_xor(xma, off, 64); xma = xma < o ? o : xma;
-        o = __shfl_xor(yma, off, 64); yma = yma < o ? o : yma;
-    }
+    tc_wave_box(xmi, ymi, xma, yma);
     if (tc_lane() == 0) {
         const double ext0 = xma - xmi, ext1 = yma - ymi;
         const double eps = 10000 * DBL_EPSILON;
@@ -560,14 +546,7 @@ TC_DEV void sort_small(SortSmallLds<IT> &lds, bool hilbert, const double *__rest
             yma = yma < b ? b : yma;
         }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        double o;
-        o = __shfl_xor(xmi, off, 64); xmi = o < xmi ? o : xmi;
-        o = __shfl_xor(ymi, off, 64); ymi = o < ymi ? o : ymi;
-        o = __shfl_xor(xma, off, 64); xma = xma < o ? o : xma;
-        o = __shfl_xor(yma, off, 64); yma = yma < o ? o : yma;
-    }
+    tc_wave_box(xmi, ymi, xma, yma);
     const bool wbad = tc_ballot(nonfinite) != 0;
     if (lane == 0) {
         s_red[wid] = make_double4(xmi, xma, ymi, yma);
@@ -826,9 +805,7 @@ __global__ __launch_bounds__(SCAN_NT) void k_census(const uint32_t *cnt, uint32_
             for (int j = 0; j < 4; ++j)
                 tot += (v[j].x + v[j].y) + (v[j].z + v[j].w);
         }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-        tot += __shfl_xor(tot, off, 64);
+    tc_offsets<32, 1>([&](auto off) { tot = tc_xor_add<off.value>(tot); });
     if (lane == 0)
         s_tot[L] = tot;
     __syncthreads();
@@ -1203,49 +1180,42 @@ __global__ __launch_bounds__(SS_NT) void k_sort_small(SortSets sets, double4 *__
     }
 }
 
-// Reduce-scatter form of the pairwise lane tree: at offsets 32, 16, ..., 1 a
-// lane keeps half of its values and adds the partner's copies of that half,
-// so after log2(NV) halvings (then plain butterfly steps) lane l holds the
-// full sum of value (l >> (6 - log2 NV)).  Every sum is formed from the same
-// pairs in the same order as tc_wave_tree_sum (a + b == b + a), so results are
-// bit-identical to reducing each value separately, with NV - 1 + (6 - log2 NV)
-// shuffles instead of 6 NV.
-template <int C> TC_DEV void rs_halve(double *v, int off, bool up)
+// Reduce-scatter form of the pairwise lane tree: at offsets 32, 16, ..., 1 the
+// lanes whose bit is clear keep the first half of their values (the larger one
+// of an odd number), the others the second, and each adds the partner's copies of
+// what it keeps; lane l ends with the full sum of value `first` of v[0 .. C), if
+// that is below `end`.  Every sum is formed from the same pairs in the same order
+// as tc_wave_tree_sum (a + b == b + a), so results are bit-identical to reducing
+// each value separately, with C + log2(C) exchanges or fewer instead of 6 C.
+template <int C, int OFF = 32> TC_DEV double wave_reduce_scatter(const double (&v)[C], int &first, int &end)
 {
+    constexpr int H = (C + 1) / 2;
+    const bool up = tc_lane() & OFF;
+    double w[H];
 #pragma unroll
-    for (int j = 0; j < C / 2; ++j) {
-        const double mine = up ? v[C / 2 + j] : v[j];
-        const double send = up ? v[j] : v[C / 2 + j];
-        v[j] = mine + __shfl_xor(send, off, 64);
+    for (int j = 0; j < H; ++j) {
+        if (H + j >= C) {
+            w[j] = tc_xor_add<OFF>(v[j]);
+        } else if constexpr (OFF >= 16) {
+            double a = v[j], b = v[H + j];
+            tc_swap<OFF>(a, b);
+            w[j] = a + b;
+        } else {
+            const double mine = up ? v[H + j] : v[j];
+            const double send = up ? v[j] : v[H + j];
+            w[j] = mine + tc_xor<OFF>(send);
+        }
     }
-}
-
-template <int NV> TC_DEV double wave_reduce_scatter(double *v)
-{
-    static_assert(NV == 4 || NV == 32 || NV == 64, "reduce-scatter width");
-    const int lane = tc_lane();
-    if (NV == 64) {
-        rs_halve<64>(v, 32, lane & 32);
-        rs_halve<32>(v, 16, lane & 16);
-        rs_halve<16>(v, 8, lane & 8);
-        rs_halve<8>(v, 4, lane & 4);
-        rs_halve<4>(v, 2, lane & 2);
-        rs_halve<2>(v, 1, lane & 1);
-    } else if (NV == 32) {
-        rs_halve<32>(v, 32, lane & 32);
-        rs_halve<16>(v, 16, lane & 16);
-        rs_halve<8>(v, 8, lane & 8);
-        rs_halve<4>(v, 4, lane & 4);
-        rs_halve<2>(v, 2, lane & 2);
-        v[0] = v[0] + __shfl_xor(v[0], 1, 64);
-    } else {
-        rs_halve<4>(v, 32, lane & 32);
-        rs_halve<2>(v, 16, lane & 16);
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1)
-            v[0] = v[0] + __shfl_xor(v[0], off, 64);
+    if constexpr (OFF == 32) {
+        first = 0;
+        end = C;
     }
-    return v[0];
+    end = up ? end : min(end, first + H);
+    first += up ? H : 0;
+    if constexpr (OFF > 1)
+        return wave_reduce_scatter<H, OFF / 2>(w, first, end);
+    else
+        return w[0];
 }
 
 // ------------------------------------------------------------------ upward
@@ -1280,9 +1250,10 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
     }
     // lane 0: mass, 16: w, 32: wx, 48: wy (bit-identical to four tree sums)
     double g4[4] = {pm, pw, px, py};
-    const double gsum = wave_reduce_scatter<4>(g4);
-    const double m = __shfl(gsum, 0, 64), w = __shfl(gsum, 16, 64);
-    const double wx = __shfl(gsum, 32, 64), wy = __shfl(gsum, 48, 64);
+    int first, end;
+    const double gsum = wave_reduce_scatter<4>(g4, first, end);
+    const double m = tc_lane_value(gsum, 0), w = tc_lane_value(gsum, 16);
+    const double wx = tc_lane_value(gsum, 32), wy = tc_lane_value(gsum, 48);
     const double xc = w != 0 ? wx / w : (x0 + 0.5 * h);
     const double yc = w != 0 ? wy / w : (y0 + 0.5 * h);
 
@@ -1324,19 +1295,18 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
     }
     double *ex = exps + (size_t)2 * P * id;
     {
-        // [Re a_1..a_p][Im a_1..a_p] reduced together; lane l ends with entry
-        // l (64 entries) or l >> 1 (32 entries)
-        constexpr int NV = 2 * P <= 32 ? 32 : 64;
-        double v[NV];
+        // [Re a_1..a_p][Im a_1..a_p] reduced together
+        double v[2 * P];
 #pragma unroll
-        for (int k = 0; k < NV; ++k)
-            v[k] = k < P ? re[k] : (k < 2 * P ? im[k - P] : 0.0);
-        const double sum = wave_reduce_scatter<NV>(v);
-        const int idx = NV == 64 ? lane : lane >> 1;
-        if (idx < 2 * P && (NV == 64 || (lane & 1) == 0)) {
-            ex[idx] = sum;
+        for (int k = 0; k < P; ++k) {
+            v[k] = re[k];
+            v[P + k] = im[k];
+        }
+        const double sum = wave_reduce_scatter<2 * P>(v, first, end);
+        if (first < end) {
+            ex[first] = sum;
             if (dexps)
-                dexps[(size_t)2 * P * id + idx] = (double)(idx < P ? idx + 1 : idx - P + 1) * sum;
+                dexps[(size_t)2 * P * id + first] = (double)(first < P ? first + 1 : first - P + 1) * sum;
         }
     }
     if (lane == 0) {
@@ -1457,11 +1427,10 @@ TC_DEV void e2e_node(int rank, const int *selfid, const double *box, TcNode *nod
         const double rx = xcp - s_rec[8 * c], ry = ycp - s_rec[8 * c + 1];
         const double v = s_rec[8 * c + 2] + sqrt(rx * rx + ry * ry);
         rr = s_rec[32 + 4 * c] != 0 && rr < v ? v : rr;
-#pragma unroll
-        for (int off = 1; off < 4; off <<= 1) {
-            const double o = __shfl_xor(rr, off, 64);
-            rr = rr < o ? o : rr;
-        }
+        double o = tc_xor<1>(rr);
+        rr = rr < o ? o : rr;
+        o = tc_xor<2>(rr);
+        rr = rr < o ? o : rr;
     }
     const double rcap = ldexp((double)1.4143f * ext, -l);
     const double rad = rcap < rr ? rcap : rr;

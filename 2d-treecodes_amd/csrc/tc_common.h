@@ -20,6 +20,7 @@
 #include <functional>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #define TC_LMAX 15
@@ -143,14 +144,102 @@ TC_DEV unsigned long long tc_ballot(bool p) { return __ballot(p); }
 
 TC_DEV unsigned long long tc_lanemask_lt() { return (1ull << tc_lane()) - 1ull; }
 
+// Exchange between lanes l and l ^ off (off a power of two, constant after
+// unrolling; all lanes active) on the vector unit: gfx950's swaps of half waves
+// and of rows of 16, and data-parallel moves within a row.  __shfl_xor goes
+// through the LDS unit, which the four SIMDs share, and there the leaf upward
+// kernel's reductions bound it (order 9, 2^24 points: 427 -> 337 us) and the direct
+// sums with few targets a leaf waited for it (FP32 potential of 31,623 points: 95 -> 85 us).
+// The swap of a with b: lanes whose bit `off` is clear get {a, a of l ^ off},
+// the others {b of l ^ off, b}.
+template <int OFF> TC_DEV void tc_swap(uint32_t &a, uint32_t &b)
+{
+    static_assert(OFF == 32 || OFF == 16, "half waves or rows");
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                             : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+template <int OFF> TC_DEV void tc_swap(double &a, double &b)
+{
+    uint32_t al = (uint32_t)__double2loint(a), ah = (uint32_t)__double2hiint(a);
+    uint32_t bl = (uint32_t)__double2loint(b), bh = (uint32_t)__double2hiint(b);
+    tc_swap<OFF>(al, bl);
+    tc_swap<OFF>(ah, bh);
+    a = __hiloint2double((int)ah, (int)al);
+    b = __hiloint2double((int)bh, (int)bl);
+}
+
+template <int OFF> TC_DEV void tc_swap(float &a, float &b)
+{
+    uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+    tc_swap<OFF>(x, y);
+    a = __uint_as_float(x);
+    b = __uint_as_float(y);
+}
+
+// v of lane l ^ off within a row
+template <int OFF> TC_DEV uint32_t tc_row_xor(uint32_t v)
+{
+    static_assert(OFF == 8 || OFF == 7 || OFF == 4 || OFF == 2 || OFF == 1, "within a row");
+    const int x = (int)v;
+    if constexpr (OFF == 8)  // rotate by 8
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x128, 0xf, 0xf, false);
+    if constexpr (OFF == 7)  // mirror of 8
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x141, 0xf, 0xf, false);
+    if constexpr (OFF == 4)  // mirror of 8, then of 4
+        return (uint32_t)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xf, 0xf, false), 0x1b, 0xf, 0xf,
+                                                  false);
+    if constexpr (OFF == 2)
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x4e, 0xf, 0xf, false);
+    return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, false);
+}
+template <int OFF> TC_DEV float tc_row_xor(float v) { return __uint_as_float(tc_row_xor<OFF>(__float_as_uint(v))); }
+template <int OFF> TC_DEV double tc_row_xor(double v)
+{
+    return __hiloint2double((int)tc_row_xor<OFF>((uint32_t)__double2hiint(v)),
+                            (int)tc_row_xor<OFF>((uint32_t)__double2loint(v)));
+}
+
+// v of lane l ^ OFF
+template <int OFF, typename T> TC_DEV T tc_xor(T v)
+{
+    if constexpr (OFF >= 16) {
+        T a = v, b = v;
+        tc_swap<OFF>(a, b);
+        return tc_lane() & OFF ? a : b;
+    } else {
+        return tc_row_xor<OFF>(v);
+    }
+}
+
+// v + (v of lane l ^ OFF): the two are the swap's results in one order or the other
+template <int OFF, typename T> TC_DEV T tc_xor_add(T v)
+{
+    if constexpr (OFF >= 16) {
+        T b = v;
+        tc_swap<OFF>(v, b);
+        return v + b;
+    } else {
+        return v + tc_row_xor<OFF>(v);
+    }
+}
+
+// f(integral_constant) for off = FROM, FROM / 2, ..., TO
+template <int FROM, int TO, typename F> TC_DEV void tc_offsets(F &&f)
+{
+    f(std::integral_constant<int, FROM>{});
+    if constexpr (FROM > TO)
+        tc_offsets<FROM / 2, TO>(static_cast<F &&>(f));
+}
+
 // Canonical pairwise tree over the 64 lanes (lane j gets p[j] + p[j ^ off] for
 // off = 32..1); lane 0 ends with ((p0+p32)+(p16+p48))+..., the same order the
 // oracle uses for leaf sums.
 TC_DEV double tc_wave_tree_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-        v = v + __shfl_xor(v, off, 64);
+    tc_offsets<32, 1>([&](auto off) { v = tc_xor_add<off.value>(v); });
     return v;
 }
 
@@ -158,20 +247,29 @@ TC_DEV double tc_wave_tree_sum(double v)
 // values; lanes may differ in the last bit).
 TC_DEV float tc_wave_sum_f32(float v)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-        v = v + __shfl_xor(v, off, 64);
+    tc_offsets<32, 1>([&](auto off) { v = tc_xor_add<off.value>(v); });
     return v;
 }
 
 TC_DEV double tc_wave_max(double v)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const double o = __shfl_xor(v, off, 64);
+    tc_offsets<32, 1>([&](auto off) {
+        const double o = tc_xor<off.value>(v);
         v = v < o ? o : v;
-    }
+    });
     return v;
+}
+
+// Minimum and maximum over the wavefront of two coordinates
+TC_DEV void tc_wave_box(double &xmi, double &ymi, double &xma, double &yma)
+{
+    tc_offsets<32, 1>([&](auto off) {
+        double o;
+        o = tc_xor<off.value>(xmi); xmi = o < xmi ? o : xmi;
+        o = tc_xor<off.value>(ymi); ymi = o < ymi ? o : ymi;
+        o = tc_xor<off.value>(xma); xma = xma < o ? o : xma;
+        o = tc_xor<off.value>(yma); yma = yma < o ? o : yma;
+    });
 }
 
 TC_DEV uint32_t tc_spread15(uint32_t x)

@@ -336,15 +336,7 @@ TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ no
         const double fx = __shfl(x, first, 64), fy = __shfl(y, first, 64);
         const double lx = valid ? x : fx, ly = valid ? y : fy;
         double mnx = lx, mxx = lx, mny = ly, mxy = ly;
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            const double a = __shfl_xor(mnx, off, 64), b = __shfl_xor(mxx, off, 64);
-            const double c = __shfl_xor(mny, off, 64), d = __shfl_xor(mxy, off, 64);
-            mnx = a < mnx ? a : mnx;
-            mxx = b > mxx ? b : mxx;
-            mny = c < mny ? c : mny;
-            mxy = d > mxy ? d : mxy;
-        }
+        tc_wave_box(mnx, mny, mxx, mxy);
         const double cwx = 0.5 * (mnx + mxx), cwy = 0.5 * (mny + mxy);
         const double ddx = lx - cwx, ddy = ly - cwy;
         const double rwave = sqrt(tc_wave_max(ddx * ddx + ddy * ddy));
@@ -473,7 +465,7 @@ TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ no
                 if constexpr (CNT)
                     nslots += 64ull * (unsigned long long)nsrc;
                 const float tx = (float)(x - nd.xcom), ty = (float)(y - nd.ycom);
-                const float ux = __shfl_xor(tx, 32, 64), uy = __shfl_xor(ty, 32, 64);
+                const float ux = tc_xor<32>(tx), uy = tc_xor<32>(ty);
                 const int half = lane >> 5;
                 const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
                 float4 *tile = reinterpret_cast<float4 *>(&s_src[wid][0]);
@@ -514,7 +506,7 @@ TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ no
                     other += (double)(o0 + o1);
                     tc_wave_sync();
                 }
-                const double leafsum = own + __shfl_xor(other, 32, 64);
+                const double leafsum = own + tc_xor<32>(other);
                 if (act)
                     acc += leafsum * (double)LN2_HALF;
             }
@@ -620,10 +612,8 @@ TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ no
             }
             // sum the four node groups' partial coefficients, then every lane
             // evaluates sum_l L_l zeta^l at its own target (Horner, FP64)
-            lre += __shfl_xor(lre, 16, 64);
-            lre += __shfl_xor(lre, 32, 64);
-            lim += __shfl_xor(lim, 16, 64);
-            lim += __shfl_xor(lim, 32, 64);
+            lre = tc_xor_add<32>(tc_xor_add<16>(lre));
+            lim = tc_xor_add<32>(tc_xor_add<16>(lim));
             const double sc = rwave > 0 ? 1.0 / rwave : 0.0;
             const double zr = (x - cwx) * sc, zi = (y - cwy) * sc;
             double hr = 0, hi = 0;
@@ -692,16 +682,10 @@ struct TcPotShared64 {
     }
 };
 
-TC_DEV void acc_add(double &a, double b) { a += b; }
-TC_DEV void acc_add(double2 &a, double2 b)
+template <int OFF> TC_DEV double acc_xor_add(double a) { return tc_xor_add<OFF>(a); }
+template <int OFF> TC_DEV double2 acc_xor_add(double2 a)
 {
-    a.x += b.x;
-    a.y += b.y;
-}
-TC_DEV double acc_shfl_xor(double a, int off) { return __shfl_xor(a, off, 64); }
-TC_DEV double2 acc_shfl_xor(double2 a, int off)
-{
-    return make_double2(__shfl_xor(a.x, off, 64), __shfl_xor(a.y, off, 64));
+    return make_double2(tc_xor_add<OFF>(a.x), tc_xor_add<OFF>(a.y));
 }
 
 // Sum over the leaf's sources [s, e) of pair(acc, dx, dy, v), d = target -
@@ -751,11 +735,10 @@ TC_DEV Acc p2p_leaf64(TcWave64 &w, Acc *s_res, const double4 *__restrict__ src, 
                 }
             }
         }
-#pragma unroll
-        for (int off = 1; off < 8; off <<= 1) {
-            acc_add(a0, acc_shfl_xor(a0, off));
-            acc_add(a1, acc_shfl_xor(a1, off));
-        }
+        // (after the first two steps the lanes of a quad agree: lane l ^ 7 has the
+        // value of l ^ 4)
+        a0 = acc_xor_add<7>(acc_xor_add<2>(acc_xor_add<1>(a0)));
+        a1 = acc_xor_add<7>(acc_xor_add<2>(acc_xor_add<1>(a1)));
         if (q == 0) {
             s_res[b + row] = a0;
             s_res[b + 8 + row] = a1;
@@ -1256,7 +1239,7 @@ TC_DEV void p2p_tile_sum(const void *__restrict__ cur, void *__restrict__ nxt, b
         // read feeds two pair evaluations.  Partner sums are exchanged at the
         // end of the tile.
         const float tx = (float)(xt - xcom), ty = (float)(yt - ycom);
-        const float ux = __shfl_xor(tx, 32, 64), uy = __shfl_xor(ty, 32, 64);
+        const float ux = tc_xor<32>(tx), uy = tc_xor<32>(ty);
         const int half = tc_lane() >> 5;
         const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
         const float4 *tile = static_cast<const float4 *>(cur);
@@ -1300,8 +1283,8 @@ TC_DEV void p2p_tile_sum(const void *__restrict__ cur, void *__restrict__ nxt, b
             ox0 += dx * f;
             oy0 += dy * f;
         }
-        fx += (double)(sx0 + sx1) + (double)__shfl_xor(ox0 + ox1, 32, 64);
-        fy += (double)(sy0 + sy1) + (double)__shfl_xor(oy0 + oy1, 32, 64);
+        fx += (double)(sx0 + sx1) + (double)tc_xor<32>(ox0 + ox1);
+        fy += (double)(sy0 + sy1) + (double)tc_xor<32>(oy0 + oy1);
     } else {
         const double2 *xy = static_cast<const double2 *>(cur);
         const double2 *vv = xy + 32;
@@ -1647,11 +1630,10 @@ __global__ __launch_bounds__(256, 4) void k_force(const TcNode *__restrict__ nod
                                     s_coef[wid], lre, lim);
         }
         // fold the groups' partial local expansions into lanes 0..E2L_G-1
-#pragma unroll
-        for (int off = 32; off >= E2L_G<P>; off >>= 1) {
-            lre += __shfl_xor(lre, off, 64);
-            lim += __shfl_xor(lim, off, 64);
-        }
+        tc_offsets<32, E2L_G<P>>([&](auto off) {
+            lre = tc_xor_add<off.value>(lre);
+            lim = tc_xor_add<off.value>(lim);
+        });
         if (timing) {
             const unsigned long long t1 = tc_clock();
             cloc += t1 - tc0;

@@ -31,6 +31,18 @@ def test_upward_variants(pkg, oracle, wl, n, leaf, order):
     ctx.close()
 
 
+# leaf sums: every order's split of the values over the lanes (halves of odd and even counts); leaves
+# of 1 to 64 points and of several 64s
+@pytest.mark.parametrize("order", [6, 8, 9, 10, 12, 14, 16, 20, 24, 32])
+@pytest.mark.parametrize("n,leaf", [(1, 1), (64, 64), (65, 65), (129, 200), (3001, 64), (3001, 257)])
+def test_leaf_orders(pkg, oracle, wl, n, leaf, order):
+    xs, ys, vs, *_ = wl.mixed_plummer_potential(n, seed=n + order)
+    ctx = pkg.Context(force_order=order, force_leaf=leaf)
+    ctx.force(0.5, xs, ys, vs, np.array([0.4]), np.array([0.4]), np.array([1.0 / 512]))
+    compare_tree(ctx.tree(), oracle.Tree(xs, ys, vs, leaf, order))
+    ctx.close()
+
+
 # one-workgroup sorts with 1, 2, 4, 8, 12, 16 keys per thread, one-launch passes with 1,024 threads a
 # tile (up to 256 tiles of 5,120 keys) and 256 beyond; many equal keys, so stability shows
 @pytest.mark.parametrize("n", [1, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 12288, 12289, 16384, 16385, 40961,
