@@ -1180,44 +1180,6 @@ __global__ __launch_bounds__(SS_NT) void k_sort_small(SortSets sets, double4 *__
     }
 }
 
-// Reduce-scatter form of the pairwise lane tree: at offsets 32, 16, ..., 1 the
-// lanes whose bit is clear keep the first half of their values (the larger one
-// of an odd number), the others the second, and each adds the partner's copies of
-// what it keeps; lane l ends with the full sum of value `first` of v[0 .. C), if
-// that is below `end`.  Every sum is formed from the same pairs in the same order
-// as tc_wave_tree_sum (a + b == b + a), so results are bit-identical to reducing
-// each value separately, with C + log2(C) exchanges or fewer instead of 6 C.
-template <int C, int OFF = 32> TC_DEV double wave_reduce_scatter(const double (&v)[C], int &first, int &end)
-{
-    constexpr int H = (C + 1) / 2;
-    const bool up = tc_lane() & OFF;
-    double w[H];
-#pragma unroll
-    for (int j = 0; j < H; ++j) {
-        if (H + j >= C) {
-            w[j] = tc_xor_add<OFF>(v[j]);
-        } else if constexpr (OFF >= 16) {
-            double a = v[j], b = v[H + j];
-            tc_swap<OFF>(a, b);
-            w[j] = a + b;
-        } else {
-            const double mine = up ? v[H + j] : v[j];
-            const double send = up ? v[j] : v[H + j];
-            w[j] = mine + tc_xor<OFF>(send);
-        }
-    }
-    if constexpr (OFF == 32) {
-        first = 0;
-        end = C;
-    }
-    end = up ? end : min(end, first + H);
-    first += up ? H : 0;
-    if constexpr (OFF > 1)
-        return wave_reduce_scatter<H, OFF / 2>(w, first, end);
-    else
-        return w[0];
-}
-
 // ------------------------------------------------------------------ upward
 // One wavefront per leaf: build_leaf (upward.cpp:61-93) = upward_setup
 // (upward-common.ispc:13-57) + upward_p2e (upward-kernels.m4:52-92), in the
@@ -1251,7 +1213,7 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
     // lane 0: mass, 16: w, 32: wx, 48: wy (bit-identical to four tree sums)
     double g4[4] = {pm, pw, px, py};
     int first, end;
-    const double gsum = wave_reduce_scatter<4>(g4, first, end);
+    const double gsum = tc_wave_scatter_sum<4>(g4, first, end);
     const double m = tc_lane_value(gsum, 0), w = tc_lane_value(gsum, 16);
     const double wx = tc_lane_value(gsum, 32), wy = tc_lane_value(gsum, 48);
     const double xc = w != 0 ? wx / w : (x0 + 0.5 * h);
@@ -1302,7 +1264,7 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
             v[k] = re[k];
             v[P + k] = im[k];
         }
-        const double sum = wave_reduce_scatter<2 * P>(v, first, end);
+        const double sum = tc_wave_scatter_sum<2 * P>(v, first, end);
         if (first < end) {
             ex[first] = sum;
             if (dexps)

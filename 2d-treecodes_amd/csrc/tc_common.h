@@ -243,6 +243,44 @@ TC_DEV double tc_wave_tree_sum(double v)
     return v;
 }
 
+// Reduce-scatter form of the pairwise lane tree: at offsets 32, 16, ..., 1 the
+// lanes whose bit is clear keep the first half of their values (the larger one
+// of an odd number), the others the second, and each adds the partner's copies of
+// what it keeps; lane l ends with the full sum of value `first` of v[0 .. C), if
+// that is below `end`.  Every sum is formed from the same pairs in the same order
+// as tc_wave_tree_sum (a + b == b + a), so results are bit-identical to reducing
+// each value separately, with C + log2(C) exchanges or fewer instead of 6 C.
+template <int C, int OFF = 32, typename T> TC_DEV T tc_wave_scatter_sum(const T (&v)[C], int &first, int &end)
+{
+    constexpr int H = (C + 1) / 2;
+    const bool up = tc_lane() & OFF;
+    T w[H];
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+        if (H + j >= C) {
+            w[j] = tc_xor_add<OFF>(v[j]);
+        } else if constexpr (OFF >= 16) {
+            T a = v[j], b = v[H + j];
+            tc_swap<OFF>(a, b);
+            w[j] = a + b;
+        } else {
+            const T mine = up ? v[H + j] : v[j];
+            const T send = up ? v[j] : v[H + j];
+            w[j] = mine + tc_xor<OFF>(send);
+        }
+    }
+    if constexpr (OFF == 32) {
+        first = 0;
+        end = C;
+    }
+    end = up ? end : min(end, first + H);
+    first += up ? H : 0;
+    if constexpr (OFF > 1)
+        return tc_wave_scatter_sum<H, OFF / 2>(w, first, end);
+    else
+        return w[0];
+}
+
 // Sum over the wavefront, butterfly order (every lane holds a sum of all 64
 // values; lanes may differ in the last bit).
 TC_DEV float tc_wave_sum_f32(float v)

@@ -444,10 +444,20 @@ TC_DEV void potential_wave32(TcPotShared32<P> &sh, const TcNode *__restrict__ no
                             }
                         }
                     }
+                    // one target: its sum in every lane (6 exchanges); more: the eight sums
+                    // scattered over the lanes (10), sum j in lane 8 j, formed from the
+                    // same pairs (16M points 9.57 -> 9.46 ms, 100,000 targets of a
+                    // resident tree 300 -> 290 us)
+                    if (g == 1) {
+                        const float sj = tc_wave_sum_f32(a[0]);
+                        if (lane == tl[0])
+                            part = (double)sj;
+                    } else {
+                        int first, end;
+                        const int sums = __float_as_int(tc_wave_scatter_sum<8>(a, first, end));
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        if (j < g) {
-                            const float sj = tc_wave_sum_f32(a[j]);
+                        for (int j = 0; j < 8; ++j) {
+                            const float sj = __int_as_float(__builtin_amdgcn_readlane(sums, 8 * j));
                             if (lane == tl[j])
                                 part = (double)sj;
                         }
