@@ -1183,26 +1183,42 @@ __global__ __launch_bounds__(SS_NT) void k_sort_small(SortSets sets, double4 *__
 // ------------------------------------------------------------------ upward
 // One wavefront per leaf: build_leaf (upward.cpp:61-93) = upward_setup
 // (upward-common.ispc:13-57) + upward_p2e (upward-kernels.m4:52-92), in the
-// canonical 64-lane strided order with the pairwise lane tree.
+// canonical 64-lane strided order with the pairwise lane tree.  What bounds it is
+// the chain of a wave's memory round trips (entries, sources, and the sources
+// again for the radius and for the coefficients) against the waves in flight: with the
+// entries in one round and the first source of a lane kept, order 9 at 2^24 points went
+// 352 -> 285 us, order 8 at 2^23 points (leaves of 64) 153 -> 129 us.  High orders would take a wave
+// of occupancy more for it than they had (order 24: 160 registers, 15.0 us at 200,000
+// points) and are held to it, at the price of a few spills (14.2; 13.8 before).
 template <int P>
-__global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, const int2 *se, const int *level,
+__global__ __launch_bounds__(256, P <= 16 ? 1 : P <= 24 ? 4 : 3) void k_leaf_upward(const uint32_t *child, const int2 *se, const int *level,
                                                       const int2 *cell, const double4 *src, const double *box,
                                                       const int *__restrict__ info, int tmax, TcNode *nodes, double *exps, double *dexps,
                                                       double4 *nodew, float4 *src32)
 {
     const int id = tc_uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    if (id > 4 * census_nodes(info, tmax) || child[id] != 0)
+    // the node's entries in one round of scalar loads (those past the tree's nodes
+    // are read inside the arrays, and dropped)
+    const int at = min(id, 4 * tmax);
+    const uint32_t inner = child[at];
+    const int2 r = se[at];
+    const int l = level[at];
+    const int2 cc = cell[at];
+    if (id > 4 * census_nodes(info, tmax) || inner != 0)
         return;
     const int lane = tc_lane();
-    const int2 r = se[id];
-    const int s = r.x, e = r.y, l = level[id];
-    const int2 cc = cell[id];
+    const int s = r.x, e = r.y;
     const double xmin = box[0], ymin = box[1], ext = box[2];
     const double h = ext / (double)(1 << l);
     const double x0 = xmin + h * (double)cc.x, y0 = ymin + h * (double)cc.y;
 
-    double pm = 0, pw = 0, px = 0, py = 0;
-    for (int i = s + lane; i < e; i += 64) {
+    // the lane's first source stays in registers for the three sums (most leaves
+    // have no second one); without one, zeros that change no sum
+    const bool has = s + lane < e;
+    const double4 q0 = has ? src[s + lane] : make_double4(0, 0, 0, 0);
+    const double a0 = fabs(q0.z);
+    double pm = q0.z, pw = a0, px = q0.x * a0, py = q0.y * a0;
+    for (int i = s + lane + 64; i < e; i += 64) {
         const double4 q = src[i];
         const double a = fabs(q.z);
         pm += q.z;
@@ -1219,8 +1235,10 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
     const double xc = w != 0 ? wx / w : (x0 + 0.5 * h);
     const double yc = w != 0 ? wy / w : (y0 + 0.5 * h);
 
-    double r2 = 0;
-    for (int i = s + lane; i < e; i += 64) {
+    const double xr0 = has ? q0.x - xc : 0.0, yr0 = has ? q0.y - yc : 0.0;
+    double r2 = xr0 * xr0 + yr0 * yr0;
+    r2 = 0 < r2 ? r2 : 0;
+    for (int i = s + lane + 64; i < e; i += 64) {
         const double4 q = src[i];
         const double xr = q.x - xc, yr = q.y - yc;
         const double d = xr * xr + yr * yr;
@@ -1233,9 +1251,7 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
 #pragma unroll
     for (int k = 0; k < P; ++k)
         re[k] = im[k] = 0;
-    for (int i = s + lane; i < e; i += 64) {
-        const double4 q = src[i];
-        const double r0 = q.x - xc, i0 = q.y - yc, v = q.z;
+    const auto add = [&](int i, double r0, double i0, double v) {
         double rtmp = r0 * v, itmp = i0 * v;
         re[0] -= rtmp;
         im[0] -= itmp;
@@ -1252,8 +1268,13 @@ __global__ __launch_bounds__(256) void k_leaf_upward(const uint32_t *child, cons
             re[k] -= rtmp;
             im[k] -= itmp;
         }
-        if (src32)
+        if (src32 && i < e)
             src32[i] = make_float4((float)r0, (float)i0, (float)v, 0.f);
+    };
+    add(s + lane, xr0, yr0, q0.z);
+    for (int i = s + lane + 64; i < e; i += 64) {
+        const double4 q = src[i];
+        add(i, q.x - xc, q.y - yc, q.z);
     }
     double *ex = exps + (size_t)2 * P * id;
     {
