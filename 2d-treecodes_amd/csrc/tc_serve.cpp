@@ -408,7 +408,8 @@ void reaper(tc_server *s)
         {
             std::lock_guard<std::mutex> lk(s->mu);
             s->freeing -= bytes;
-            s->cv_work.notify_all();
+            if (!s->queue.empty())
+                s->cv_work.notify_all();
         }
         rl.lock();
     }
@@ -671,7 +672,10 @@ void worker(tc_server *s, int slot)
         pick->t_done = now_ms();
         pick->done = true;
         s->cv_done.notify_all();
-        s->cv_work.notify_all();
+        // (with nothing queued the idle slots stay in line: woken for nothing, they would
+        // line up again behind this one, which would then take every short request)
+        if (!s->queue.empty())
+            s->cv_work.notify_all();
         reap(s, victims, mine, &old_bufs);
     }
 }
