@@ -16,17 +16,22 @@
 
 namespace {
 
-constexpr int RS_TILE = 5120;  // radix sort: keys per tile
-// Threads per tile.  Many tiles: 256 threads of 20 keys (three tiles per CU).  Few
-// tiles (RS_WIDE_TILES or fewer, one or two per CU): 1,024 threads of 5, so that a
-// tile's ranking, a chain of LDS round trips per key slot, is a quarter as
-// long: 12.8 -> 10.4 us a pass at 2^16 keys, 20.5 -> 17.9 at 2^20.
-constexpr int RS_NT = 256, RS_NT_WIDE = 1024, RS_WIDE_TILES = 256;
-constexpr int RS_BINS = 256;   // 8-bit digits: passes at bits 0, 8, 16, 24 (30-bit keys)
+// Radix sort of many points: 10-bit digits (three passes over the 30-bit keys;
+// with 8-bit digits four), tiles of 1,024 threads with IT keys each.  Few keys per
+// thread while the tiles fit the CUs once (a tile's ranking is a chain of LDS round
+// trips per key), more where the tiles go in turns: longer digit runs to write, fewer
+// tiles to look back over.  Sort of n keys (box, keys, passes), against 8-bit digits
+// with tiles of 5,120 keys: 2^16 52.1 -> 48.7 us, 2^20 94.6 -> 89.4, 2^21 146 -> 112,
+// 2^22 227 -> 184, 2^23 346 -> 297, 2^24 625 -> 534; with 5 keys per thread 141, 219, 376,
+// 750 from 2^21 on, with 8 333 at 2^23 and 652 at 2^24, with 15 126 at 2^21 and 202 at 2^22.
+constexpr int RS_BITS = 10, RS_BINS = 1 << RS_BITS, RS_PASSES = 3, RS_NT = 1024;
+static_assert(RS_PASSES * RS_BITS >= 2 * TC_LMAX, "the passes cover the keys");
+constexpr int rs_items(int n) { return n <= 256 * 5 * RS_NT ? 5 : n <= 1 << 22 ? 8 : 15; }
+constexpr int SS_BINS = 256;   // one-workgroup sort: 8-bit digits at bits 0, 8, 16, 24
 // Key kernel: most workgroups (each adds its digit totals once), and points per
 // workgroup and step.  Few points are spread thinner, since a workgroup's
 // steps are a chain of memory round trips: 16.9 -> 8 us at 2^16 points, which were 13 steps of 5,120 before.
-constexpr int KH_GRID = 1024, KH_TILE_MIN = 1024;
+constexpr int KH_GRID = 1024, KH_TILE_MIN = 1024, KH_TILE_MAX = 5120;
 constexpr int SCAN_NT = 1024;  // threads of the census workgroup
 
 __constant__ double c_binom[64 * 64];  // C(n, k) rounded to double, n, k < 64
@@ -207,21 +212,21 @@ TC_DEV uint32_t hilbert15(uint32_t x, uint32_t y)
 }
 
 // ------------------------------------------------------------------ radix sort
-// Stable LSD radix sort of (key, index) pairs, 8-bit digits, one launch per
-// pass (k_rs_pass_lb): each tile of RS_TILE keys is ranked stably in LDS with
+// Stable LSD radix sort of (key, index) pairs, one launch per pass
+// (k_rs_pass_lb): each tile of RS_NT IT keys is ranked stably in LDS with
 // wavefront ballots, digit d of tile t is placed at (keys of smaller digits,
 // from the digit totals the key kernel adds up) + (digit d in earlier tiles,
 // by look-back over the counts the earlier tiles publish), and the tile's digit
 // runs are written contiguously.
-// Lanes of the wave holding the same 8-bit digit d as this lane (among lanes
+// Lanes of the wave holding the same digit d as this lane (among lanes
 // with ok set): a lane differs from this one where, for some bit, its ballot
 // bit differs from this lane's own bit.  The per-lane 0 / ~0 of each bit is a
 // sign-extended bit field, so each bit costs a ballot and four 32-bit logic ops.
-TC_DEV unsigned long long wave_digit_peers(uint32_t d, bool ok)
+template <int BITS> TC_DEV unsigned long long wave_digit_peers(uint32_t d, bool ok)
 {
     uint32_t diff_lo = 0, diff_hi = 0;
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (int b = 0; b < BITS; ++b) {
         const unsigned long long bb = tc_ballot((d >> b) & 1u);
         const uint32_t own = (uint32_t)((int32_t)(d << (31 - b)) >> 31);
         diff_lo |= (uint32_t)bb ^ own;
@@ -234,37 +239,38 @@ TC_DEV unsigned long long wave_digit_peers(uint32_t d, bool ok)
 // One tile of a radix pass: the tile's keys are ranked stably in LDS and
 // written out as contiguous digit runs.  start(tot, s_w) is called by every
 // thread of the block after the ranking (it may use the block scratch s_w for
-// collective scans); for digit threadIdx.x (below RS_BINS), of which the tile
-// holds tot keys, it returns the global position of the tile's first key of that
-// digit.
-template <int NT, class Start>
+// collective scans); for digit threadIdx.x, of which the tile holds tot keys, it
+// returns the global position of the tile's first key of that digit.  From 8 keys per
+// thread on keys and indices take turns in one exchange buffer, so that two tiles
+// (at 15 keys one) fit a CU's LDS.
+template <int IT, class Start>
 TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, uint32_t *vout, int n, int shift,
                     int tile, Start &&start)
 {
-    constexpr int IT = RS_TILE / NT, NW = NT / 64, WITEMS = 64 * IT;  // keys per thread, waves per tile, keys per wave
-    static_assert(NT * IT == RS_TILE && NT >= RS_BINS, "whole tiles, a thread per digit");
-    __shared__ uint32_t s_k[RS_TILE];
-    __shared__ uint32_t s_v[RS_TILE];
-    __shared__ uint32_t s_tileoff[RS_BINS];
-    __shared__ uint32_t s_gbase[RS_BINS];
-    __shared__ uint32_t s_wrun[NW][RS_BINS];  // per-wave digit counts, then per-wave tile offsets
+    constexpr int NT = RS_NT, KEYS = NT * IT, NW = NT / 64, WITEMS = 64 * IT;  // waves per tile, keys per wave
+    constexpr bool TURNS = IT >= 8;
+    static_assert(KEYS < 65536 && NT == RS_BINS, "16-bit counts, a thread per digit");
+    __shared__ uint32_t s_k[KEYS * (TURNS ? 1 : 2)];
+    uint32_t *const s_v = s_k + (TURNS ? 0 : KEYS);
+    __shared__ uint32_t s_gofs[RS_BINS];                  // a digit's global start less its start in the tile
+    __shared__ alignas(4) uint16_t s_wrun[NW][RS_BINS];   // per-wave digit counts, then per-wave tile offsets
     __shared__ uint32_t s_w[NW + 1];
 
     const int tid = threadIdx.x, lane = tc_lane(), wid = tid >> 6;
-    const int base = tile * RS_TILE;
-    const int cnt = min(RS_TILE, n - base);
-    for (int d = lane; d < RS_BINS; d += 64)
-        s_wrun[wid][d] = 0;
+    const int base = tile * KEYS;
+    const int cnt = min(KEYS, n - base);
+    for (int d = lane; d < RS_BINS / 2; d += 64)
+        reinterpret_cast<uint32_t *>(s_wrun[wid])[d] = 0;
     tc_wave_sync();
 
     // Each wave ranks its own contiguous WITEMS keys (item j of lane l is key
     // base + wid*WITEMS + 64 j + l), so the order (wave, j, lane) is the input
     // order and the ranks are stable without block barriers: peers with the
-    // same digit are found with 8 ballots, the wave's running count per digit
-    // lives in s_wrun[wid] (all lanes read it before the leader updates it).
+    // same digit are found with a ballot per bit, the wave's running count per
+    // digit lives in s_wrun[wid] (all lanes read it before the leader updates it).
     // Bounds are tested on the offset within the tile, so base + offset is
     // only formed below n (no int overflow for n near INT_MAX).
-    uint32_t k[IT], v[IT], dr[IT];
+    uint32_t k[IT], v[IT], pos[IT];
 #pragma unroll
     for (int j = 0; j < IT; ++j) {
         const int o = wid * WITEMS + j * 64 + lane;
@@ -277,14 +283,14 @@ TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, ui
     for (int j = 0; j < IT; ++j) {
         const bool ok = wid * WITEMS + j * 64 + lane < cnt;
         const uint32_t d = (k[j] >> shift) & (RS_BINS - 1);
-        const unsigned long long peers = wave_digit_peers(d, ok);
+        const unsigned long long peers = wave_digit_peers<RS_BITS>(d, ok);
         const uint32_t lower = __popcll(peers & tc_lanemask_lt());
         const uint32_t run = ok ? s_wrun[wid][d] : 0u;
         tc_wave_sync();
         if (ok && lower == 0)
-            s_wrun[wid][d] = run + (uint32_t)__popcll(peers);
+            s_wrun[wid][d] = (uint16_t)(run + (uint32_t)__popcll(peers));
         tc_wave_sync();
-        dr[j] = ((run + lower) << 8) | d;
+        pos[j] = run + lower;
     }
     __syncthreads();
     {
@@ -294,124 +300,143 @@ TC_DEV void rs_tile(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, ui
         uint32_t c[NW], tot = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            c[w] = tid < RS_BINS ? s_wrun[w][tid] : 0u;
+            c[w] = s_wrun[w][tid];
             tot += c[w];
         }
         const uint32_t g = start(tot, s_w);
         uint32_t off = block_scan_excl<NT>(tot, s_w, nullptr);
-        if (tid < RS_BINS) {
-            s_gbase[tid] = g;
-            s_tileoff[tid] = off;
+        s_gofs[tid] = g - off;
 #pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                s_wrun[w][tid] = off;
-                off += c[w];
-            }
+        for (int w = 0; w < NW; ++w) {
+            s_wrun[w][tid] = (uint16_t)off;
+            off += c[w];
         }
     }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < IT; ++j) {
+        pos[j] += s_wrun[wid][(k[j] >> shift) & (RS_BINS - 1)];
         if (wid * WITEMS + j * 64 + lane < cnt) {
-            const uint32_t pos = s_wrun[wid][dr[j] & 255u] + (dr[j] >> 8);
-            s_k[pos] = k[j];
-            s_v[pos] = v[j];
+            s_k[pos[j]] = k[j];
+            if constexpr (!TURNS)
+                s_v[pos[j]] = v[j];
         }
     }
     __syncthreads();
-
-    for (int p = tid; p < cnt; p += NT) {
-        const uint32_t kk = s_k[p];
-        const uint32_t d = (kk >> shift) & (RS_BINS - 1);
-        const uint32_t dst = s_gbase[d] + (uint32_t)p - s_tileoff[d];
-        kout[dst] = kk;
-        vout[dst] = s_v[p];
+    uint32_t dst[IT];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const int p = tid + j * NT;
+        dst[j] = 0;
+        if (p < cnt) {
+            const uint32_t kk = s_k[p];
+            dst[j] = s_gofs[(kk >> shift) & (RS_BINS - 1)] + (uint32_t)p;
+            kout[dst[j]] = kk;
+            if constexpr (!TURNS)
+                vout[dst[j]] = s_v[p];
+        }
+    }
+    if constexpr (TURNS) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IT; ++j)
+            if (wid * WITEMS + j * 64 + lane < cnt)
+                s_v[pos[j]] = v[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            const int p = tid + j * NT;
+            if (p < cnt)
+                vout[dst[j]] = s_v[p];
+        }
     }
 }
 
 // Above SS_N points each pass is one launch.  The region (zeroed by
-// k_bbox_partial before the keys) holds hist4[4][RS_BINS], every pass's digit
+// k_bbox_partial before the keys) holds RS_PASSES x RS_BINS words, every pass's digit
 // totals over all keys (k_keys_hist); one ticket per pass (64 words); and for
-// each pass the tiles' published digit counts, flags[ntiles][RS_BINS] as 64-bit
-// words: status in the high half (LB_AGG: the tile's own count, LB_INC: its
-// count plus those of all earlier tiles), the count in the low half.
-constexpr int LB_HIST = 4 * RS_BINS;
+// each pass the tiles' published digit counts, flags[ntiles][RS_BINS]: 0 before,
+// the tile's own count plus one, then LB_INC | its count plus those of all earlier
+// tiles (at most the number of keys, 31 bits).
+constexpr int LB_HIST = RS_PASSES * RS_BINS;
 constexpr int LB_TICKETS = 64;
-constexpr unsigned long long LB_AGG = 1ull << 32, LB_INC = 2ull << 32;
+constexpr uint32_t LB_INC = 1u << 31;
 constexpr int RS_SPIN_MAX = 1 << 22;  // polls of one unpublished count before the pass gives up
 constexpr int RS_LB_BATCH = 4;        // earlier tiles' counts read per round trip
 
 // 32-bit words of the region for a sort of ntiles tiles
-static size_t lb_words(int ntiles) { return (size_t)LB_HIST + LB_TICKETS + (size_t)4 * 2 * RS_BINS * ntiles; }
+static size_t lb_words(int ntiles)
+{
+    return (size_t)LB_HIST + LB_TICKETS + (size_t)RS_PASSES * RS_BINS * ntiles;
+}
 
 // One pass of the sort (decoupled look-back).  Tiles are taken in ticket
-// order; a tile publishes its digit counts (LB_AGG) as soon as it has ranked
+// order; a tile publishes its digit counts as soon as it has ranked
 // its keys, then walks back over the tiles before it, adding their counts,
 // until it meets one that has published LB_INC, and publishes its own LB_INC.
-// A tile only ever waits for an LB_AGG, which a tile with a smaller ticket
+// A tile only ever waits for a first count, which a tile with a smaller ticket
 // (started earlier) publishes without waiting: every wait ends.  Digit d of
 // tile t starts at (keys of smaller digits, from hist) + (digit d in tiles
 // 0..t-1), exactly as with a scan of the tile histograms.  A count that stays
 // unpublished for RS_SPIN_MAX polls sets bit 1 of *err (reported by the host
 // as a failed sort) and ends the walk.
-template <int NT>
-__global__ __launch_bounds__(NT) void k_rs_pass_lb(SortSets sets, int pass)
+template <int IT>
+__global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(SortSets sets, int pass)
 {
     __shared__ int s_tile;
     const SortSet &t = (int)blockIdx.x < sets.s[0].ntiles ? sets.s[0] : sets.s[1];
     const uint32_t *const hist = t.lb + RS_BINS * pass;
     uint32_t *const err = t.bad;
-    unsigned long long *const flags =
-        reinterpret_cast<unsigned long long *>(t.lb + LB_HIST + LB_TICKETS) + (size_t)RS_BINS * t.ntiles * pass;
-    // ping-pong out -> scratch -> out -> scratch -> out; the first pass makes the indices
-    const bool odd = pass & 1;
+    uint32_t *const flags = t.lb + LB_HIST + LB_TICKETS + (size_t)RS_BINS * t.ntiles * pass;
+    // ping-pong scratch -> out -> scratch -> out; the first pass makes the indices
+    static_assert(RS_PASSES & 1, "the keys start in the scratch");
+    const bool odd = !(pass & 1);
     const uint32_t *const kin = odd ? t.k2 : t.keys, *const vin = pass == 0 ? nullptr : (odd ? t.v2 : t.perm);
     uint32_t *const kout = odd ? t.keys : t.k2, *const vout = odd ? t.perm : t.v2;
     if (threadIdx.x == 0)
         s_tile = (int)atomicAdd(t.lb + LB_HIST + pass, 1u);
     __syncthreads();
     const int tile = s_tile;
-    rs_tile<NT>(kin, vin, kout, vout, t.n, 8 * pass, tile, [&](uint32_t tot, uint32_t *s_w) {
+    rs_tile<IT>(kin, vin, kout, vout, t.n, RS_BITS * pass, tile, [&](uint32_t tot, uint32_t *s_w) {
         const int d = threadIdx.x;
-        const bool digit = NT == RS_BINS || d < RS_BINS;
-        unsigned long long *fd = flags + (digit ? d : 0);  // fd[t * RS_BINS]: digit d of tile t
-        if (digit)
-            __hip_atomic_store(&fd[(size_t)tile * RS_BINS], (tile ? LB_AGG : LB_INC) | tot, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t before = hist[d];
+        uint32_t *fd = flags + d;  // fd[t * RS_BINS]: digit d of tile t
+        __hip_atomic_store(&fd[(size_t)tile * RS_BINS], tile ? tot + 1u : LB_INC | tot, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
         uint32_t pre = 0;
-        bool done = tile == 0 || !digit;
+        bool done = tile == 0;
         int u = tile;  // tiles u .. tile-1 are summed
         while (!done) {
             // the counts of tiles u-1, u-2, ..., RS_LB_BATCH loads in flight at once
             const int nt = min(RS_LB_BATCH, u);
-            unsigned long long c[RS_LB_BATCH];
+            uint32_t c[RS_LB_BATCH];
 #pragma unroll
             for (int j = 0; j < RS_LB_BATCH; ++j)
                 c[j] = j < nt ? __hip_atomic_load(&fd[(size_t)(u - 1 - j) * RS_BINS], __ATOMIC_RELAXED,
                                                   __HIP_MEMORY_SCOPE_AGENT)
-                              : 0ull;
+                              : 0u;
 #pragma unroll
             for (int j = 0; j < RS_LB_BATCH; ++j) {
                 if (!done && j < nt) {
-                    unsigned long long w = c[j];
+                    uint32_t w = c[j];
                     // tile u-1-j has not published yet: wait for it
-                    for (int spin = 0; !(w >> 32) && spin < RS_SPIN_MAX; ++spin) {
+                    for (int spin = 0; !w && spin < RS_SPIN_MAX; ++spin) {
                         __builtin_amdgcn_s_sleep(2);
                         w = __hip_atomic_load(&fd[(size_t)(u - 1 - j) * RS_BINS], __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT);
                     }
-                    if (!(w >> 32))
+                    if (!w)
                         atomicOr(err, 2u);
-                    pre += (uint32_t)w;
-                    done = (w & LB_INC) || !(w >> 32);
+                    pre += w & LB_INC ? w & ~LB_INC : w ? w - 1u : 0u;
+                    done = (w & LB_INC) || !w;
                 }
             }
             u -= nt;
         }
-        if (tile && digit)
+        if (tile)
             __hip_atomic_store(&fd[(size_t)tile * RS_BINS], LB_INC | (pre + tot), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-        return block_scan_excl<NT>(digit ? hist[d] : 0u, s_w, nullptr) + pre;
+        return block_scan_excl<RS_NT>(before, s_w, nullptr) + pre;
     });
 }
 
@@ -420,18 +445,18 @@ __global__ __launch_bounds__(NT) void k_rs_pass_lb(SortSets sets, int pass)
 // {x, y, v, 0} in input order, so the gather after the sort reads one 32-byte
 // record per source; targets by hilbert15.  Steps of kstep points (a multiple of
 // 1,024) are taken in turn by a set's kgrid workgroups, and each workgroup adds the
-// digit totals of all four passes into lb (zeroed before) once.  Each
+// digit totals of all passes into lb (zeroed before) once.  Each
 // workgroup finishes the bounding box from k_bbox_partial's np partials and
 // per-workgroup flags itself (a set's first one writes it and the non-finite flag).
 __global__ __launch_bounds__(256) void k_keys_hist(SortSets sets)
 {
-    __shared__ uint32_t h[4 * RS_BINS];
+    __shared__ uint32_t h[LB_HIST];
     __shared__ double s_box[4];
     const bool second = (int)blockIdx.x >= sets.s[0].kgrid;
     const SortSet &t = second ? sets.s[1] : sets.s[0];
     const int bi = blockIdx.x - (second ? sets.s[0].kgrid : 0), n = t.n, step = t.kstep;
     const double *x = t.x, *y = t.y, *v = t.v;
-    for (int i = threadIdx.x; i < 4 * RS_BINS; i += 256)
+    for (int i = threadIdx.x; i < LB_HIST; i += 256)
         h[i] = 0;
     if (threadIdx.x < 64)
         bbox_finish(t.part, t.np, s_box);
@@ -451,7 +476,7 @@ __global__ __launch_bounds__(256) void k_keys_hist(SortSets sets)
     // four points a turn, loaded before the first is stored (the compiler cannot
     // tell the arrays apart)
     constexpr int U = 4;
-    static_assert(KH_TILE_MIN % (256 * U) == 0 && RS_TILE % (256 * U) == 0, "whole turns");
+    static_assert(KH_TILE_MIN % (256 * U) == 0 && KH_TILE_MAX % (256 * U) == 0, "whole turns");
     for (long long base = (long long)bi * step; base < n; base += (long long)t.kgrid * step) {
         for (int j = 0; j < step; j += 256 * U) {
             const long long i0 = base + j + threadIdx.x;
@@ -470,18 +495,17 @@ __global__ __launch_bounds__(256) void k_keys_hist(SortSets sets)
                     break;
                 const uint32_t qx = quantise(xi[u], xmin, scale), qy = quantise(yi[u], ymin, scale);
                 const uint32_t k = v ? tc_spread15(qx) | (tc_spread15(qy) << 1) : hilbert15(qx, qy);
-                t.keys[i] = k;
+                t.k2[i] = k;
                 if (t.packed)
                     t.packed[i] = make_double4(xi[u], yi[u], vi[u], 0.0);
-                atomicAdd(&h[k & 255u], 1u);
-                atomicAdd(&h[RS_BINS + ((k >> 8) & 255u)], 1u);
-                atomicAdd(&h[2 * RS_BINS + ((k >> 16) & 255u)], 1u);
-                atomicAdd(&h[3 * RS_BINS + (k >> 24)], 1u);
+#pragma unroll
+                for (int q = 0; q < RS_PASSES; ++q)
+                    atomicAdd(&h[q * RS_BINS + ((k >> (RS_BITS * q)) & (RS_BINS - 1))], 1u);
             }
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 4 * RS_BINS; i += 256)
+    for (int i = threadIdx.x; i < LB_HIST; i += 256)
         if (h[i])
             atomicAdd(&t.lb[i], h[i]);
 }
@@ -504,7 +528,7 @@ static_assert(SS_N == TC_SORT_SMALL_MAX, "one-workgroup sort size");
 // The one-workgroup sort of one point set (the body of k_sort_small and of
 // k_sort_small_batch's workgroups); the sorted keys stay in lds.k.
 template <int IT> struct SortSmallLds {
-    uint32_t k[SS_NT * IT], v[SS_NT * IT], wrun[SS_NT / 64][RS_BINS];
+    uint32_t k[SS_NT * IT], v[SS_NT * IT], wrun[SS_NT / 64][SS_BINS];
 };
 template <int IT>
 TC_DEV void sort_small(SortSmallLds<IT> &lds, bool hilbert, const double *__restrict__ x,
@@ -515,7 +539,7 @@ TC_DEV void sort_small(SortSmallLds<IT> &lds, bool hilbert, const double *__rest
 {
     constexpr int NW = SS_NT / 64, WITEMS = 64 * IT;
     uint32_t *const s_k = lds.k, *const s_v = lds.v;
-    uint32_t(*const s_wrun)[RS_BINS] = lds.wrun;
+    uint32_t(*const s_wrun)[SS_BINS] = lds.wrun;
     __shared__ uint32_t s_w[NW + 1];
     __shared__ double4 s_red[NW];
     __shared__ double s_box[4];
@@ -590,15 +614,15 @@ TC_DEV void sort_small(SortSmallLds<IT> &lds, bool hilbert, const double *__rest
 
 #pragma unroll 1
     for (int shift = 0;; shift += 8) {
-        for (int d = lane; d < RS_BINS; d += 64)
+        for (int d = lane; d < SS_BINS; d += 64)
             s_wrun[wid][d] = 0;
         tc_wave_sync();
         // wave-local stable ranks, as in rs_tile
 #pragma unroll
         for (int j = 0; j < IT; ++j) {
             const bool ok = wid * WITEMS + j * 64 + lane < n;
-            const uint32_t d = (k[j] >> shift) & (RS_BINS - 1);
-            const unsigned long long peers = wave_digit_peers(d, ok);
+            const uint32_t d = (k[j] >> shift) & (SS_BINS - 1);
+            const unsigned long long peers = wave_digit_peers<8>(d, ok);
             const uint32_t lower = __popcll(peers & tc_lanemask_lt());
             const uint32_t run = ok ? s_wrun[wid][d] : 0u;
             tc_wave_sync();
@@ -614,11 +638,11 @@ TC_DEV void sort_small(SortSmallLds<IT> &lds, bool hilbert, const double *__rest
             uint32_t c[NW], tot = 0;
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
-                c[w] = tid < RS_BINS ? s_wrun[w][tid] : 0u;
+                c[w] = tid < SS_BINS ? s_wrun[w][tid] : 0u;
                 tot += c[w];
             }
             uint32_t off = block_scan_excl<SS_NT>(tot, s_w, nullptr);
-            if (tid < RS_BINS) {
+            if (tid < SS_BINS) {
 #pragma unroll
                 for (int w = 0; w < NW; ++w) {
                     s_wrun[w][tid] = off;
@@ -1031,7 +1055,7 @@ TC_DEV void small_topology(SortSmallLds<IT> &lds, const SmallTopo &tp, int n, co
     const int tid = threadIdx.x, lane = tc_lane(), wid = tid >> 6, cap = tp.cap;
     const uint32_t *const key = lds.k;
     uint32_t *const ist = lds.v;             // position | level << 14 by breadth-first rank
-    uint32_t(*const cnt)[RS_BINS] = lds.wrun;  // [wave][level], then first ranks
+    uint32_t(*const cnt)[SS_BINS] = lds.wrun;  // [wave][level], then first ranks
     __shared__ int s_start[TC_LMAX + 1];
     __syncthreads();  // the sort's last reads of lds.v and lds.wrun
     int lo[IT], hi[IT];
@@ -1698,7 +1722,7 @@ static const uint32_t *tc_bbox_bad_flag(TcScratch &ws, int n)
 // sort): np bounding-box partials, the non-finite flag where tc_bbox_bad_flag finds
 // it, per-workgroup flags after it.
 static SortSet sort_set(const double *x, const double *y, const double *v, int n, double *box, uint32_t *keys,
-                        uint32_t *perm, bool records, TcScratch &ws, bool small)
+                        uint32_t *perm, double4 *records, TcScratch &ws, bool small)
 {
     SortSet t = {};
     t.x = x;
@@ -1718,11 +1742,16 @@ static SortSet sort_set(const double *x, const double *y, const double *v, int n
     t.part = ws.bbox_part.as<double4>();
     t.bad = const_cast<uint32_t *>(tc_bbox_bad_flag(ws, n));
     t.pbad = t.bad + 64;
-    t.ntiles = tiles_of(n, RS_TILE);
+    t.ntiles = tiles_of(n, RS_NT * rs_items(n));
     if (lb_words(t.ntiles) > (size_t)INT_MAX)
         throw TcError(-3, "tc_sort_points: too many points");
-    ws.hist.reserve(sizeof(uint32_t) * lb_words(t.ntiles));
-    t.lb = ws.hist.as<uint32_t>();
+    // the counts of a sort with records lie where the sorted records come later
+    if (records && sizeof(uint32_t) * lb_words(t.ntiles) <= sizeof(double4) * (size_t)n) {
+        t.lb = reinterpret_cast<uint32_t *>(records);
+    } else {
+        ws.hist.reserve(sizeof(uint32_t) * lb_words(t.ntiles));
+        t.lb = ws.hist.as<uint32_t>();
+    }
     ws.k2.reserve(sizeof(uint32_t) * (size_t)n);
     ws.v2.reserve(sizeof(uint32_t) * (size_t)n);
     t.k2 = ws.k2.as<uint32_t>();
@@ -1731,8 +1760,8 @@ static SortSet sort_set(const double *x, const double *y, const double *v, int n
         ws.packed.reserve(sizeof(double4) * (size_t)n);
         t.packed = ws.packed.as<double4>();
     }
-    // at most RS_TILE points a step, at least KH_TILE_MIN, about one step per CU
-    t.kstep = std::min(RS_TILE, std::max(KH_TILE_MIN, tiles_of(tiles_of(n, 1024), 256) * 1024));
+    // at most KH_TILE_MAX points a step, at least KH_TILE_MIN, about one step per CU
+    t.kstep = std::min(KH_TILE_MAX, std::max(KH_TILE_MIN, tiles_of(tiles_of(n, 1024), 256) * 1024));
     t.kgrid = std::min(tiles_of(n, t.kstep), KH_GRID);
     return t;
 }
@@ -1755,7 +1784,7 @@ static void sort_sets(const SortSets &t, double4 *src_out, const SmallTopo &tp, 
         }
         return;
     }
-    // the box, the keys with all four passes' digit totals, then one launch per pass
+    // the box, the keys with all passes' digit totals, then one launch per pass
     const int ntiles = t.s[0].ntiles + t.s[1].ntiles;
     k_bbox_partial<<<t.s[0].np + t.s[1].np, 256, 0, st>>>(t, (int)lb_words(t.s[0].ntiles),
                                                           sets == 2 ? (int)lb_words(t.s[1].ntiles) : 0);
@@ -1763,10 +1792,11 @@ static void sort_sets(const SortSets &t, double4 *src_out, const SmallTopo &tp, 
     TC_HIP(hipGetLastError());
     if (ev)
         TC_HIP(hipEventRecord(ev[0], st));
-    const bool wide = ntiles <= RS_WIDE_TILES;
-    const auto pass_kernel = wide ? k_rs_pass_lb<RS_NT_WIDE> : k_rs_pass_lb<RS_NT>;
-    for (int pass = 0; pass < 4; ++pass)
-        pass_kernel<<<ntiles, wide ? RS_NT_WIDE : RS_NT, 0, st>>>(t, pass);
+    // (two sets are sorted together only where both have the fewest keys per thread)
+    const int items = rs_items(t.s[0].n);
+    const auto pass_kernel = items == 5 ? k_rs_pass_lb<5> : items == 8 ? k_rs_pass_lb<8> : k_rs_pass_lb<15>;
+    for (int pass = 0; pass < RS_PASSES; ++pass)
+        pass_kernel<<<ntiles, RS_NT, 0, st>>>(t, pass);
     if (src_out)
         k_gather_src<<<tiles_of(t.s[0].n, 256), 256, 0, st>>>(t.s[0].packed, t.s[0].perm, t.s[0].n, src_out);
     TC_HIP(hipGetLastError());
@@ -1779,7 +1809,7 @@ void tc_morton_sort(const double *x, const double *y, int n, double *box_d, uint
 {
     SortSets t = {};
     // (any non-null strengths make Morton keys; without records they are not read)
-    t.s[0] = sort_set(x, y, x, n, box_d, keys, perm, false, ws, n <= SS_N);
+    t.s[0] = sort_set(x, y, x, n, box_d, keys, perm, nullptr, ws, n <= SS_N);
     sort_sets(t, nullptr, SmallTopo{}, st, nullptr);
 }
 
@@ -1790,13 +1820,14 @@ static SortSet target_set(const double *xt, const double *yt, int m, TcScratch &
     ws.tperm.reserve(sizeof(uint32_t) * (size_t)m + 64);
     ws.info.reserve(sizeof(int) * 32 + sizeof(double) * 4);
     return sort_set(xt, yt, nullptr, m, reinterpret_cast<double *>(ws.info.as<char>() + 128), ws.tkeys.as<uint32_t>(),
-                    ws.tperm.as<uint32_t>(), false, ws, small);
+                    ws.tperm.as<uint32_t>(), nullptr, ws, small);
 }
 
 // Sources and targets up to here in total go through one set of launches; beyond, the
 // GPU is filled by either, and the targets' sort runs beside the build on a stream of
 // its own.
 constexpr int SORT_JOINT_MAX = 1 << 20;
+static_assert(rs_items(SORT_JOINT_MAX) == 5, "one tile size for both sets");
 bool tc_sorts_jointly(int n, int m)
 {
     if (n <= 0 || m <= 0)
@@ -1892,7 +1923,7 @@ void tc_build_tree(TcTree &t, const double *x, const double *y, const double *v,
     uint32_t *keys = t.keys.as<uint32_t>(), *perm = t.perm.as<uint32_t>();
     const bool small = n <= SS_N;
     SortSets sets = {};
-    sets.s[0] = sort_set(x, y, v, n, box, keys, perm, true, ws, small);
+    sets.s[0] = sort_set(x, y, v, n, box, keys, perm, t.src.as<double4>(), ws, small);
     const uint32_t *tbad = nullptr;
     if (targets) {
         sets.s[1] = target_set(targets->x, targets->y, targets->m, *targets->ws, small);

@@ -61,6 +61,23 @@ def test_sort_variants(pkg, oracle, wl, n):
     ctx.close()
 
 
+# one-launch passes with 5, 8 and 15 keys per thread: whole tiles, one key more or less, the largest
+# of each; few distinct keys, and keys in their order and in reverse
+@pytest.mark.parametrize("n", [3 * 5120, 4 * 5120 + 1, 256 * 5120 + 8192, 257 * 8192 - 1, 1 << 22, (1 << 22) + 1,
+                               274 * 15360])
+def test_sort_tiles(pkg, oracle, wl, n):
+    st = wl.Stream(n)
+    t = np.arange(n) / n
+    for x, y in [(np.floor(st.uniform(n) * 3) / 3, np.floor(st.uniform(n) * 4) / 4), (t, t), (1 - t, 0 * t)]:
+        ctx = pkg.Context()
+        box, keys, perm = ctx.empty(4), ctx.empty(n, np.uint32), ctx.empty(n, np.uint32)
+        ctx.morton_sort_device(ctx.to_device(x), ctx.to_device(y), box, keys, perm)
+        ctx.synchronize()
+        operm, oks = oracle.sort(oracle.keys(x, y, oracle.bbox(x, y)))
+        assert np.array_equal(keys.numpy(), oks) and np.array_equal(perm.numpy(), operm)
+        ctx.close()
+
+
 # FP64 potential: 8, 16, 32, 64 targets per wave, whatever the wave the same bits; leaves of one
 # and of several source tiles, full and ragged; 1 to 64 active lanes a leaf
 @pytest.mark.parametrize("m", [1, 7, 8192, 8193, 49152, 49153, 98304, 98305])
