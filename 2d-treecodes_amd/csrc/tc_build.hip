@@ -24,6 +24,7 @@ namespace {
 // with tiles of 5,120 keys: 2^16 52.1 -> 48.7 us, 2^20 94.6 -> 89.4, 2^21 146 -> 112,
 // 2^22 227 -> 184, 2^23 346 -> 297, 2^24 625 -> 534; with 5 keys per thread 141, 219, 376,
 // 750 from 2^21 on, with 8 333 at 2^23 and 652 at 2^24, with 15 126 at 2^21 and 202 at 2^22.
+// With the scans on the vector unit and before the look-back: 45.0, 87.5, 110, 179, 291, 522.
 constexpr int RS_BITS = 10, RS_BINS = 1 << RS_BITS, RS_PASSES = 3, RS_NT = 1024;
 static_assert(RS_PASSES * RS_BITS >= 2 * TC_LMAX, "the passes cover the keys");
 constexpr int rs_items(int n) { return n <= 256 * 5 * RS_NT ? 5 : n <= 1 << 22 ? 8 : 15; }
@@ -42,25 +43,13 @@ TC_DEV uint32_t block_scan_excl(uint32_t v, uint32_t *s_w, uint32_t *total)
 {
     constexpr int NW = NT / 64;
     const int lane = tc_lane(), wid = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= off)
-            x += y;
-    }
+    const uint32_t x = tc_wave_scan(v);
     if (lane == 63)
         s_w[wid] = x;
     __syncthreads();
     if (wid == 0) {
         const uint32_t w = lane < NW ? s_w[lane] : 0u;
-        uint32_t z = w;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(z, off, 64);
-            if (lane >= off)
-                z += y;
-        }
+        const uint32_t z = tc_wave_scan(w);
         if (lane < NW)
             s_w[lane] = z - w;
         if (lane == NW - 1)
@@ -393,16 +382,18 @@ __global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(SortSets sets, int pass)
     const bool odd = !(pass & 1);
     const uint32_t *const kin = odd ? t.k2 : t.keys, *const vin = pass == 0 ? nullptr : (odd ? t.v2 : t.perm);
     uint32_t *const kout = odd ? t.keys : t.k2, *const vout = odd ? t.perm : t.v2;
+    const uint32_t before = hist[threadIdx.x];
     if (threadIdx.x == 0)
         s_tile = (int)atomicAdd(t.lb + LB_HIST + pass, 1u);
     __syncthreads();
     const int tile = s_tile;
     rs_tile<IT>(kin, vin, kout, vout, t.n, RS_BITS * pass, tile, [&](uint32_t tot, uint32_t *s_w) {
         const int d = threadIdx.x;
-        const uint32_t before = hist[d];
         uint32_t *fd = flags + d;  // fd[t * RS_BINS]: digit d of tile t
         __hip_atomic_store(&fd[(size_t)tile * RS_BINS], tile ? tot + 1u : LB_INC | tot, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
+        // (before the walk: the other tiles publish meanwhile)
+        const uint32_t first = block_scan_excl<RS_NT>(before, s_w, nullptr);
         uint32_t pre = 0;
         bool done = tile == 0;
         int u = tile;  // tiles u .. tile-1 are summed
@@ -436,7 +427,7 @@ __global__ __launch_bounds__(RS_NT) void k_rs_pass_lb(SortSets sets, int pass)
         if (tile)
             __hip_atomic_store(&fd[(size_t)tile * RS_BINS], LB_INC | (pre + tot), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-        return block_scan_excl<RS_NT>(before, s_w, nullptr) + pre;
+        return first + pre;
     });
 }
 
@@ -859,13 +850,7 @@ __global__ __launch_bounds__(SCAN_NT) void k_census(const uint32_t *cnt, uint32_
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t sum = (v[j].x + v[j].y) + (v[j].z + v[j].w);
-            uint32_t x = sum;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const uint32_t y = __shfl_up(x, off, 64);
-                if (lane >= off)
-                    x += y;
-            }
+            const uint32_t x = tc_wave_scan(sum);
             const int b = b0 + 256 * j + 4 * lane;
             uint4 o;
             o.x = start + x - sum;
@@ -1088,14 +1073,7 @@ TC_DEV void small_topology(SortSmallLds<IT> &lds, const SmallTopo &tp, int n, co
             w[q] = lane < TC_LMAX ? cnt[q][lane] : 0u;
             tot += w[q];
         }
-        uint32_t x = tot;
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            const uint32_t y = __shfl_up(x, off, 64);
-            if (lane >= off)
-                x += y;
-        }
-        uint32_t start = x - tot;
+        uint32_t start = tc_wave_scan(tot) - tot;
         if (lane <= TC_LMAX) {
             s_start[lane] = min((int)start, tp.tmax);
             tp.info[lane] = (int)start;
@@ -1593,7 +1571,7 @@ __global__ __launch_bounds__(256) void k_e2e_level(const int *__restrict__ selfi
 // level and E2E_CHAIN_T nodes or fewer this way.  Upward pass above the leaves,
 // with one launch per level above 64 nodes and one workgroup for the levels
 // below it (bound by one CU's FP64 rate): 235 -> 146 us at 2^24 sources (order 9),
-// 142 -> 90 at 2^23 (order 8), 45 -> 17 at 2^16 (order 12), 71 -> 37 at 10,000
+// 142 -> 90 at 2^23 (order 8), 45 -> 16 at 2^16 (order 12), 71 -> 32 at 10,000
 // (order 24).
 constexpr int E2E_CHAIN_T = 4096;
 // A build whose node bound is at most this is queued without waiting for its census

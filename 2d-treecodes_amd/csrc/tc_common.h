@@ -234,6 +234,21 @@ template <int FROM, int TO, typename F> TC_DEV void tc_offsets(F &&f)
         tc_offsets<FROM / 2, TO>(static_cast<F &&>(f));
 }
 
+// Inclusive sum over the lanes 0 .. l (all lanes active): shifts by 1, 2, 4 and 8
+// within rows of 16, then the last lane of a row to the next row, of the first half
+// to the second.  Six additions; __shfl_up is an LDS round trip a step.
+TC_DEV uint32_t tc_wave_scan(uint32_t v)
+{
+    int x = (int)v;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return (uint32_t)x;
+}
+
 // Canonical pairwise tree over the 64 lanes (lane j gets p[j] + p[j ^ off] for
 // off = 32..1); lane 0 ends with ((p0+p32)+(p16+p48))+..., the same order the
 // oracle uses for leaf sums.
